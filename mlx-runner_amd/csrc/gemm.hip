@@ -1,8 +1,7 @@
-// Prefill quantized matmul (M > 8) and the dense bf16 linear fallback.
+// Prefill quantized matmul (M > 8) for the shapes the pipelined GEMMs do not take.
 //
 // y[M, N] = x[M, K] @ deq(W)[N, K].T for the prefill chunks mlx-runner feeds
-// through the same qmm call sites (src/engine.zig:364-382, M <= 2048 per chunk),
-// and y = x @ W.T for dense bf16 weights (linear, src/model.zig:200-211).
+// through the same qmm call sites (src/engine.zig:364-382, M <= 2048 per chunk).
 //
 // Tiling (gfx950, wave64, 256 threads):
 //   block tile 128 (x rows) x 128 (W rows), K step 32;
@@ -21,8 +20,6 @@
 #include "qmm_launch.h"
 
 namespace qmm {
-
-constexpr int DENSE_BF16 = 2;
 
 namespace {
 constexpr int BM = 128, BN = 128, BK = 32, LDK = BK + 8;  // LDS row pitch (bf16), 80 bytes
@@ -46,7 +43,7 @@ __device__ __forceinline__ void load_w16(const uint8_t *__restrict__ w, const ui
       out[2 * j] = __builtin_bit_cast(uint32_t, fp8x2_to_bf16x2<false>(d[j]));
       out[2 * j + 1] = __builtin_bit_cast(uint32_t, fp8x2_to_bf16x2<true>(d[j]));
     }
-  } else if constexpr (MODE == NVFP4) {
+  } else {
     const uint2 q = *(const uint2 *)(w + n * (int64_t)(K >> 1) + (k >> 1));
     const float sc = __builtin_amdgcn_cvt_f32_fp8((int)s[n * (int64_t)(K >> 4) + (k >> 4)], 0);
     const uint32_t d[2] = {q.x, q.y};
@@ -59,11 +56,6 @@ __device__ __forceinline__ void load_w16(const uint8_t *__restrict__ w, const ui
       out[4 * j + 2] = pack_bf16x2(c.x * sc, c.y * sc);
       out[4 * j + 3] = pack_bf16x2(e.x * sc, e.y * sc);
     }
-  } else {
-    const uint16_t *wr = (const uint16_t *)w + n * (int64_t)K + k;
-    const uint4 a = ((const uint4 *)wr)[0], b = ((const uint4 *)wr)[1];
-    out[0] = a.x; out[1] = a.y; out[2] = a.z; out[3] = a.w;
-    out[4] = b.x; out[5] = b.y; out[6] = b.z; out[7] = b.w;
   }
 }
 
@@ -178,76 +170,6 @@ hipError_t launch_gemm(const QmmArgs &a, hipStream_t st) {
   else
     hipLaunchKernelGGL((gemm_bf16_kernel<NVFP4>), grid, dim3(256), 0, st, (const uint16_t *)a.x, a.w, a.s,
                        (uint16_t *)a.y, a.M, a.N, a.K);
-  return hipGetLastError();
-}
-
-// ---------------------------------------------------------------- dense bf16 linear
-
-// M <= 8: one wave per 4 W rows, lanes over 16-byte (8-element) chunks.
-template <int M>
-__global__ __launch_bounds__(64) void gemv_bf16_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w,
-                                                       uint16_t *__restrict__ y, int N, int K) {
-  constexpr int R = 4;
-  const int lane = threadIdx.x;
-  const int n0 = blockIdx.x * R;
-  const int C = K >> 3;
-  float acc[R][M];
-#pragma unroll
-  for (int r = 0; r < R; ++r)
-#pragma unroll
-    for (int m = 0; m < M; ++m) acc[r][m] = 0.f;
-  for (int c = lane; c < C; c += 64) {
-    uint4 q[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int n = n0 + r < N ? n0 + r : N - 1;
-      q[r] = load_stream16((const uint4 *)(w + (int64_t)n * K) + c);
-    }
-#pragma unroll
-    for (int m = 0; m < M; ++m) {
-      const uint4 xv = ((const uint4 *)(x + (int64_t)m * K))[c];
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        float t = acc[r][m];
-        t = dot2_bf16(__builtin_bit_cast(bf16x2_t, q[r].x), xv.x, t);
-        t = dot2_bf16(__builtin_bit_cast(bf16x2_t, q[r].y), xv.y, t);
-        t = dot2_bf16(__builtin_bit_cast(bf16x2_t, q[r].z), xv.z, t);
-        t = dot2_bf16(__builtin_bit_cast(bf16x2_t, q[r].w), xv.w, t);
-        acc[r][m] = t;
-      }
-    }
-  }
-  float out = 0.f;
-#pragma unroll
-  for (int r = 0; r < R; ++r)
-#pragma unroll
-    for (int m = 0; m < M; ++m) {
-      float t = wave_sum(acc[r][m]);
-      out = (lane == r * M + m) ? t : out;
-    }
-  if (lane < R * M) {
-    const int r = lane / M, m = lane % M;
-    if (n0 + r < N) y[(int64_t)m * N + n0 + r] = f32_to_bf16_rne(out);
-  }
-}
-
-hipError_t launch_linear_bf16(const uint16_t *x, const uint16_t *w, uint16_t *y, int M, int N, int K,
-                              hipStream_t st) {
-  if (K % 16 != 0 || M <= 0 || N <= 0) return hipErrorInvalidValue;
-  if (M <= 8) {
-    dim3 grid((N + 3) / 4);
-    switch (M) {
-#define QMM_GEMV_CASE(MM) \
-  case MM: hipLaunchKernelGGL((gemv_bf16_kernel<MM>), grid, dim3(64), 0, st, x, w, y, N, K); break;
-      QMM_GEMV_CASE(1) QMM_GEMV_CASE(2) QMM_GEMV_CASE(3) QMM_GEMV_CASE(4)
-      QMM_GEMV_CASE(5) QMM_GEMV_CASE(6) QMM_GEMV_CASE(7) QMM_GEMV_CASE(8)
-#undef QMM_GEMV_CASE
-    }
-    return hipGetLastError();
-  }
-  dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
-  hipLaunchKernelGGL((gemm_bf16_kernel<DENSE_BF16>), grid, dim3(256), 0, st, x, (const uint8_t *)w, nullptr, y, M,
-                     N, K);
   return hipGetLastError();
 }
 

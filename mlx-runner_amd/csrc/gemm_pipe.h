@@ -111,19 +111,19 @@ __device__ __forceinline__ void gp_store_tile_bf16(const f32x16_t (&acc)[FI][FJ]
       }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   constexpr int LPR = FJ * 4;    // lanes per row (16-byte pieces)
-  constexpr int RPI = 64 / LPR;  // rows per instruction
+  constexpr int ITS = NI * 32 * LPR / 64;  // instructions
   if (vec && row0 + (I0 + NI) * 32 <= M && col0 + FJ * 32 <= col_end) {  // the whole block is inside
 #pragma unroll
-    for (int it = 0; it < NI * 32 / RPI; ++it) {
-      const int row = it * RPI + lane / LPR, piece = lane % LPR;
+    for (int it = 0; it < ITS; ++it) {
+      const int q = it * 64 + lane, row = q / LPR, piece = q % LPR;
       const uint4 d = *(const uint4 *)(region + row * PITCH + piece * 16);
       *(uint4 *)yo.at(row0 + I0 * 32 + row, col0 + piece * 8) = d;
     }
     return;
   }
 #pragma unroll
-  for (int it = 0; it < NI * 32 / RPI; ++it) {
-    const int row = it * RPI + lane / LPR, piece = lane % LPR;
+  for (int it = 0; it < ITS; ++it) {
+    const int q = it * 64 + lane, row = q / LPR, piece = q % LPR;
     const uint4 d = *(const uint4 *)(region + row * PITCH + piece * 16);
     const int gr = row0 + I0 * 32 + row, gc = col0 + piece * 8;
     if (gr < M) {
@@ -145,7 +145,7 @@ __device__ __forceinline__ void gp_store_tile_bf16(const f32x16_t (&acc)[FI][FJ]
 // the block's slot (8 waves: 8 * FI * FJ * 1 KiB per slot).  Accumulator rows i with
 // 32 i >= live_rows (the wave's rows past the last x row: padding of a short x) are
 // neither stored nor summed.
-template <int FI, int FJ>
+template <int FI, int FJ, int NW = 8>
 __device__ __forceinline__ void gp_store_partial(const f32x16_t (&acc)[FI][FJ], float *__restrict__ slot, int wave,
                                                  int lane, int live_rows) {
   float4 *pw = (float4 *)slot + (size_t)wave * FI * FJ * 4 * 64 + lane;
@@ -169,14 +169,14 @@ __device__ __forceinline__ void gp_store_partial(const f32x16_t (&acc)[FI][FJ], 
 // as the tile epilogue rounds (rows from M on and columns from col_end on are not stored).
 // All S loads are issued before the first add, so a thread waits for one round trip, not S.
 constexpr int GP_MAX_SPLIT = 8;
-template <int FI, int FJ>
+template <int FI, int FJ, int NW = 8>
 __device__ __forceinline__ void gp_reduce_quad(const float *__restrict__ part, const YOut yo, int M, int col_end,
                                                int t, int S, int wave, int q, int lane, int row0, int col0) {
   const int i = q / (FJ * 4), j = (q / 4) % FJ, v4 = q % 4;
   const int r = row0 + 32 * i + 8 * v4 + 4 * (lane >> 5), c = col0 + 32 * j + (lane & 31);
   if (r >= M || c >= col_end) return;  // not stored by the split blocks either (rows past M)
-  const float4 *pw = (const float4 *)part + ((size_t)t * S * 8 + wave) * FI * FJ * 4 * 64 + q * 64 + lane;
-  const size_t slot = (size_t)8 * FI * FJ * 4 * 64;  // float4s per slot
+  const float4 *pw = (const float4 *)part + ((size_t)t * S * NW + wave) * FI * FJ * 4 * 64 + q * 64 + lane;
+  const size_t slot = (size_t)NW * FI * FJ * 4 * 64;  // float4s per slot
   float4 f[GP_MAX_SPLIT];
 #pragma unroll
   for (int k = 0; k < GP_MAX_SPLIT; ++k) f[k] = pw[(k < S ? k : S - 1) * slot];

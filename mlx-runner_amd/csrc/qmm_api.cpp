@@ -1090,8 +1090,13 @@ int qmm_linear(qmm_array *res, qmm_array x, qmm_array w, qmm_stream s) {
   Arr *ya;
   if (alloc_arr(res, oshape, QMM_BFLOAT16, st, &ya)) return finish(1);
   if (M == 0 || N == 0) return finish(0);
+  void *ws = nullptr;
+  bool transient = false;
+  const size_t need = linear_bf16_workspace((int)M, N, K);
+  if (need && workspace(st, need, &ws, &transient)) return finish(1);
   hipError_t e = launch_linear_bf16((const uint16_t *)xa->data, (const uint16_t *)wa->data, (uint16_t *)ya->data,
-                                    (int)M, N, K, st);
+                                    (int)M, N, K, ws, st);
+  if (transient) (void)hipFreeAsync(ws, st);  // stream-ordered: released after the kernels that use it
   if (e != hipSuccess) return finish(fail_hip(e, op));
   return finish(0);
 }

@@ -8,6 +8,7 @@ import functools
 
 import numpy as np
 import pytest
+import torch
 
 import oracle as O
 import qmm as Q
@@ -309,6 +310,29 @@ def test_dense_linear_matches_fp32_reference(M):
     refb = np.array([[O.f64_to_bf16_bits(v) for v in r] for r in ref], np.uint16)
     ok, fro, worst = O.check_tolerance(f32(y), f32(refb), **TOL)
     assert ok, (fro, worst)
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (9, 1, 16), (10, 65, 48), (64, 63, 64), (65, 129, 1040),      # one partial tile, K ends inside a step
+    (33, 1000, 1040), (129, 273, 3328), (548, 256, 3584),         # tiles split along K
+    (1030, 492, 2848), (700, 2500, 1296),                         # 128-row tiles, whole and left over
+    (1000, 10240, 272), (1000, 10239, 288), (1300, 16400, 528),   # 256-row tiles: one round, and tiles left over
+])
+def test_dense_linear_tiles(M, N, K):
+    """The dense GEMM at the edges of its tiles, K steps and splits, against float64 on the
+    GPU: within the one bf16 rounding (2^-8 of the value) and the fp32 sums' error, which is
+    below 2^-24 K of sum |x| |w|."""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + N + K)
+    x = torch.randn((M, K), generator=gen, device="cuda").to(torch.bfloat16)
+    w = (torch.randn((N, K), generator=gen, device="cuda") * 0.02).to(torch.bfloat16)
+    y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+    for _ in range(2):
+        Q.linear(Q.Array.from_torch(x), Q.Array.from_torch(w), out=Q.Array.from_torch(y),
+                 stream=Q.Stream.torch_current())
+    ref = x.double() @ w.double().t()
+    bound = ref.abs() * 2.0 ** -8 + (x.double().abs() @ w.double().abs().t()) * (K * 2.0 ** -24) + 1e-30
+    assert torch.all((y.double() - ref).abs() <= bound)
 
 
 # ---------------------------------------------------------------- MLP activation and the fused gate/up
