@@ -4,6 +4,7 @@ Bars: dequant and quantize bit-exact; qmm bf16 outputs within relative
 Frobenius 1e-3 and max-abs 4 bf16 ulp of each row's max |y| (oracle rounds its
 double sum once to bf16); f32 outputs within the same bound.
 """
+import ctypes
 import functools
 
 import numpy as np
@@ -104,6 +105,35 @@ def test_quantize_bit_exact(mode, src):
     rq, rs = O.quantize(mode, W)
     assert np.array_equal(s.numpy(), rs)
     assert np.array_equal(wq.numpy(), rq)
+
+
+@pytest.mark.parametrize("mode", ["mxfp8", "nvfp4"])
+@pytest.mark.parametrize("src", ["bf16", "f32"])
+@pytest.mark.parametrize("N,K", [(1, 32), (3, 96), (33, 992), (65, 4128)])
+def test_convert_ragged_bit_exact(mode, src, N, K):
+    """Chunks of 8 elements: sizes that end inside a block's last pass, every magnitude of
+    group (largest scales, subnormal scales, zeros of both signs), values on the midpoints of
+    their scale; and back, on a buffer of 2-byte alignment."""
+    rng = np.random.default_rng(N + K)
+    W = rng.standard_normal((N, K)).astype(np.float32)
+    W *= np.exp2(rng.integers(-40, 40, (N, K // 16))).astype(np.float32).repeat(16, 1)
+    mids = np.array([.25, .75, 1.25, 1.75, 2.5, 3.5, 5, 6, -.25, -.75, -2.5, -5, 0, -0., 1e-3, -1e-3], np.float32)
+    for r in range(0, N, 2):
+        W[r, 16:32] = mids * np.float32(2.0 ** rng.integers(-6, 6)) * np.float32(1 + rng.integers(0, 8) / 8)
+    if src == "bf16":
+        W = f32(bf16(W))
+    wa = Q.Array.from_numpy(bf16(W), Q.BFLOAT16) if src == "bf16" else Q.Array.from_numpy(W, Q.FLOAT32)
+    wq, s = Q.quantize(wa, mode)
+    rq, rs = O.quantize(mode, W)
+    assert np.array_equal(s.numpy(), rs)
+    assert np.array_equal(wq.numpy(), rq)
+    buf = torch.zeros(N * K + 1, dtype=torch.bfloat16, device="cuda")
+    out, stream = Q.Array.from_torch(buf[1:].view(N, K)), Q.Stream()
+    Q.check(Q.lib.qmm_dequantize(ctypes.byref(out.h), wq.h, s.h, Q.qmm_array(None), Q.opt_int(), Q.opt_int(),
+                                 mode.encode(), Q.qmm_array(None), Q.qmm_optional_dtype(0, False), stream.h))
+    stream.sync()
+    d, ref = out.numpy(), O.dequant_bf16(mode, rq, rs, K)
+    assert np.array_equal(d, ref)
 
 
 @pytest.mark.parametrize("mode", ["mxfp8", "nvfp4"])
