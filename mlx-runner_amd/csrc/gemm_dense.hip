@@ -106,20 +106,6 @@ __device__ const uint4 dn_zero = {0, 0, 0, 0};
 // 16-byte piece p of a row's 128 bytes is stored at slot p ^ dn_swz(row).
 __device__ __forceinline__ int dn_swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 
-// Tile t of a call, in the order the blocks take them (tile_of's: groups of 4 x tiles, x
-// tile fastest).
-__device__ __forceinline__ void dn_tile(int t, int tiles_m, int tiles_n, int *tm, int *tn) {
-  constexpr int G = 4;
-  const int first = t / (G * tiles_n) * G, gm = min(tiles_m - first, G), i = t - first * tiles_n;
-  *tm = first + i % gm;
-  *tn = i / gm;
-}
-// Item b of n dealt to XCD b % 8: each XCD takes a contiguous run of items.
-__device__ __forceinline__ int dn_xcd_run(int b, int n) {
-  const int base = n / 8, rem = n % 8, x = b % 8;
-  return x * base + min(x, rem) + b / 8;
-}
-
 template <class G>
 __global__ __launch_bounds__(G::THREADS, G::LDS <= 81920 ? 2 * G::NW / 4 : G::NW / 4) void gemm_dense_kernel(
     const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, uint16_t *__restrict__ y, int M, int N, int K,
@@ -131,23 +117,11 @@ __global__ __launch_bounds__(G::THREADS, G::LDS <= 81920 ? 2 * G::NW / 4 : G::NW
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % G::WM, wn = wave / G::WM;
   const int tiles_m = (M + G::TM - 1) / G::TM, tiles_n = (N + G::TN - 1) / G::TN;
-  // blocks [0, whole_tiles) run whole tiles, the others the K ranges of the tiles that are left
-  const int steps = (K + D_BK - 1) / D_BK, b = blockIdx.x;
-  const bool split = b >= whole_tiles && S > 1;
-  int t, kr = 0;
-  if (b < whole_tiles) {
-    t = dn_xcd_run(b, whole_tiles);
-  } else {  // x tiles of one W range of one K range next to each other
-    const int left = tiles_m * tiles_n - whole_tiles, u = dn_xcd_run(b - whole_tiles, left * S);
-    const int gm = whole_tiles == 0 && tiles_m <= 4 ? tiles_m : 1;
-    kr = u / gm % S;
-    t = whole_tiles + u / (gm * S) * gm + u % gm;
-  }
-  int tm, tn;
-  dn_tile(t, tiles_m, tiles_n, &tm, &tn);
-  const int m0 = tm * G::TM, n0 = tn * G::TN;
-  const int s_begin = split ? (int)((int64_t)kr * steps / S) : 0;
-  const int s_end = split ? (int)((int64_t)(kr + 1) * steps / S) : steps;
+  const int steps = (K + D_BK - 1) / D_BK;
+  const GpBlock blk = gp_block(blockIdx.x, tiles_m, tiles_n, whole_tiles, S);
+  const int m0 = blk.tm * G::TM, n0 = blk.tn * G::TN;
+  const int s_begin = blk.split ? (int)((int64_t)blk.kr * steps / S) : 0;
+  const int s_end = blk.split ? (int)((int64_t)(blk.kr + 1) * steps / S) : steps;
 
   // A DMA fills 1 KiB: rows 8 g + [0, 8) of a stage of x (or W), g = wave + NW i; lane l the
   // 16-byte slot l % 8 of row l / 8, which holds piece (l % 8) ^ swz(row) of the row's step.
@@ -265,34 +239,20 @@ __global__ __launch_bounds__(G::THREADS, G::LDS <= 81920 ? 2 * G::NW / 4 : G::NW
   for (; s < s_end; ++s) step(std::integral_constant<int, 0>{}, s);
   gp_lds_barrier();
 
-  if (split) {
-    gp_store_partial<FI, FJ, G::NW>(acc, part + (size_t)((t - whole_tiles) * S + kr) * G::TM * G::TN, wave, lane,
-                                    M - (m0 + wm * 32 * FI));
+  const int row0 = m0 + wm * 32 * FI, col0 = n0 + wn * 32 * FJ;
+  if (blk.split) {
+    gp_store_partial<FI, FJ, G::NW>(acc, part + (size_t)((blk.t - whole_tiles) * S + blk.kr) * G::TM * G::TN, wave, lane,
+                                    M - row0);
     return;
   }
-  const YOut yo{y, nullptr, nullptr, nullptr, INT32_MAX, INT32_MAX, INT32_MAX, N, 0, 0, 0};
-  const bool vec = yout_vec(yo);
-  uint8_t *region = lds + wave * G::REGION;
-  const int row0 = m0 + wm * 32 * FI, col0 = n0 + wn * 32 * FJ;
-  gp_store_tile_bf16<FI, FJ, 0, 1>(acc, region, lane, yo, M, row0, col0, N, vec);
-  if constexpr (FI > 1) gp_store_tile_bf16<FI, FJ, 1, 1>(acc, region, lane, yo, M, row0, col0, N, vec);
-  if constexpr (FI > 2) gp_store_tile_bf16<FI, FJ, 2, 1>(acc, region, lane, yo, M, row0, col0, N, vec);
-  if constexpr (FI > 3) gp_store_tile_bf16<FI, FJ, 3, 1>(acc, region, lane, yo, M, row0, col0, N, vec);
+  const YOut yo = yout_one(y, N);
+  gp_store_rows<FI, FJ, 0>(acc, lds + wave * G::REGION, lane, yo, M, row0, col0, N, yout_vec(yo));
 }
 
-// The split tiles' results: one thread per float4 of a tile's partial layout.
 template <class G>
 __global__ __launch_bounds__(256) void gemm_dense_reduce_kernel(const float *__restrict__ part, uint16_t *__restrict__ y,
                                                                int M, int N, int whole_tiles, int S) {
-  constexpr int NQ = G::FI * G::FJ * 4;
-  const int g = blockIdx.x * 256 + threadIdx.x;
-  const int t = g / (G::NW * NQ * 64), rem = g - t * (G::NW * NQ * 64);
-  const int wave = rem / (NQ * 64), q = (rem >> 6) % NQ, lane = rem & 63;
-  int tm, tn;
-  dn_tile(whole_tiles + t, (M + G::TM - 1) / G::TM, (N + G::TN - 1) / G::TN, &tm, &tn);
-  const YOut yo{y, nullptr, nullptr, nullptr, INT32_MAX, INT32_MAX, INT32_MAX, N, 0, 0, 0};
-  gp_reduce_quad<G::FI, G::FJ, G::NW>(part, yo, M, N, t, S, wave, q, lane, tm * G::TM + (wave % G::WM) * 32 * G::FI,
-                                      tn * G::TN + (wave / G::WM) * 32 * G::FJ);
+  gp_reduce_tile<G>(part, yout_one(y, N), M, N, whole_tiles, S, blockIdx.x * 256 + threadIdx.x);
 }
 
 // ---------------------------------------------------------------- the plan
@@ -305,51 +265,19 @@ using DnH = DnGeom<4, 2, 2, 2, 2, 4>;     // 256 x 128
 using Dn128 = DnGeom<2, 2, 2, 2, 2, 3>;   // 128 x 128, two blocks per CU
 using Dn64 = DnGeom<2, 1, 1, 4, 2, 4>;    // 64 x 128, two blocks per CU
 using DnS = DnGeom<1, 1, 2, 2, 2, 4>;     // 64 x 64, three blocks per CU
-// us per K step of each configuration, with one block on every CU and with per_cu blocks on
-// every CU (measured on calls of whole rounds and of at most one block per CU, weights cold).
-struct DnCost {
-  int TM, TN, per_cu;
-  float one, full;
-};
-constexpr DnCost DN_COST[] = {{256, 256, 1, 1.24f, 1.24f}, {256, 160, 1, 1.10f, 1.10f}, {192, 256, 1, 1.20f, 1.20f},
-                              {256, 128, 1, 0.91f, 0.91f}, {128, 128, 2, 0.64f, 0.90f}, {64, 128, 2, 0.56f, 0.74f},
-                              {64, 64, 3, 0.42f, 0.72f}};
-constexpr int DN_CONFIGS = sizeof(DN_COST) / sizeof(DN_COST[0]);
+constexpr GpCost DN_COST[] = {{256, 256, 1, 3.f, {1.24f}},         {256, 160, 1, 3.f, {1.10f}},
+                              {192, 256, 1, 3.f, {1.20f}},         {256, 128, 1, 3.f, {0.91f}},
+                              {128, 128, 2, 3.f, {0.64f, 0.90f}},  {64, 128, 2, 3.f, {0.56f, 0.74f}},
+                              {64, 64, 3, 3.f, {0.42f, 0.57f, 0.72f}}};
 }  // namespace
 
-// The configuration of a call: the least estimated time over every tile size and every split
-// of the tiles left after the whole rounds (at most GP_MAX_SPLIT ways, one round of blocks, at
-// least 4 K steps each).  Per round: its K steps and ~3 us of start and epilogue; a split adds
-// the reduce, ~4 us and its partial sums' traffic.  On 39 shapes over the declared range the
-// plan's time is 1.05 of the best configuration's on average, at most 1.35.
-struct DnPlan {
-  int cfg, whole, left, S;  // whole tiles, then `left` tiles split S ways along K
-  float us;
-};
-static DnPlan dense_plan(int M, int N, int K, int cus) {
-  DnPlan best{0, 0, 0, 1, 1e30f};
-  if (cus <= 0) cus = 256;  // (no device answers: the launch reports it)
-  const int steps = (K + D_BK - 1) / D_BK;
-  for (int c = 0; c < DN_CONFIGS; ++c) {
-    const DnCost &d = DN_COST[c];
-    const int64_t T = (int64_t)((M + d.TM - 1) / d.TM) * ((N + d.TN - 1) / d.TN);
-    const int64_t slots = (int64_t)cus * d.per_cu, whole = T / slots * slots, left = T - whole;
-    const float base = (float)(whole / slots) * (steps * d.full + 3.f);
-    for (int S = 1; S <= GP_MAX_SPLIT; ++S) {
-      if (S > 1 && (left == 0 || left * S > slots || steps < 4 * S)) break;
-      float us = base;
-      if (left) us += (float)((steps + S - 1) / S) * (left * S <= cus ? d.one : d.full) + 3.f;
-      if (S > 1) us += 4.f + (float)left * S * d.TM * d.TN * 8.f / 4e6f;
-      if (us < best.us) best = DnPlan{c, (int)whole, (int)left, S, us};
-    }
-  }
-  if (best.S == 1) best.whole += best.left, best.left = 0;
-  return best;
+static GpPlan dense_plan(int M, int N, int K) {
+  return gp_plan(DN_COST, sizeof(DN_COST) / sizeof(DN_COST[0]), M, N, (K + D_BK - 1) / D_BK, 1, device_cu_count());
 }
 
 template <class G>
 static hipError_t launch_dense_cfg(const uint16_t *x, const uint16_t *w, uint16_t *y, int M, int N, int K,
-                                   const DnPlan &p, float *part, hipStream_t st) {
+                                   const GpPlan &p, float *part, hipStream_t st) {
   static std::atomic<uint64_t> lds_set{0};
   hipError_t e = ensure_dynamic_lds(lds_set, (const void *)gemm_dense_kernel<G>, G::LDS);
   if (e != hipSuccess) return e;
@@ -364,7 +292,7 @@ static hipError_t launch_dense_cfg(const uint16_t *x, const uint16_t *w, uint16_
 }
 
 static hipError_t launch_dense_plan(const uint16_t *x, const uint16_t *w, uint16_t *y, int M, int N, int K,
-                                    const DnPlan &p, float *part, hipStream_t st) {
+                                    const GpPlan &p, float *part, hipStream_t st) {
   switch (p.cfg) {
     case 0: return launch_dense_cfg<Dn256>(x, w, y, M, N, K, p, part, st);
     case 1: return launch_dense_cfg<Dn160>(x, w, y, M, N, K, p, part, st);
@@ -378,14 +306,14 @@ static hipError_t launch_dense_plan(const uint16_t *x, const uint16_t *w, uint16
 
 size_t linear_bf16_workspace(int M, int N, int K) {
   if (M <= QMV_MAX_M) return 0;
-  const DnPlan p = dense_plan(M, N, K, device_cu_count());
+  const GpPlan p = dense_plan(M, N, K);
   return (size_t)p.left * p.S * DN_COST[p.cfg].TM * DN_COST[p.cfg].TN * sizeof(float);
 }
 
 hipError_t launch_linear_bf16(const uint16_t *x, const uint16_t *w, uint16_t *y, int M, int N, int K, void *ws,
                               hipStream_t st) {
   if (K % 16 != 0 || M <= 0 || N <= 0) return hipErrorInvalidValue;
-  if (M > QMV_MAX_M) return launch_dense_plan(x, w, y, M, N, K, dense_plan(M, N, K, device_cu_count()), (float *)ws, st);
+  if (M > QMV_MAX_M) return launch_dense_plan(x, w, y, M, N, K, dense_plan(M, N, K), (float *)ws, st);
   dim3 grid((N + 3) / 4);
   switch (M) {
 #define QMM_GEMV_CASE(MM) \

@@ -618,14 +618,16 @@ static bool gemm_mxfp8_pipe_ok(const QmmArgs &a) {
 static size_t round256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 hipError_t launch_repack_scales(const uint8_t *s, int64_t N, int nb, uint32_t *out, hipStream_t st) {
-  const int dpr = nb / 4;
-  const bool wide = dpr % 4 == 0 && (uintptr_t)s % 16 == 0;
+  const int dpr = (nb + 3) / 4;
+  const bool dwords = nb % 4 == 0 && (uintptr_t)s % 4 == 0, wide = dwords && dpr % 4 == 0 && (uintptr_t)s % 16 == 0;
   const int64_t threads = (int64_t)round256(N) * dpr / (wide ? 4 : 1);
   const int64_t blocks = (threads + 255) / 256 < 65536 ? (threads + 255) / 256 : 65536;
   if (wide)
     hipLaunchKernelGGL(repack_scales_kernel<4>, dim3(blocks), dim3(256), 0, st, s, N, nb, out);
-  else
+  else if (dwords)
     hipLaunchKernelGGL(repack_scales_kernel<1>, dim3(blocks), dim3(256), 0, st, s, N, nb, out);
+  else
+    hipLaunchKernelGGL(repack_scales_kernel<0>, dim3(blocks), dim3(256), 0, st, s, N, nb, out);
   return hipGetLastError();
 }
 
@@ -694,7 +696,7 @@ size_t gemm_mxfp8_workspace(const QmmArgs &a) {
   return bytes + 256;
 }
 
-size_t tiled_scales_bytes(int64_t N, int nb) { return (size_t)round256((size_t)N) * (size_t)nb; }
+size_t tiled_scales_bytes(int64_t N, int nb) { return (size_t)round256((size_t)N) * (size_t)((nb + 3) / 4 * 4); }
 
 int gemm_tiled_scale_bytes_per_row(const QmmArgs &a) {
   if (qmm_on_decode(a) || a.x_f32 || a.K <= 0) return 0;

@@ -7,24 +7,24 @@
 // which no 8-bit MFMA operand format holds, and the scaled MFMAs take only
 // E8M0 scales per 32; in bf16 (8 bits) the dequantized weight is exact.
 //
-// Same pipeline as the mxfp8 kernel: 256 x 256 block tile, K step 64, 8 waves
-// in two ping-pong groups, a 3-stage LDS ring filled by LDS DMA two steps ahead,
-// one barrier per interval.  The 64 elements of a step are taken in an order
-// of our choosing (the same for x and W, so the sum is unchanged): K sub-step
-// ks (of 4) takes elements 8 ks + [0, 8) for operand lane half 0 and
-// 32 + 8 ks + [0, 8) for half 1, so a lane's four 8-element W pieces are one
-// contiguous 16-byte piece of its row.  Per stage:
-//   * x tile, 256 rows x 64 bf16 (128 bytes per row, moved in whole 128-byte
-//     row segments); 16-byte slot S of row r stored at slot S ^ aswz(r);
-//   * W tile kept in nvfp4, 256 rows x 32 bytes, row-major, moved by one
-//     16-byte-per-lane DMA per wave (32 rows);
-//   * the step's E4M3 scales, one dword (4 groups of 16) per W row, from the
-//     tile-major repacked copy.
-// Each wave owns 128 x 64 of the tile (4 x 2 accumulators).  The loading
-// interval reads the wave's W fragments and scales and dequantizes them in
-// registers (E2M1 -> f32, times the scale, -> bf16: exact), beside the other
-// group's MFMAs; the computing interval reads x fragments per K sub-step and
-// runs the MFMAs.
+// What bounds it: at tall x the matrix cores at the clock the power limit leaves (a large
+// bf16 library product reaches ~1.45 PFLOP/s here), at short x the latency of a step.  So:
+//   * K steps of 64, x by DMA in whole 128-byte cache lines per row into a ring of SX
+//     stages.  A row's W piece of a step is 32 bytes, so W moves in stages of four steps,
+//     128 bytes per row as well, with their scales; two such stages are four steps of lead,
+//     which covers the ~1.2 us that cold W takes.
+//   * The waves lie side by side along W (1 x 4), so that one wave of the block dequantizes
+//     a W element (VALU work), in pairs spread between the MFMAs of the sub-step before it
+//     is used, beside the reads of that sub-step's x; one barrier per K step.
+//   * The tile height is chosen per call (nv_plan), and the tiles left over after the whole
+//     rounds are split along K over the idle CUs, fp32 partial sums reduced in K order
+//     (deterministic) by a second kernel.
+// Measured, us per call, weights cold (M x N x K; the former kernel, two groups of waves in
+// turns with W moved 32 bytes per row and step, in brackets): 2048 x 16480 x 5120  271 (318,
+// 1.28 PFLOP/s now), 500 x 10240 x 5120  57 (63), 48 x 17408 x 5120  26 (30), 200 x 6144 x
+// 5120  26 (32).  256 x 256 tiles in 8 waves of 128 x 64, which dequantize every element
+// twice: 276 in the first.  K that is not a multiple of 64, which ran gemm.hip's kernel:
+// 33 x 1000 x 1056 28 -> 9.4.
 #include <type_traits>
 
 #include "gemm_pipe.h"
@@ -34,110 +34,121 @@
 namespace qmm {
 
 namespace {
-constexpr int V_BM = 256, V_BN = 256, V_BK = 64, V_THREADS = 512;
-constexpr int V_WTILE = 256 * 32;  // W: 256 rows x 64 nvfp4
-constexpr int V_STILE = 1024;      // scale dwords
-constexpr int V_STAGES = 3;
-// Per x-tile height TM (256, or 128 for the last tile-columns of a call): the x tile,
-// TM rows x 64 bf16, one stage, the ring, the x fragments per wave (FI, of 32 rows), and
-// the DMAs per wave per step: FI x, 1 W, and for wave 0 the step's 256 scale dwords
-// (1 KiB, one DMA).
-template <int TM>
+constexpr int V_BK = 64;   // K elements of a step: 128 bytes of an x row, 32 of a W row
+constexpr int V_SS = 4;    // steps of a W stage: 128 bytes of a W row, 16 of its scales
+// A block's tile: WM x WN waves of (32 FI) x (32 FJ); LDS rings of SX stages of x (a step
+// each) and two stages of W and its scales (V_SS steps each).
+template <int FI_, int FJ_, int WM_, int WN_, int SX_>
 struct NvGeom {
-  static constexpr int ATILE = TM * 128;
-  static constexpr int STAGE = ATILE + V_WTILE + V_STILE;  // 41 KiB at 256, 25 KiB at 128
-  static constexpr size_t LDS = (size_t)V_STAGES * STAGE;  // 123 KiB at 256
-  static constexpr int FI = TM / 64;
-  static constexpr int DMA = FI + 1, DMA_S = FI + 2;
+  static constexpr int FI = FI_, FJ = FJ_, WM = WM_, WN = WN_, SX = SX_;
+  static constexpr int TM = 32 * FI * WM, TN = 32 * FJ * WN, NW = WM * WN, THREADS = 64 * NW;
+  static constexpr int XT = TM * 128, WT = TN * 128, ST = TN * 16;
+  static constexpr int WOFF = SX * XT, SOFF = WOFF + 2 * WT;  // the rings' places
+  static constexpr int LDS = SOFF + 2 * ST;
+  static constexpr int NX = TM / 8 / NW;           // x DMAs per wave per step
+  static constexpr int NWD = TN / 8 / NW;          // W DMAs per wave per stage, in two halves:
+  static constexpr int NA = NWD / 2 + 1, NB = NWD - NWD / 2;  // NA with the scales' one
+  static_assert(TM / 8 % NW == 0 && TN / 8 % NW == 0 && TN % 64 == 0 && NW % 2 == 0 && SX >= 2 && SX <= 4, "");
+  static constexpr int REGION = 32 * (64 * FJ + 32);
+  static_assert(NW * REGION <= LDS, "the epilogue regions fit the rings");
+  // DMAs that may be in flight at the barrier of step j of a stage (see the kernel): those
+  // issued after x of the next step, and at j = 3 none of the next W stage's
+  static constexpr int in_flight(int j) {
+    int n = (SX - 2) * NX;
+    for (int i = j + 1 - SX; i < j; ++i) n += (i & 3) == 3 ? NA : (i & 3) == 0 ? NB : 0;
+    return j == 3 && n > 2 * NX ? 2 * NX : j == 3 && SX < 4 ? (SX - 2) * NX : n;
+  }
 };
-// Every launch allocates the 256-row ring (the two-height kernel runs both in one launch).
-constexpr size_t V_LDS = NvGeom<256>::LDS;
 }  // namespace
 
-__device__ __forceinline__ int aswz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
-// W tile: row r's two 16-byte halves are stored swapped when wswz(r) = 1, so that the
-// fragment reads of 16 consecutive rows (one half each) fall in distinct banks (rows
-// r and r + 8, and r and r + 4 on 32 banks, would otherwise share them)
-__device__ __forceinline__ int wswz(int r) { return ((r >> 2) ^ (r >> 3)) & 1; }
+// Zeros that stand for the pieces of the last step and stage past K.
+__device__ const uint4 nv_zero = {0, 0, 0, 0};
 
-// Tile `bid` of the TM x 256 tiling of x rows [0, M) and W rows [n_begin, n_end)
-// (n_begin a multiple of 256), over the K steps [s_begin, s_end).  With `part` null the
-// tile's bf16 result goes to y; otherwise (a K range of a split tile) the fp32
-// accumulators go to `part` (gp_store_partial's layout).
-template <int TM>
-__device__ __forceinline__ void nv_tile(int bid, const uint16_t *__restrict__ x, const uint8_t *__restrict__ w,
-                                        const uint8_t *__restrict__ sp, const YOut yo, int M, int N, int K,
-                                        int n_begin, int n_end, int s_begin, int s_end, float *__restrict__ part) {
-  using G = NvGeom<TM>;
-  // Wave layout: 2 (x rows) x 4 (W rows), waves of TM / 2 x 64, or at TM = 64 1 x 8, waves
-  // of 64 x 32, so that each W element is dequantized by one wave of the block (at short x
-  // the dequantization, not the MFMA work, is what a step costs).
-  constexpr bool COLS = TM == 64;
-  constexpr int XD = G::FI;                // x DMAs per wave per step
-  constexpr int FI = COLS ? 2 : TM / 64;   // x fragments (32 rows) per wave
-  constexpr int FJ = COLS ? 1 : 2;         // W fragments (32 rows) per wave
-  constexpr int WM = COLS ? TM : TM / 2, WN = 32 * FJ;
+// 16-byte piece p of a row's 128 bytes is stored at slot p ^ nv_swz(row).
+__device__ __forceinline__ int nv_swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
+
+template <class G>
+__global__ __launch_bounds__(G::THREADS, G::LDS <= 81920 ? 2 * G::NW / 4 : G::NW / 4) void gemm_nvfp4_kernel(
+    const uint16_t *__restrict__ x, const uint8_t *__restrict__ w, const uint8_t *__restrict__ sp, const YOut yo, int M,
+    int N, int K, int whole_tiles, int S, float *__restrict__ part) {
+  constexpr int FI = G::FI, FJ = G::FJ, NX = G::NX, NWD = G::NWD, SX = G::SX;
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const uint32_t lds0 = lds_addr(lds);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = COLS ? 0 : wave & 1, wn = COLS ? wave : wave >> 1;  // rows wm WM + [0, WM), cols wn WN + [0, WN)
-  int tm, tn;
-  tile_of(bid, (M + TM - 1) / TM, (n_end - n_begin + V_BN - 1) / V_BN, &tm, &tn);
-  const int m0 = tm * TM, n0 = n_begin + tn * V_BN;
-  const int steps = K / V_BK;
-  const int64_t wrow = K >> 1;  // bytes per W row
+  const int wm = wave % G::WM, wn = wave / G::WM;
+  const int tiles_m = (M + G::TM - 1) / G::TM, tiles_n = (N + G::TN - 1) / G::TN;
+  const int steps = (K + V_BK - 1) / V_BK, stages = (steps + V_SS - 1) / V_SS;
+  const GpBlock blk = gp_block(blockIdx.x, tiles_m, tiles_n, whole_tiles, S);
+  const int m0 = blk.tm * G::TM, n0 = blk.tn * G::TN;
+  // the block's W stages [g_begin, g_end) and steps [s_begin, s_end)
+  const int g_begin = blk.split ? (int)((int64_t)blk.kr * stages / S) : 0;
+  const int g_end = blk.split ? (int)((int64_t)(blk.kr + 1) * stages / S) : stages;
+  const int s_begin = g_begin * V_SS, s_end = min(g_end * V_SS, steps);
 
-  // DMA sources (step 0).  x: wave-instruction g = wave + 8 i fills slots q = 64 g + lane,
-  // rows 8 g + [0, 8) of the tile.  When all 8 are past the last x row (a short x), it moves
-  // 4 bytes per lane instead of 16: the same instruction count (the waits count them), a
-  // quarter of the bytes, and those rows' results are not stored.
-  // Every DMA source is a wave-uniform base (SGPRs: the tile's first row and the step)
-  // plus a 32-bit lane offset within the tile's rows.
-  const uint8_t *xb = (const uint8_t *)x + (int64_t)m0 * K * 2;
-  uint32_t xoff[XD];
-  bool xdead[XD];
+  // A DMA fills 1 KiB: rows 8 g + [0, 8) of a stage of x (or W), g = wave + NW i; lane l the
+  // 16-byte slot l % 8 of row l / 8, which holds piece (l % 8) ^ swz(row) of the row's 128 bytes.
+  const int64_t wrow = K >> 1;
+  const uint8_t *xb = (const uint8_t *)x + (int64_t)m0 * K * 2, *wb = w + (int64_t)n0 * wrow;
+  const int dr = 8 * wave + (lane >> 3), dp = (lane & 7) ^ nv_swz(dr);  // rows 8 NW apart share a swizzle
+  uint32_t xo[NX], wo[NWD];
 #pragma unroll
-  for (int i = 0; i < XD; ++i) {
-    const int g = wave + 8 * i;
-    const int q = 64 * g + lane, row = q >> 3, part = (q & 7) ^ aswz(row);
-    xoff[i] = (uint32_t)((min(m0 + row, M - 1) - m0) * K + part * 8) * 2;
-    xdead[i] = m0 + 8 * g >= M;
-  }
-  // W: wave w moves rows 32 w + lane / 2, LDS half lane % 2 of the row (the row's half
-  // (lane % 2) ^ wswz(row) of the step's 32 bytes)
-  const int wr = 32 * wave + (lane >> 1);
-  const uint8_t *wb = w + (int64_t)n0 * wrow;
-  const uint32_t woff = (uint32_t)((min(n0 + wr, N - 1) - n0) * wrow) + 16 * ((lane & 1) ^ wswz(wr));
-  // scales: wave 0, lane l copies the scale dwords of rows 4 l .. 4 l + 3 (the step's 1 KiB block)
-  const uint8_t *sb = sp + (int64_t)(n0 >> 8) * steps * 1024;
-  const uint32_t soff = 16 * lane;
-  const bool sw = wave == 0;
-  auto issue = [&](int s) __attribute__((always_inline)) {
-    const uint32_t st = lds0 + (uint32_t)((s % V_STAGES) * G::STAGE);
+  for (int i = 0; i < NX; ++i) xo[i] = (uint32_t)(min(m0 + dr + 8 * G::NW * i, M - 1) - m0) * (uint32_t)(2 * K) + dp * 16;
 #pragma unroll
-    for (int i = 0; i < XD; ++i) {
-      if (xdead[i]) gp_dma4s(xb + s * 128, xoff[i], st + (wave + 8 * i) * 1024);
-      else gp_dma16s(xb + s * 128, xoff[i], st + (wave + 8 * i) * 1024);
+  for (int i = 0; i < NWD; ++i) wo[i] = (uint32_t)((min(n0 + dr + 8 * G::NW * i, N - 1) - n0) * wrow) + dp * 16;
+  // scales: the tile-major copy holds, per 256 rows and step, 256 dwords; a stage's V_SS x TN
+  // dwords take TN / 64 DMAs of four rows per lane, one per wave (the waves past that repeat one)
+  const int sq = (wave % (G::TN / 64)) * 64 + lane, sd = sq / (G::TN / 4), sr = n0 + sq % (G::TN / 4) * 4;
+  const uint8_t *sb = sp + ((int64_t)(sr >> 8) * steps * 256 + (sr & 255)) * 4;
+  const uint32_t sl = (uint32_t)(G::SOFF + (wave % (G::TN / 64)) * 1024);
+
+  auto issue_x = [&](int i, int s) __attribute__((always_inline)) {
+    gp_dma16s(xb + (int64_t)s * 128, xo[i], lds0 + (uint32_t)((s % SX) * G::XT + (wave + G::NW * i) * 1024));
+  };
+  auto issue_w = [&](int i, int g) __attribute__((always_inline)) {
+    gp_dma16s(wb + (int64_t)g * 128, wo[i], lds0 + (uint32_t)(G::WOFF + (g & 1) * G::WT + (wave + G::NW * i) * 1024));
+  };
+  // (a stage's steps past the last one repeat it)
+  auto issue_s = [&](int g) __attribute__((always_inline)) {
+    gp_dma16(sb + (int64_t)min(g * V_SS + sd, steps - 1) * 1024, lds0 + sl + (uint32_t)((g & 1) * G::ST));
+  };
+  // the x DMAs of step s, a whole one or the rows' last, whose pieces past K are zeros
+  auto issue_x_any = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+      if ((s + 1) * V_BK <= K) {
+        issue_x(i, s);
+      } else {
+        const uint8_t *p = xb + xo[i] + (int64_t)s * 128;
+        if (s * V_BK + 8 * dp >= K) p = (const uint8_t *)&nv_zero;
+        gp_dma16(p, lds0 + (uint32_t)((s % SX) * G::XT + (wave + G::NW * i) * 1024));
+      }
     }
-    gp_dma16s(wb + s * 32, woff, st + G::ATILE + wave * 1024);
-    if (sw) gp_dma16s(sb + s * 1024, soff, st + G::ATILE + V_WTILE);
+  };
+  // W DMAs [i0, i1) of stage g, likewise
+  auto issue_w_any = [&](int i0, int i1, int g) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NWD; ++i) {
+      if (i < i0 || i >= i1) continue;
+      if ((g + 1) * V_SS * V_BK <= K) {
+        issue_w(i, g);
+      } else {
+        const uint8_t *p = wb + wo[i] + (int64_t)g * 128;
+        if (g * V_SS * V_BK + 32 * dp >= K) p = (const uint8_t *)&nv_zero;
+        gp_dma16(p, lds0 + (uint32_t)(G::WOFF + (g & 1) * G::WT + (wave + G::NW * i) * 1024));
+      }
+    }
   };
 
-  // fragment geometry (32x32x16 bf16 operands: lane l holds row l % 32 and, in
-  // sub-step ks, the step's elements 32 fh + 8 ks + [0, 8) with fh = l / 32:
-  // x slot 4 fh + ks, W dword 4 fh + ks)
+  // Fragments (32x32x16 bf16 operands: lane l holds row l % 32 and half fh = l / 32 of the 16
+  // K): sub-step ks takes the step's elements 32 fh + 8 ks + [0, 8), piece 4 fh + ks of the x
+  // row; a lane's four W pieces are then the 16 bytes 2 j + fh of the W row (step j of its
+  // stage), and their scales bytes 2 fh and 2 fh + 1 of the row's dword.
   const int fr = lane & 31, fh = lane >> 5;
-  // (32 rows apart, fragments differ by whole 16-row swizzle periods, so one lane offset
-  // per sub-step serves every fragment: x fragment i of sub-step ks at xo[ks] + 4096 i, W
-  // fragment j at ob + 1024 j, its scale dword at os + 128 j)
-  const int ra = wm * WM + fr, rb = wn * WN + fr;
-  const int ab = (4 * fh) ^ aswz(ra);  // physical slot of logical slot 4 fh + ks is ks ^ ab
-  int xo[4];
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks) xo[ks] = ra * 128 + 16 * (ks ^ ab);
-  const int ob = G::ATILE + rb * 32 + 16 * (fh ^ wswz(rb));
-  const int os = G::ATILE + V_WTILE + rb * 4;
+  const int ra = wm * 32 * FI + fr, rb = wn * 32 * FJ + fr;
+  const int oa = ra * 128 + 16 * ((4 * fh) ^ nv_swz(ra));
+  const int ob = G::WOFF + rb * 128 + 16 * (fh ^ nv_swz(rb));
+  const int os = G::SOFF + rb * 4 + 2 * fh;
 
   f32x16_t acc[FI][FJ];
 #pragma unroll
@@ -147,306 +158,233 @@ __device__ __forceinline__ void nv_tile(int bid, const uint16_t *__restrict__ x,
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
 
-  // Ping-pong (as in the mxfp8 kernel): group 0 (waves 0-3) loads step k in interval 2k
-  // and computes it in 2k + 1, group 1 (waves 4-7) one interval later; each SIMD holds one
-  // wave of each group.
-  //   * Loading interval: every LDS read of the step (the W fragments and scales, and the
-  //     x fragments of all four sub-steps), then the DMAs of step k + 2, then the
-  //     dequantization of sub-step 0.  Stage k is therefore last read in interval 2k + 1,
-  //     and DMA(k + 2), which refills stage k - 1, can be issued by each group in its
-  //     loading interval of step k (2k, 2k + 1); at the barrier ending interval 2k + 1
-  //     every wave waits for its DMA(k + 1) (only DMA(k + 2), DMA_S / DMA loads, remain).
-  //   * Computing interval: the 32 MFMAs (8 per sub-step), with the dequantization of
-  //     sub-steps 1-3 interleaved, four VALU instructions after each MFMA.  The VALU work
-  //     runs beside the wave's own MFMAs, and both intervals of a SIMD carry some of it.
-  //     (Measured at lm_head prefill against other splits: all four sub-steps dequantized
-  //     in the loading interval 4.3% slower, two of them 1-2% slower; 3 or 2 VALU per
-  //     MFMA 5-8% slower; the DMAs issued before the LDS reads within 1%, after the
-  //     dequantization 5% slower.)
-  const int grp = wave >> 2;
-  issue(s_begin);
-  if (s_end - s_begin > 1) issue(s_begin + 1);
-  if (s_end - s_begin <= 1) gp_wait_barrier<0>();
-  else if (sw) gp_wait_barrier<G::DMA_S>();
-  else gp_wait_barrier<G::DMA>();
+  bf16x8_t af[2][FI], bf[2][FJ];  // sub-step ks's fragments, in set ks % 2
+  uint4 wq[FJ];                   // the step's W fragments as stored
+  uint32_t wsc[FJ];
+  auto read_x = [&](int s, int ks, int i) __attribute__((always_inline)) {
+    af[ks & 1][i] = *(const bf16x8_t *)(lds + (s % SX) * G::XT + (oa ^ (16 * ks)) + 4096 * i);
+  };
+  auto read_w = [&](int s, int j) __attribute__((always_inline)) {
+    const int g = s >> 2, t = s & 3;
+    wq[j] = *(const uint4 *)(lds + (g & 1) * G::WT + (ob ^ (32 * t)) + 4096 * j);
+    wsc[j] = *(const uint16_t *)(lds + (g & 1) * G::ST + os + t * (G::TN * 4) + 128 * j);
+  };
+  // pair p (of 4) of W fragment j for sub-step ks: E2M1 -> f32, times the scale, -> bf16, exact
+  auto deq = [&](int ks, int j, int p) __attribute__((always_inline)) {
+    const uint32_t word = ks == 0 ? wq[j].x : ks == 1 ? wq[j].y : ks == 2 ? wq[j].z : wq[j].w;
+    const float sc = ks < 2 ? __builtin_amdgcn_cvt_f32_fp8((int)wsc[j], 0) : __builtin_amdgcn_cvt_f32_fp8((int)wsc[j], 1);
+    f32x2_t v;
+    if (p == 0) v = fp4x2_to_f32x2<0>(word);
+    else if (p == 1) v = fp4x2_to_f32x2<1>(word);
+    else if (p == 2) v = fp4x2_to_f32x2<2>(word);
+    else v = fp4x2_to_f32x2<3>(word);
+    bf[ks & 1][j][2 * p] = (__bf16)(v.x * sc);
+    bf[ks & 1][j][2 * p + 1] = (__bf16)(v.y * sc);
+  };
+  constexpr int NM = FI * FJ, ND = 4 * FJ;  // MFMAs and dequantized pairs of a sub-step
 
-  auto pp_step = [&](auto grp_c, auto dma_c, int s) __attribute__((always_inline)) {
-    constexpr int GRP = decltype(grp_c)::value;
-    constexpr bool DMA = decltype(dma_c)::value;
-    const uint8_t *st = lds + (s % V_STAGES) * G::STAGE;
-    uint4 wq[FJ];
-    uint32_t wsc[FJ];
+  // Order of the DMAs: W and scales of the first stage, x of the first SX steps, the first
+  // half of the second stage; then at each step s, x of step s + SX followed by the second
+  // half of the next W stage (at a stage's first step) or the first half of the one after
+  // (at its last step).
+  issue_w_any(0, NWD, g_begin);
+  issue_s(g_begin);
+#pragma unroll 1
+  for (int t = 0; t < SX && s_begin + t < s_end; ++t) issue_x_any(s_begin + t);
+  if (g_begin + 1 < g_end) {
+    issue_w_any(0, NWD / 2, g_begin + 1);
+    issue_s(g_begin + 1);
+  }
+  if (g_begin + 1 < g_end && s_end - s_begin >= SX) gp_wait_barrier<(SX - 1) * NX + G::NA>();
+  else gp_wait_barrier<0>();
 #pragma unroll
-    for (int j = 0; j < FJ; ++j) {
-      wq[j] = *(const uint4 *)(st + ob + 1024 * j);
-      wsc[j] = *(const uint32_t *)(st + os + 128 * j);
-    }
-    bf16x8_t af[4][FI];
+  for (int j = 0; j < FJ; ++j) read_w(s_begin, j);
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
+  for (int i = 0; i < FI; ++i) read_x(s_begin, 0, i);
 #pragma unroll
-      for (int i = 0; i < FI; ++i) af[ks][i] = *(const bf16x8_t *)(st + xo[ks] + 4096 * i);
-    __builtin_amdgcn_sched_barrier(0);
-    if constexpr (DMA) issue(s + 2);
-    // W sub-step ks, fragment j: 8 nvfp4 elements times the E4M3 scale of group 2 fh + ks / 2
-    bf16x8_t bf[4][FJ];
-    auto deq = [&](int ks, int j) __attribute__((always_inline)) {
-      const uint32_t word = ks == 0 ? wq[j].x : ks == 1 ? wq[j].y : ks == 2 ? wq[j].z : wq[j].w;
-      bf[ks][j] = deq8_nvfp4(word, (wsc[j] >> (8 * (2 * fh + (ks >> 1)))) & 0xFF);
-    };
-#pragma unroll
-    for (int j = 0; j < FJ; ++j) deq(0, j);
-    // sub-step 0's W is pinned here, so that its VALU work stays in the loading interval
-#pragma unroll
-    for (int j = 0; j < FJ; ++j) asm volatile("" : "+v"(bf[0][j]));
-    __builtin_amdgcn_sched_barrier(0);
-    if constexpr (GRP == 0) gp_lds_barrier();  // ends interval 2s
-    else if constexpr (DMA) {                  // ends interval 2s + 1
-      if (sw) gp_wait_barrier<G::DMA_S>();
-      else gp_wait_barrier<G::DMA>();
-    } else {
-      gp_wait_barrier<0>();
-    }
-    __builtin_amdgcn_sched_barrier(0);
+  for (int d = 0; d < ND; ++d) deq(0, d % FJ, d / FJ);
+
+  // Step s = V_SS g + T.  Sub-step ks's MFMAs run beside the reads and the dequantization of
+  // the next sub-step's fragments.  Before sub-step 3 every read of the step's stages is done
+  // and, after the barrier, every wave's: its x stage, and after a W stage's last step that
+  // stage, are refilled.
+  // MODE 2: all of it whole; 3: as 2, but no W stage g + 2; 1: whatever is in the range, each
+  // barrier waiting for every DMA.
+  auto step = [&](auto mode_c, auto t_c, int g) __attribute__((always_inline)) {
+    constexpr int MODE = decltype(mode_c)::value, T = decltype(t_c)::value;
+    const int s = V_SS * g + T;
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
-      if (ks < 3) {
-#pragma unroll
-        for (int j = 0; j < FJ; ++j) deq(ks + 1, j);
+      if (ks == 3) {
+        if constexpr (MODE >= 2) gp_wait_barrier<G::in_flight(T)>();
+        else gp_wait_barrier<0>();
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (MODE == 1) {
+          if (s + SX < s_end) issue_x_any(s + SX);
+          if (T == 0 && g + 1 < g_end) issue_w_any(NWD / 2, NWD, g + 1);
+          if (T == 3 && g + 2 < g_end) {
+            issue_w_any(0, NWD / 2, g + 2);
+            issue_s(g + 2);
+          }
+        }
       }
+      // the DMAs of this sub-step: x, then W, the scales last
+      constexpr int NWH = T == 0 ? G::NB : T == 3 && MODE == 2 ? G::NA : 0;
+      constexpr int W0 = T == 0 ? NWD / 2 : 0;
+      constexpr int NI = NX + NWH;
 #pragma unroll
-      for (int j = 0; j < FJ; ++j)
+      for (int m = 0; m < NM; ++m) {
+        if (ks == 3) {
+          if constexpr (MODE >= 2) {
 #pragma unroll
-        for (int i = 0; i < FI; ++i)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[ks][i], bf[ks][j], acc[i][j], 0, 0, 0);
-    }
+            for (int i = m * NI / NM; i < (m + 1) * NI / NM; ++i) {
+              if (i < NX) issue_x(i, s + SX);
+              else if (T == 0) issue_w(W0 + i - NX, g + 1);
+              else if (i - NX < NWD / 2) issue_w(i - NX, g + 2);
+              else issue_s(g + 2);
+            }
+          }
+          if (m == 0) {
 #pragma unroll
-    for (int m = 0; m < 4 * FI * FJ; ++m) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-      __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);  // then four VALU
+            for (int j = 0; j < FJ; ++j) read_w(s + 1, j);
+          }
+#pragma unroll
+          for (int i = m * FI / NM; i < (m + 1) * FI / NM; ++i) read_x(s + 1, 0, i);
+          // the W fragments have arrived by the second half
+          if (2 * m >= NM || NM == 1) {
+            constexpr int H = NM - NM / 2;
+            const int mm = m - NM / 2;
+#pragma unroll
+            for (int d = mm * ND / H; d < (mm + 1) * ND / H; ++d) deq(0, d % FJ, d / FJ);
+          }
+        } else {
+#pragma unroll
+          for (int i = m * FI / NM; i < (m + 1) * FI / NM; ++i) read_x(s, ks + 1, i);
+#pragma unroll
+          for (int d = m * ND / NM; d < (m + 1) * ND / NM; ++d) deq(ks + 1, d % FJ, d / FJ);
+        }
+        const int j = m / FI, i = m % FI;
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[ks & 1][i], bf[ks & 1][j], acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
-    __builtin_amdgcn_sched_barrier(0);
-    if constexpr (GRP == 1) gp_barrier_only();  // ends interval 2s + 2 (no LDS read in it)
-    else if constexpr (DMA) {                   // ends interval 2s + 1
-      if (sw) gp_wait_barrier<G::DMA_S>();
-      else gp_wait_barrier<G::DMA>();
-    } else {
-      gp_wait_barrier<0>();
-    }
-    __builtin_amdgcn_sched_barrier(0);
   };
-  auto pp_run = [&](auto grp_c) __attribute__((always_inline)) {
-    constexpr int GRP = decltype(grp_c)::value;
-    if constexpr (GRP == 1) gp_barrier_only();  // group 1 starts one interval late
-    int s = s_begin;
-    for (; s + 2 < s_end; ++s) pp_step(grp_c, std::true_type{}, s);
-    for (; s < s_end; ++s) pp_step(grp_c, std::false_type{}, s);
-    if constexpr (GRP == 0) gp_barrier_only();  // matches group 1's extra barrier
-  };
-  if (grp == 0) pp_run(std::integral_constant<int, 0>{});
-  else pp_run(std::integral_constant<int, 1>{});
-  if (part) {  // a K range of a split tile: the raw accumulators
-    gp_store_partial<FI, FJ>(acc, part, wave, lane, M - (m0 + wm * WM));
+  using I0 = std::integral_constant<int, 0>;
+  using I1 = std::integral_constant<int, 1>;
+  using I2 = std::integral_constant<int, 2>;
+  using I3 = std::integral_constant<int, 3>;
+  int g = g_begin;
+  // the stages whose SX steps ahead and W stage ahead are whole (MODE 3: and W stage g + 2 is not)
+  const int whole = min(g_end, K / (V_SS * V_BK));
+#pragma unroll 1
+  for (; g + 2 < whole; ++g) {
+    step(I2{}, I0{}, g);
+    step(I2{}, I1{}, g);
+    step(I2{}, I2{}, g);
+    step(I2{}, I3{}, g);
+  }
+  if (g + 2 == whole && whole == g_end) {
+    step(I3{}, I0{}, g);
+    step(I3{}, I1{}, g);
+    step(I3{}, I2{}, g);
+    step(I3{}, I3{}, g);
+    ++g;
+  }
+#pragma unroll 1
+  for (; g < g_end; ++g) {
+    const int n = s_end - V_SS * g;
+    step(I1{}, I0{}, g);
+    if (n > 1) step(I1{}, I1{}, g);
+    if (n > 2) step(I1{}, I2{}, g);
+    if (n > 3) step(I1{}, I3{}, g);
+  }
+  gp_lds_barrier();
+
+  const int row0 = m0 + wm * 32 * FI, col0 = n0 + wn * 32 * FJ;
+  if (blk.split) {
+    gp_store_partial<FI, FJ, G::NW>(acc, part + (size_t)((blk.t - whole_tiles) * S + blk.kr) * G::TM * G::TN, wave, lane,
+                                    M - row0);
     return;
   }
-  (void)steps;
-
-  // epilogue through LDS (the ring is idle: every wave has passed the last barrier, after
-  // which no fragment read or DMA is outstanding), in two halves of the wave's 128 rows
-  // so that the eight regions fit the ring
-  constexpr int NI = FI < 2 ? FI : 2;  // accumulator rows per half
-  constexpr int REGION = 32 * NI * (64 * FJ + 32);
-  // (the 256- and 128-row instances run with the 256-row ring, the 64-row one with its own)
-  static_assert(8 * REGION <= (TM == 64 ? G::LDS : V_LDS), "the epilogue regions fit the launch's ring");
   const bool vec = yout_vec(yo);
-  uint8_t *region = lds + wave * REGION;
-  gp_store_tile_bf16<FI, FJ, 0, NI>(acc, region, lane, yo, M, m0 + wm * WM, n0 + wn * WN, n_end, vec);
-  if constexpr (FI == 4)
-    gp_store_tile_bf16<FI, FJ, 2, 2>(acc, region, lane, yo, M, m0 + wm * WM, n0 + wn * WN, n_end, vec);
+  uint8_t *region = lds + wave * G::REGION;
+  gp_store_rows<FI, FJ, 0>(acc, region, lane, yo, M, row0, col0, N, vec);
 }
 
-__global__ __launch_bounds__(V_THREADS) void gemm_nvfp4_pipe_kernel(const uint16_t *__restrict__ x,
-                                                                    const uint8_t *__restrict__ w,
-                                                                    const uint8_t *__restrict__ sp,
-                                                                    const YOut yo, int M, int N, int K) {
-  nv_tile<256>(blockIdx.x, x, w, sp, yo, M, N, K, 0, N, 0, K / V_BK, nullptr);
+template <class G>
+__global__ __launch_bounds__(256) void gemm_nvfp4_reduce_kernel(const float *__restrict__ part, const YOut yo, int M,
+                                                                int N, int whole_tiles, int S) {
+  gp_reduce_tile<G>(part, yo, M, N, whole_tiles, S, blockIdx.x * 256 + threadIdx.x);
 }
 
-// Every TM x 256 tile split S ways along K: block b runs K range b % S of tile b / S and
-// leaves its fp32 accumulators in slot b of `part` (TM KiB each); gemm_nvfp4_split_reduce
-// then sums them.  For calls of fewer tiles than CUs (short prefill chunks, narrow
-// projections), which would otherwise leave most CUs idle.  The 64-row instance (x of at
-// most 64 rows) moves 17 KiB per K step and runs two blocks per CU (its 51 KiB ring and
-// at most 128 registers per lane), so a CU keeps two blocks' loads in flight.
-template <int TM>
-__device__ __forceinline__ void nv_ksplit_block(const uint16_t *__restrict__ x, const uint8_t *__restrict__ w,
-                                                const uint8_t *__restrict__ sp, const YOut yo, int M,
-                                                int N, int K, int S, float *__restrict__ part) {
-  const int b = blockIdx.x, t = b / S, k = b - t * S, steps = K / V_BK;
-  nv_tile<TM>(t, x, w, sp, yo, M, N, K, 0, N, k * steps / S, (k + 1) * steps / S,
-              part ? part + (size_t)b * TM * 256 : nullptr);
-}
-template <int TM>
-__global__ __launch_bounds__(V_THREADS) void gemm_nvfp4_pipe_ksplit_kernel(const uint16_t *__restrict__ x,
-                                                                           const uint8_t *__restrict__ w,
-                                                                           const uint8_t *__restrict__ sp,
-                                                                           const YOut yo, int M, int N,
-                                                                           int K, int S, float *__restrict__ part) {
-  nv_ksplit_block<TM>(x, w, sp, yo, M, N, K, S, part);
-}
-__global__ __launch_bounds__(V_THREADS, 2) void gemm_nvfp4_pipe_ksplit64_kernel(const uint16_t *__restrict__ x,
-                                                                                const uint8_t *__restrict__ w,
-                                                                                const uint8_t *__restrict__ sp,
-                                                                                const YOut yo, int M,
-                                                                                int N, int K, int S,
-                                                                                float *__restrict__ part) {
-  nv_ksplit_block<64>(x, w, sp, yo, M, N, K, S, part);
+// ---------------------------------------------------------------- the plan
+
+namespace {
+using Nv256 = NvGeom<8, 2, 1, 4, 2>;  // 256 x 256
+using Nv192 = NvGeom<6, 2, 1, 4, 2>;  // 192 x 256
+using NvW = NvGeom<4, 2, 1, 4, 2>;    // 128 x 256
+using Nv128 = NvGeom<4, 1, 1, 4, 2>;  // 128 x 128, two blocks per CU
+using Nv64 = NvGeom<2, 1, 1, 4, 4>;   // 64 x 128, two blocks per CU
+using Nv32 = NvGeom<1, 1, 1, 4, 4>;   // 32 x 128, three blocks per CU
+// (fitted to 45 shapes of the declared range with every tile and split, rms error 7%; the
+// plan's choice is 1.01 of the best of them on average, at most 1.26)
+constexpr GpCost NV_COST[] = {{256, 256, 1, 9.7f, {1.10f}},         {192, 256, 1, 8.9f, {0.86f}},
+                              {128, 256, 1, 9.7f, {0.58f}},         {128, 128, 2, 7.8f, {0.42f, 0.69f}},
+                              {64, 128, 2, 8.6f, {0.26f, 0.43f}},   {32, 128, 3, 8.4f, {0.22f, 0.34f, 0.48f}}};
+}  // namespace
+
+static GpPlan nv_plan(const QmmArgs &a) {
+  return gp_plan(NV_COST, sizeof(NV_COST) / sizeof(NV_COST[0]), a.M, a.N, (a.K + V_BK - 1) / V_BK, V_SS,
+                 device_cu_count());
 }
 
-// The split tiles' results: one thread per float4 of a tile's partial layout
-// (gp_reduce_quad), 8 * FI * FJ * 4 * 64 threads per tile, nv_reduce_blocks<TM> blocks of 256.
-template <int TM>
-constexpr int nv_reduce_blocks() {
-  return TM == 64 ? 2 * 2 * 1 * 4 : 2 * (TM / 64) * 2 * 4;  // 2 * FI * FJ * 4
-}
-template <int TM>
-__global__ __launch_bounds__(256) void gemm_nvfp4_split_reduce_kernel(const float *__restrict__ part,
-                                                                       const YOut yo, int M, int N, int S) {
-  // the wave layout of nv_tile<TM>
-  constexpr bool COLS = TM == 64;
-  constexpr int FI = COLS ? 2 : TM / 64, FJ = COLS ? 1 : 2;
-  constexpr int WM = COLS ? TM : TM / 2, WN = 32 * FJ;
-  constexpr int NQ = FI * FJ * 4;  // float4s per lane per wave
-  static_assert(8 * NQ * 64 == 256 * nv_reduce_blocks<TM>(), "whole blocks per tile");
-  const int g = blockIdx.x * 256 + threadIdx.x;
-  const int t = g / (8 * NQ * 64), rem = g - t * (8 * NQ * 64);
-  const int wave = rem / (NQ * 64), q = (rem >> 6) % NQ, lane = rem & 63;
-  int tm, tn;
-  tile_of(t, (M + TM - 1) / TM, (N + V_BN - 1) / V_BN, &tm, &tn);
-  const int wm = COLS ? 0 : wave & 1, wn = COLS ? wave : wave >> 1;
-  gp_reduce_quad<FI, FJ>(part, yo, M, N, t, S, wave, q, lane, tm * TM + wm * WM, tn * V_BN + wn * WN);
+template <class G>
+static hipError_t launch_nv(const QmmArgs &a, const GpPlan &p, const uint8_t *tiled, float *part, hipStream_t st) {
+  static std::atomic<uint64_t> lds_set{0};
+  hipError_t e = ensure_dynamic_lds(lds_set, (const void *)gemm_nvfp4_kernel<G>, G::LDS);
+  if (e != hipSuccess) return e;
+  const YOut yo = yout_of(a);  // y, or a grouped call's parts
+  hipLaunchKernelGGL((gemm_nvfp4_kernel<G>), dim3(p.whole + p.left * p.S), dim3(G::THREADS), G::LDS, st,
+                     (const uint16_t *)a.x, a.w, tiled, yo, a.M, a.N, a.K, p.whole, p.S, part);
+  e = hipGetLastError();
+  if (e != hipSuccess || p.left == 0) return e;
+  hipLaunchKernelGGL((gemm_nvfp4_reduce_kernel<G>), dim3(p.left * (G::NW * G::FI * G::FJ)), dim3(256), 0, st,
+                     (const float *)part, yo, a.M, a.N, p.whole, p.S);
+  return hipGetLastError();
 }
 
-// Both tile heights in one launch: blocks [0, tiles1) are the 256-row tiles of W rows
-// [0, n_split), the rest the 128-row tiles of W rows [n_split, N).  Blocks start in
-// index order as CUs free up, so a partial last round of 256-row tiles runs as twice as
-// many half tiles, each moving 25 of the 41 KiB a full tile moves per K step.
-__global__ __launch_bounds__(V_THREADS) void gemm_nvfp4_pipe_split_kernel(const uint16_t *__restrict__ x,
-                                                                          const uint8_t *__restrict__ w,
-                                                                          const uint8_t *__restrict__ sp,
-                                                                          const YOut yo, int M, int N,
-                                                                          int K, int n_split, int tiles1) {
-  const int b = blockIdx.x, steps = K / V_BK;
-  if (b < tiles1)
-    nv_tile<256>(b, x, w, sp, yo, M, N, K, 0, n_split, 0, steps, nullptr);
-  else
-    nv_tile<128>(b - tiles1, x, w, sp, yo, M, N, K, n_split, N, 0, steps, nullptr);
-}
-
-static size_t round256v(size_t v) { return (v + 255) & ~(size_t)255; }
-
-// K % 64 (whole steps; the scale dword of a step is 4 groups); x and W rows
-// 16-byte aligned for the DMA, scale rows 4-byte aligned for the repack.
+// K % 32: 16-byte W pieces; x and W rows 16-byte aligned for the DMA.
 bool gemm_nvfp4_ok(const QmmArgs &a) {
-  return a.mode == NVFP4 && !a.x_f32 && a.K % V_BK == 0 && a.K > 0 && a.M > 0 && a.N > 0 &&
-         (uintptr_t)a.x % 16 == 0 && (uintptr_t)a.w % 16 == 0 && (uintptr_t)a.s % 4 == 0;
+  return a.mode == NVFP4 && !a.x_f32 && a.K % 32 == 0 && a.K > 0 && a.M > 0 && a.N > 0 && (uintptr_t)a.x % 16 == 0 &&
+         (uintptr_t)a.w % 16 == 0;
 }
 
-// x of at most 128 rows runs its own tile height, 64 rows (two blocks per CU) up to 64
-// rows and 128 up to 128, split S ways along K where the tiles leave block slots idle (at
-// most one round of blocks, each at least 8 K steps) and whole (S = 1, stored directly)
-// where there are more tiles than slots.  Taller x runs 256-row tiles, split the same way
-// when a call has at most half as many tiles as CUs: the plan, or S = 0 for the
-// whole-tile paths.
-struct NvSplit {
-  int TM, tiles, S;
-};
-static NvSplit nv_split_plan(const QmmArgs &a, int cus) {
-  const int TM = a.M <= 64 ? 64 : a.M <= 128 ? 128 : 256;
-  const int T = ((a.M + TM - 1) / TM) * ((a.N + V_BN - 1) / V_BN), steps = a.K / V_BK;
-  if (cus <= 0 || (TM == 256 && 2 * T > cus)) return NvSplit{TM, T, 0};
-  int S = (TM == 64 ? 2 * cus : cus) / T;
-  if (S > 8) S = 8;
-  if (S > steps / 8) S = steps / 8;
-  if (S >= 2) return NvSplit{TM, T, S};
-  return NvSplit{TM, T, TM == 256 ? 0 : 1};
-}
-
-// Workspace: the scales repacked tile-major, unless they come so (a.s_tiled), then (split
-// tiles) the fp32 partial sums, TM KiB per block, 256-byte aligned.
+// Workspace: the scales repacked tile-major, unless they come so (a.s_tiled), then the split
+// tiles' fp32 partial sums.
+static size_t nv_scales_bytes(const QmmArgs &a) { return a.s_tiled ? 0 : tiled_scales_bytes(a.N, a.K / 16); }
 size_t gemm_nvfp4_workspace(const QmmArgs &a) {
-  size_t bytes = a.s_tiled ? 0 : round256v(a.N) * (size_t)(a.K / 16);
-  const NvSplit p = nv_split_plan(a, device_cu_count());
-  if (p.S >= 2) bytes = round256v(bytes) + (size_t)p.tiles * p.S * p.TM * 256 * 4;
-  return bytes + 256;
+  const GpPlan p = nv_plan(a);
+  return nv_scales_bytes(a) + (size_t)p.left * p.S * NV_COST[p.cfg].TM * NV_COST[p.cfg].TN * sizeof(float);
 }
 
 hipError_t launch_gemm_nvfp4(const QmmArgs &a, void *ws, hipStream_t st) {
   if (!gemm_nvfp4_ok(a)) return hipErrorInvalidValue;
-  hipError_t e = hipSuccess;
   const uint8_t *tiled = (const uint8_t *)a.s_tiled;
   if (!tiled) {
-    e = launch_repack_scales(a.s, (int64_t)a.N, a.K / 16, (uint32_t *)ws, st);
+    const hipError_t e = launch_repack_scales(a.s, (int64_t)a.N, a.K / 16, (uint32_t *)ws, st);
     if (e != hipSuccess) return e;
     tiled = (const uint8_t *)ws;
   }
-  static std::atomic<uint64_t> lds_set{0}, lds_split{0}, lds_k256{0}, lds_k128{0}, lds_k64{0};
-  e = ensure_dynamic_lds(lds_set, (const void *)gemm_nvfp4_pipe_kernel, (int)V_LDS);
-  if (e == hipSuccess) e = ensure_dynamic_lds(lds_split, (const void *)gemm_nvfp4_pipe_split_kernel, (int)V_LDS);
-  if (e == hipSuccess) e = ensure_dynamic_lds(lds_k256, (const void *)gemm_nvfp4_pipe_ksplit_kernel<256>, (int)V_LDS);
-  if (e == hipSuccess) e = ensure_dynamic_lds(lds_k128, (const void *)gemm_nvfp4_pipe_ksplit_kernel<128>, (int)V_LDS);
-  if (e == hipSuccess)
-    e = ensure_dynamic_lds(lds_k64, (const void *)gemm_nvfp4_pipe_ksplit64_kernel, (int)NvGeom<64>::LDS);
-  if (e != hipSuccess) return e;
-  const YOut yo = yout_of(a);  // y, or a grouped call's parts
-  const NvSplit sp = nv_split_plan(a, device_cu_count());
-  if (sp.S) {
-    // (S = 1: whole tiles of this height, stored directly: no partial sums, no reduce)
-    float *part = sp.S >= 2 ? (float *)((uint8_t *)ws + round256v(a.s_tiled ? 0 : round256v(a.N) * (size_t)(a.K / 16)))
-                            : nullptr;
-    const int blocks = sp.tiles * sp.S;
-    if (sp.TM == 64) {
-      hipLaunchKernelGGL(gemm_nvfp4_pipe_ksplit64_kernel, dim3(blocks), dim3(V_THREADS), NvGeom<64>::LDS, st,
-                         (const uint16_t *)a.x, a.w, tiled, yo, a.M, a.N, a.K, sp.S, part);
-      e = hipGetLastError();
-      if (e == hipSuccess && part)
-        hipLaunchKernelGGL(gemm_nvfp4_split_reduce_kernel<64>, dim3(sp.tiles * nv_reduce_blocks<64>()), dim3(256), 0,
-                           st, (const float *)part, yo, a.M, a.N, sp.S);
-    } else if (sp.TM == 128) {
-      hipLaunchKernelGGL(gemm_nvfp4_pipe_ksplit_kernel<128>, dim3(blocks), dim3(V_THREADS), V_LDS, st,
-                         (const uint16_t *)a.x, a.w, tiled, yo, a.M, a.N, a.K, sp.S, part);
-      e = hipGetLastError();
-      if (e == hipSuccess && part)
-        hipLaunchKernelGGL(gemm_nvfp4_split_reduce_kernel<128>, dim3(sp.tiles * nv_reduce_blocks<128>()), dim3(256), 0,
-                           st, (const float *)part, yo, a.M, a.N, sp.S);
-    } else {
-      hipLaunchKernelGGL(gemm_nvfp4_pipe_ksplit_kernel<256>, dim3(blocks), dim3(V_THREADS), V_LDS, st,
-                         (const uint16_t *)a.x, a.w, tiled, yo, a.M, a.N, a.K, sp.S, part);
-      e = hipGetLastError();
-      if (e == hipSuccess && part)
-        hipLaunchKernelGGL(gemm_nvfp4_split_reduce_kernel<256>, dim3(sp.tiles * nv_reduce_blocks<256>()), dim3(256), 0,
-                           st, (const float *)part, yo, a.M, a.N, sp.S);
-    }
-    return e == hipSuccess ? hipGetLastError() : e;
+  float *part = (float *)((uint8_t *)ws + nv_scales_bytes(a));  // (a multiple of 1 KiB)
+  const GpPlan p = nv_plan(a);
+  switch (p.cfg) {
+    case 0: return launch_nv<Nv256>(a, p, tiled, part, st);
+    case 1: return launch_nv<Nv192>(a, p, tiled, part, st);
+    case 2: return launch_nv<NvW>(a, p, tiled, part, st);
+    case 3: return launch_nv<Nv128>(a, p, tiled, part, st);
+    case 4: return launch_nv<Nv64>(a, p, tiled, part, st);
+    default: return launch_nv<Nv32>(a, p, tiled, part, st);
   }
-  // When the 256 x 256 tiles leave a partial last round of whole tile-columns that half
-  // the CUs or fewer would run, those columns run as 128 x 256 tiles in the same launch.
-  const int tiles_m = (a.M + V_BM - 1) / V_BM, tiles_n = (a.N + V_BN - 1) / V_BN;
-  const int cus = device_cu_count();
-  const int rem = cus > 0 ? (tiles_m * tiles_n) % cus : 0;
-  int n_split = a.N;
-  if (rem != 0 && rem % tiles_m == 0 && 2 * rem <= cus && tiles_m * tiles_n > cus)
-    n_split = (tiles_n - rem / tiles_m) * V_BN;
-  const int tiles1 = tiles_m * ((n_split + V_BN - 1) / V_BN);
-  if (n_split == a.N) {
-    hipLaunchKernelGGL(gemm_nvfp4_pipe_kernel, dim3(tiles1), dim3(V_THREADS), V_LDS, st, (const uint16_t *)a.x, a.w,
-                       tiled, yo, a.M, a.N, a.K);
-    return hipGetLastError();
-  }
-  const int tiles2 = ((a.M + 127) / 128) * ((a.N - n_split + V_BN - 1) / V_BN);
-  hipLaunchKernelGGL(gemm_nvfp4_pipe_split_kernel, dim3(tiles1 + tiles2), dim3(V_THREADS), V_LDS, st,
-                     (const uint16_t *)a.x, a.w, tiled, yo, a.M, a.N, a.K, n_split, tiles1);
-  return hipGetLastError();
 }
 
 }  // namespace qmm

@@ -26,6 +26,40 @@ __device__ __forceinline__ void tile_of(int b, int tiles_m, int tiles_n, int *tm
   *tn = idx / gm;
 }
 
+// A call's blocks: [0, whole_tiles) run whole tiles, the others the S K-ranges of the tiles
+// that are left (whole_tiles on).  Tiles are numbered in tile_of's order; each XCD (block %
+// 8) takes a contiguous run, and of a call that is all split, at few x tiles, the x tiles of
+// one W range of one K range run next to each other, so that they share its W.
+struct GpBlock {
+  int t, tm, tn, kr;
+  bool split;
+};
+__device__ __forceinline__ void gp_tile_at(int t, int tiles_m, int tiles_n, int *tm, int *tn) {
+  constexpr int G = 4;
+  const int first = t / (G * tiles_n) * G, gm = min(tiles_m - first, G), i = t - first * tiles_n;
+  *tm = first + i % gm;
+  *tn = i / gm;
+}
+__device__ __forceinline__ int gp_xcd_run(int b, int n) {
+  const int base = n / 8, rem = n % 8, x = b % 8;
+  return x * base + min(x, rem) + b / 8;
+}
+__device__ __forceinline__ GpBlock gp_block(int b, int tiles_m, int tiles_n, int whole_tiles, int S) {
+  GpBlock r;
+  r.split = b >= whole_tiles;
+  r.kr = 0;
+  if (!r.split) {
+    r.t = gp_xcd_run(b, whole_tiles);
+  } else {
+    const int left = tiles_m * tiles_n - whole_tiles, u = gp_xcd_run(b - whole_tiles, left * S);
+    const int gm = whole_tiles == 0 && tiles_m <= 4 ? tiles_m : 1;
+    r.kr = u / gm % S;
+    r.t = whole_tiles + u / (gm * S) * gm + u % gm;
+  }
+  gp_tile_at(r.t, tiles_m, tiles_n, &r.tm, &r.tn);
+  return r;
+}
+
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
 // LDS DMA: lane i's 16 (4) bytes at g land at LDS byte l + 16 i (4 i); l must be
@@ -190,34 +224,104 @@ __device__ __forceinline__ void gp_reduce_quad(const float *__restrict__ part, c
     if (r + e < M) *yo.at(r + e, c) = __builtin_bit_cast(uint16_t, (__bf16)v[e]);
 }
 
+// The same for a kernel of geometry G (tiles of TM x TN, WM x WN waves of 32 FI x 32 FJ),
+// thread i of the call: the tiles whole_tiles on, in gp_tile_at's order.
+template <class G>
+__device__ __forceinline__ void gp_reduce_tile(const float *__restrict__ part, const YOut yo, int M, int N,
+                                               int whole_tiles, int S, int i) {
+  constexpr int NQ = G::FI * G::FJ * 4, TILE = G::NW * NQ * 64;
+  static_assert(TILE % 256 == 0, "whole blocks per tile");
+  const int t = i / TILE, rem = i - t * TILE;
+  const int wave = rem / (NQ * 64), q = (rem >> 6) % NQ, lane = rem & 63;
+  int tm, tn;
+  gp_tile_at(whole_tiles + t, (M + G::TM - 1) / G::TM, (N + G::TN - 1) / G::TN, &tm, &tn);
+  gp_reduce_quad<G::FI, G::FJ, G::NW>(part, yo, M, N, t, S, wave, q, lane, tm * G::TM + (wave % G::WM) * 32 * G::FI,
+                                      tn * G::TN + (wave / G::WM) * 32 * G::FJ);
+}
+
+// gp_store_tile_bf16 of all FI accumulator rows, one at a time.
+template <int FI, int FJ, int I>
+__device__ __forceinline__ void gp_store_rows(const f32x16_t (&acc)[FI][FJ], uint8_t *region, int lane, const YOut yo,
+                                              int M, int row0, int col0, int col_end, bool vec) {
+  gp_store_tile_bf16<FI, FJ, I, 1>(acc, region, lane, yo, M, row0, col0, col_end, vec);
+  if constexpr (I + 1 < FI) gp_store_rows<FI, FJ, I + 1>(acc, region, lane, yo, M, row0, col0, col_end, vec);
+}
+
+// y as one part.
+__device__ __forceinline__ YOut yout_one(uint16_t *y, int N) {
+  return YOut{y, nullptr, nullptr, nullptr, INT32_MAX, INT32_MAX, INT32_MAX, N, 0, 0, 0};
+}
+
 // Weight scales [N, nb bytes] (row-major, as loaded) -> tile-major: for each
 // 256-row tile and each dword column d of the rows, 256 contiguous dwords (one
-// per row): out[((tile * (nb / 4) + d) * 256 + r % 256] = row r's dword d.  A
-// thread reads CH consecutive dwords of one row; rows past N (up to the next
-// multiple of 256) repeat row N - 1.  Consecutive threads take consecutive rows,
+// per row): out[((tile * dpr + d) * 256 + r % 256] = row r's dword d, dpr = ceil(nb / 4),
+// the bytes past nb zero.  A thread reads CH consecutive dwords of one row (CH = 0: one
+// dword, byte by byte, for rows that are not whole aligned dwords); rows past N (up to the
+// next multiple of 256) repeat row N - 1.  Consecutive threads take consecutive rows,
 // so every write is coalesced.
 template <int CH>
 __global__ __launch_bounds__(256) void repack_scales_kernel(const uint8_t *__restrict__ s, int64_t N, int nb,
                                                             uint32_t *__restrict__ out) {
-  const int dpr = nb >> 2, chunks = dpr / CH;  // host: dpr % CH == 0
+  constexpr int C = CH ? CH : 1;
+  const int dpr = (nb + 3) >> 2, chunks = dpr / C;  // host: dpr % C == 0
   const int64_t total = ((N + 255) >> 8) * chunks * 256;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
     const int64_t rr = i & 255, tc = i >> 8;
     const int64_t tile = tc / chunks, c = tc % chunks;
     const int64_t r = min(tile * 256 + rr, N - 1);
-    const uint8_t *src = s + r * nb + 4 * CH * c;
-    uint32_t d[CH];
+    const uint8_t *src = s + r * nb + 4 * C * c;
+    uint32_t d[C];
     if constexpr (CH == 4) {
       const uint4 u = *(const uint4 *)src;
       d[0] = u.x, d[1] = u.y, d[2] = u.z, d[3] = u.w;
-    } else {
+    } else if constexpr (CH == 1) {
       d[0] = *(const uint32_t *)src;
+    } else {
+      d[0] = 0;
+      for (int b = 0; b < 4 && 4 * c + b < nb; ++b) d[0] |= (uint32_t)src[b] << (8 * b);
     }
 #pragma unroll
-    for (int k = 0; k < CH; ++k) out[((tile * dpr + CH * c + k) << 8) + rr] = d[k];
+    for (int k = 0; k < C; ++k) out[((tile * dpr + C * c + k) << 8) + rr] = d[k];
   }
 }
 
-// Host: launch the repack (16-byte reads when the rows allow it); declared in qmm_launch.h.
+// ---------------------------------------------------------------- host: the plan of a call
+
+// A tile size: TM x TN, per_cu blocks of it on a CU, and its measured cost: us per K step with
+// 1, 2, .. blocks on every CU, and us per round beside that.
+struct GpCost {
+  int TM, TN, per_cu;
+  float round, step[3];
+};
+struct GpPlan {
+  int cfg, whole, left, S;  // whole tiles, then `left` tiles split S ways along K
+};
+// The least estimated time over every tile size and every split of the tiles left after the
+// whole rounds (at most GP_MAX_SPLIT ways, one round of blocks, at least 4 K steps each, in
+// units of `unit` steps).  A split adds the reduce: its launch and its partial sums' traffic.
+inline GpPlan gp_plan(const GpCost *costs, int n, int M, int N, int steps, int unit, int cus) {
+  if (cus <= 0) cus = 256;  // (no device answers: the launch reports it)
+  GpPlan best{0, 0, 0, 1};
+  float best_us = 1e30f;
+  for (int c = 0; c < n; ++c) {
+    const GpCost &d = costs[c];
+    const int64_t T = (int64_t)((M + d.TM - 1) / d.TM) * ((N + d.TN - 1) / d.TN);
+    const int64_t slots = (int64_t)cus * d.per_cu, whole = T / slots * slots, left = T - whole;
+    const float base = (float)(whole / slots) * ((float)steps * d.step[d.per_cu - 1] + d.round);
+    const int units = (steps + unit - 1) / unit;
+    for (int S = 1; S <= GP_MAX_SPLIT; ++S) {
+      if (S > 1 && (left == 0 || left * S > slots || units < S || steps < 4 * S)) break;
+      float us = base;
+      if (left) {
+        const int per = (int)((left * S + cus - 1) / cus), mine = (units + S - 1) / S * unit;
+        us += (float)(mine < steps ? mine : steps) * d.step[(per < d.per_cu ? per : d.per_cu) - 1] + d.round;
+      }
+      if (S > 1) us += 1.5f + (float)left * S * (M < d.TM ? M : d.TM) * d.TN * 8.f / 6.6e6f;
+      if (us < best_us) best_us = us, best = GpPlan{c, (int)whole, (int)left, S};
+    }
+  }
+  if (best.S == 1) best.whole += best.left, best.left = 0;
+  return best;
+}
 
 }  // namespace qmm

@@ -365,6 +365,36 @@ def test_dense_linear_tiles(M, N, K):
     assert torch.all((y.double() - ref).abs() <= bound)
 
 
+@pytest.mark.parametrize("mode", ["nvfp4", "mxfp8"])
+@pytest.mark.parametrize("M,N,K", [
+    (17, 1, 32), (33, 129, 96), (64, 257, 224), (65, 300, 288),       # K ends inside a step or a stage of W
+    (33, 1000, 1056), (200, 320, 1024), (372, 328, 3456),             # tiles split along K
+    (68, 2700, 3392), (383, 2416, 992), (1030, 1000, 544),            # 64- and 128-row tiles
+    (520, 5000, 256), (1691, 10240, 288), (2049, 16480, 512),         # 256-wide tiles, rounds and tiles left over
+])
+def test_prefill_tiles(mode, M, N, K):
+    """The prefill GEMMs at the edges of their tiles, K steps, W stages and splits, against
+    float64 on the GPU: within the bf16 rounding (2^-8 of the value) and the fp32 sums' (and
+    the mxfp8 split of x, at most 2^-12 of a block's largest) error, below 2^-12 + K 2^-24 of
+    sum |x| |w| taken with each 32-block's largest |x|."""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + N + K)
+    x = torch.randn((M, K), generator=gen, device="cuda").to(torch.bfloat16)
+    W = (torch.randn((N, K), generator=gen, device="cuda") * 0.02).to(torch.bfloat16)
+    st = Q.Stream.torch_current()
+    wq, sc = Q.quantize(Q.Array.from_torch(W), mode, stream=st)
+    Wd = torch.empty((N, K), dtype=torch.float32, device="cuda")
+    Wd.copy_(torch.from_numpy(Q.dequantize(wq, sc, mode, dtype=Q.FLOAT32, stream=st).numpy(st)))
+    y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+    for _ in range(2):
+        Q.quantized_matmul(Q.Array.from_torch(x), wq, sc, mode, out=Q.Array.from_torch(y), stream=st)
+    ref = x.double() @ Wd.double().t()
+    xm = x.double().abs().view(M, K // 32, 32).amax(-1, keepdim=True).expand(M, K // 32, 32).reshape(M, K)
+    eps = K * 2.0 ** -24 + (2.0 ** -12 if mode == "mxfp8" else 0.0)
+    bound = ref.abs() * 2.0 ** -8 + (xm @ Wd.double().abs().t()) * eps + 1e-30
+    assert torch.all((y.double() - ref).abs() <= bound)
+
+
 # ---------------------------------------------------------------- MLP activation and the fused gate/up
 def test_silu_mul_matches_oracle():
     """src/model.zig:405-415 / :451-456 on the GPU: bf16 chain within one ulp of the
