@@ -13,10 +13,23 @@
 // two scaled MFMAs (hi, lo) per weight fragment into the same accumulator:
 // the weight tile is loaded once, the MFMA work doubles.
 //
-// Tiling: 512 threads (8 waves, 4 x 2), block tile 256 (x rows) x 256 (W rows),
-// K step 64, LDS double-buffered (rows padded to 80 bytes: conflict-free
-// 16-byte fragment reads), one barrier per K step; each wave owns 64 x 128
-// as 2 x 4 32x32 accumulators.
+// What bounds it: at tall x the matrix cores at the clock the power limit leaves (a large
+// fp8 library product reaches ~3.07 PFLOP/s here; 2048 x 34816 x 5120 runs at 2.93, hi and lo
+// both counted), at short x the latency of a step.  So:
+//   * K steps of 64: a row's hi and lo bytes of a step lie together, 128 bytes, a cache line;
+//     W moves in stages of two steps, 128 bytes per row too (64 wasted half of each line).
+//   * x and W go to LDS rings by DMA; the lo fragments are read beside the products of the
+//     hi parts, the next step's beside those of the lo parts; one barrier per step.
+//   * The tile is chosen per call (mx_plan), and the tiles left over after the whole rounds are
+//     split along K over the idle CUs, fp32 partial sums reduced in K order (deterministic) by
+//     a second kernel.
+// Measured, us per call with the split, weights cold (M x N x K; the former kernel, two groups
+// of waves in turns, two barriers per step, in brackets): 2048 x 5120 x 17408  272 (322),
+// 2048 x 17408 x 5120  269 (282), 200 x 5120 x 17408  54 (61), 48 x 17408 x 5120  35 (46),
+// 385 x 4129 x 1280  20 (32); K % 128 != 0, which ran unpipelined kernels: 68 x 27408 x 3392
+// 41 (199), 147 x 2181 x 8672  25 (325).
+// gate, up and silu(gate) * up of an MLP in one launch (MLP below), 2048 x (2 x 17408) x 5120:
+// 556 us and a reduce of 13, against 268 + 268 and 78 for silu * mul over memory.
 #include <type_traits>
 
 #include "gemm_pipe.h"
@@ -27,29 +40,8 @@ namespace qmm {
 
 // ---------------------------------------------------------------- x split pre-pass
 
-// LDS / pre-tiled operand swizzle of the pipelined GEMM: 16-byte slot p of row r
-// (64 bytes of one K step) is stored at slot p ^ p_swz(r) of the row.
-__host__ __device__ __forceinline__ int p_swz(int r) { return ((r >> 1) ^ (r >> 2)) & 3; }
+constexpr int X_BK = 64;  // K elements of a step: 64 bytes of hi and 64 of lo of an x row
 
-// Scale byte of (row r, 32-block b) in the tile-major layout the pipelined GEMM
-// loads: [r / 256][b / 4][r % 256][b % 4], i.e. for each 256-row tile and pair of
-// 64-wide K steps, 256 contiguous dwords (one per row).  Needs K % 128 == 0.
-__host__ __device__ __forceinline__ int64_t packed_scale_index(int64_t r, int b, int K) {
-  return (((r >> 8) * (K >> 7) + (b >> 2)) * 256 + (r & 255)) * 4 + (b & 3);
-}
-
-// Two lanes per (row, 32-block), sixteen elements each, so every hi / lo store
-// is one 16-byte slot.  PACKED: scales in the tile-major layout above and hi /
-// lo pre-tiled the way the pipelined GEMM's LDS holds them: for each 256-row
-// tile and 64-wide K step, one contiguous 16 KiB block of 1024 slots of 16
-// bytes, slot 4 r + (p ^ p_swz(r)) holding bytes [16 p, 16 p + 16) of row r's
-// step.  Otherwise row-major [rows, K] and [rows, K / 32].  One thread per
-// (row, half block): rows * K / 16 < 2^31 (checked by the host).
-//
-// hi = RNE_E4M3(x / 2^sh), lo = RNE_E4M3((x - hi * 2^sh) / 2^sl) with the block
-// scales sh, sl from ceil_scale_exp, so no element is clamped.  The rounding is
-// v_cvt_pk_fp8_f32 (OCP E4M3, nearest-even; measured identical to a software
-// nearest-even on every input this pass produces); x - hi * 2^sh is exact in f32.
 // The split of 16 consecutive elements (lane pair l, l ^ 1 shares a 32-block): E4M3
 // hi / lo words and the block's exponents th, tl.
 __device__ __forceinline__ void split16(const uint4 q0, const uint4 q1, uint32_t (&hw)[4], uint32_t (&lw)[4], int &th,
@@ -97,530 +89,387 @@ __device__ __forceinline__ void split16(const uint4 q0, const uint4 q1, uint32_t
   }
 }
 
-// Row-major form: one thread per (row, 16 elements).
-__global__ __launch_bounds__(256) void split_x_kernel(const uint16_t *__restrict__ x, uint32_t total, int rows, int K,
-                                                      uint8_t *__restrict__ xh, uint8_t *__restrict__ xl,
-                                                      uint8_t *__restrict__ sh, uint8_t *__restrict__ sl) {
-  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-  // lanes past the end (the grid is whole blocks) compute on a clamped index and
-  // store nothing; total is even, so the two lanes of a block are both live or not
-  const bool live = i < total;
-  const uint32_t ii = live ? i : total - 1;
-  const uint32_t L = (uint32_t)K >> 4;  // threads per row
-  const uint32_t r = ii / L, c = ii - r * L;
-  const int b = (int)(c >> 1), j = (int)(c & 1);
-  const uint4 *src = (const uint4 *)(x + (int64_t)r * K + 16 * c);
-  uint32_t hw[4], lw[4];
-  int th, tl;
-  split16(src[0], src[1], hw, lw, th, tl);
-  if (!live) return;
-  const int64_t o = (int64_t)r * K + 16 * c;
-  *(uint4 *)(xh + o) = make_uint4(hw[0], hw[1], hw[2], hw[3]);
-  *(uint4 *)(xl + o) = make_uint4(lw[0], lw[1], lw[2], lw[3]);
-  if (j == 0) {
-    sh[(int64_t)r * (K >> 5) + b] = (uint8_t)(th + 127);
-    sl[(int64_t)r * (K >> 5) + b] = (uint8_t)(tl + 127);
-  }
-}
-
-// Pre-tiled form for the pipelined GEMM: a wave takes 16 rows x U consecutive 64-wide K
-// steps; in each step lane l takes row l / 4, 16 elements l % 4 of the step, so a row's
-// 64 output bytes (one slot row of the step's block) come from 4 adjacent lanes and the
-// wave writes 1 KiB of consecutive slots.  All U steps' reads (16 whole 128-byte row
-// pieces each) are issued before the first is split, so a wave has U x 2 KiB in flight.
-// total = waves x 64 threads, waves = rows16 / 16 x S / U with S = K / 64 (S % U == 0);
-// rows past `rows` (up to the 16-row group) read the last row and store nothing.
+// x [rows, K] -> xs: per row and step 128 bytes, the step's 64 hi then its 64 lo bytes (zeros
+// past K), rows of steps x 128 bytes; and the block scales, a dword per row and step (hi and
+// lo of the step's first 32-block, then of its second), tile-major: for each 256 rows and pair
+// of steps, 2 x 256 consecutive dwords.  A wave takes 16 rows x U steps; in each step lane l
+// takes row l / 4, 16 elements l % 4 of the step.  All reads are issued before the first is
+// split.  Rows past `rows` (up to the 16-row group) read the last row and store nothing.
 template <int U>
-__global__ __launch_bounds__(256) void split_x_packed_kernel(const uint16_t *__restrict__ x, uint32_t total, int rows,
-                                                             int K, uint8_t *__restrict__ xh, uint8_t *__restrict__ xl,
-                                                             uint8_t *__restrict__ sh, uint8_t *__restrict__ sl) {
-  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-  const bool live = i < total;  // whole waves: a wave is all live or all not
-  const uint32_t ii = live ? i : total - 1;
-  const uint32_t SU = ((uint32_t)K >> 6) / U, w = ii >> 6, l = ii & 63;
-  const uint32_t rg = w / SU, st0 = U * (w - rg * SU);
-  const uint32_t r = 16 * rg + (l >> 2);
-  const uint32_t rl = (int)r < rows ? r : (uint32_t)rows - 1;
+__global__ __launch_bounds__(256) void split_x_kernel(const uint16_t *__restrict__ x, int rows, int K, int steps,
+                                                      uint8_t *__restrict__ xs, uint32_t *__restrict__ sx) {
+  const int lane = threadIdx.x & 63;
+  const int su = (steps + U - 1) / U, w = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int rg = w / su, st0 = U * (w - rg * su);
+  if (16 * rg >= rows) return;  // (the grid is whole blocks; a wave leaves as one)
+  const int r = 16 * rg + (lane >> 2), c = lane & 3;
+  const uint16_t *src = x + (int64_t)min(r, rows - 1) * K + 16 * c;
   uint4 q[U][2];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    const uint4 *src = (const uint4 *)(x + (int64_t)rl * K + 16 * (4 * (st0 + u) + (l & 3)));
-    q[u][0] = src[0];
-    q[u][1] = src[1];
+    q[u][0] = q[u][1] = make_uint4(0, 0, 0, 0);
+    if (X_BK * (st0 + u) + 16 * c < K) {
+      q[u][0] = *(const uint4 *)(src + X_BK * (st0 + u));
+      q[u][1] = *(const uint4 *)(src + X_BK * (st0 + u) + 8);
+    }
   }
-  const int rr = (int)(r & 255);
-  const int64_t tile = (int64_t)(r >> 8) * (K >> 6);
-  const bool store = live && (int)r < rows;
-  // Scale bytes: step st0 + u of row r holds blocks 2 (st0 + u) + {0, 1} (lanes l % 4 in
-  // {0, 1}, {2, 3}); st0 is even, so steps u = 2P, 2P + 1 fill the four bytes of the row's
-  // tile-major dword st0 / 2 + P in block order.  Each lane packs the bytes of its own
-  // blocks and takes the other block's from lane l ^ 2; then lane l % 4 = 2 t + P stores
-  // whole dword P of hi (t = 0) or lo (t = 1) scales.
-  constexpr int PW = U / 2;
-  uint32_t ph[PW], pl[PW];
-#pragma unroll
-  for (int p = 0; p < PW; ++p) ph[p] = pl[p] = 0u;
-  const int hb = (int)((l >> 1) & 1);  // the lane's block within the step
+  const int pairs = (steps + 1) / 2;
 #pragma unroll
   for (int u = 0; u < U; ++u) {
+    const int st = st0 + u;
+    if (st >= steps) break;
     uint32_t hw[4], lw[4];
     int th, tl;
     split16(q[u][0], q[u][1], hw, lw, th, tl);
-    const uint32_t c = 4 * (st0 + u) + (l & 3);
-    const int b = (int)(c >> 1), j = (int)(c & 1);
-    const int sft = 8 * (2 * (u & 1) + hb);
-    ph[u >> 1] |= (uint32_t)(th + 127) << sft;
-    pl[u >> 1] |= (uint32_t)(tl + 127) << sft;
-    if (store) {
-      const int64_t o = (tile + (b >> 1)) * 16384 + 16 * (4 * rr + ((2 * (b & 1) + j) ^ p_swz(rr)));
-      *(uint4 *)(xh + o) = make_uint4(hw[0], hw[1], hw[2], hw[3]);
-      *(uint4 *)(xl + o) = make_uint4(lw[0], lw[1], lw[2], lw[3]);
+    uint32_t sc = (uint32_t)(th + 127) | (uint32_t)(tl + 127) << 8;
+    sc |= (uint32_t)__shfl_xor((int)sc, 2) << 16;  // lanes 0 of 4: the step's two blocks
+    if (r < rows) {
+      uint8_t *o = xs + ((int64_t)r * steps + st) * 128 + 16 * c;
+      *(uint4 *)o = make_uint4(hw[0], hw[1], hw[2], hw[3]);
+      *(uint4 *)(o + 64) = make_uint4(lw[0], lw[1], lw[2], lw[3]);
+      if (c == 0) sx[(((int64_t)(r >> 8) * pairs + (st >> 1)) * 2 + (st & 1)) * 256 + (r & 255)] = sc;
     }
-  }
-#pragma unroll
-  for (int p = 0; p < PW; ++p) {
-    ph[p] |= (uint32_t)__shfl_xor((int)ph[p], 2);
-    pl[p] |= (uint32_t)__shfl_xor((int)pl[p], 2);
-  }
-  const int t = (int)((l >> 1) & 1), p = (int)(l & 1);
-  if (store && p < PW) {
-    const uint32_t v = PW == 1 ? (t ? pl[0] : ph[0]) : (t ? (p ? pl[PW - 1] : pl[0]) : (p ? ph[PW - 1] : ph[0]));
-    uint8_t *dst = t ? sl : sh;
-    *(uint32_t *)(dst + packed_scale_index(r, 2 * (st0 + 2 * p), K)) = v;
   }
 }
 
 // ---------------------------------------------------------------- GEMM
 
 namespace {
-constexpr int F_BM = 256, F_BN = 256, F_BK = 64, F_PITCH = 80;  // bytes per LDS row (64 + 16 pad)
-constexpr int F_TILE = 256 * F_PITCH;                            // one operand tile
-constexpr int F_THREADS = 512;                                   // 8 waves: 4 (M) x 2 (N)
-}  // namespace
-
-struct Fp8Smem {
-  uint8_t a_hi[2][F_TILE];
-  uint8_t a_lo[2][F_TILE];
-  uint8_t b[2][F_TILE];
-  uint8_t s_hi[2][256 * 2];
-  uint8_t s_lo[2][256 * 2];
-  uint8_t s_b[2][256 * 2];
-};
-
-__global__ __launch_bounds__(F_THREADS) void gemm_mxfp8_kernel(
-    const uint8_t *__restrict__ xh, const uint8_t *__restrict__ xl, const uint8_t *__restrict__ sh,
-    const uint8_t *__restrict__ sl, const uint8_t *__restrict__ w, const uint8_t *__restrict__ sw,
-    uint16_t *__restrict__ y, int M, int N, int K) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem_raw[];
-  Fp8Smem &sm = *reinterpret_cast<Fp8Smem *>(smem_raw);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;  // wave tile: rows wm*64 + [0,64), cols wn*128 + [0,128)
-  int tm, tn;
-  tile_of(blockIdx.x, (M + F_BM - 1) / F_BM, (N + F_BN - 1) / F_BN, &tm, &tn);
-  const int m0 = tm * F_BM, n0 = tn * F_BN;
-  const int nb = K >> 5;  // scale bytes per row
-  const int steps = K / F_BK;
-
-  // loader: 16-byte chunk c = tid + 512*j (j < 2) of each 256 x 64 tile: row c>>2, part c&3
-  uint4 ra_h[2], ra_l[2], rb[2];
-  uint16_t rs0, rs1;  // tid < 256: x-hi scales (rs0) and W scales (rs1) of row tid; else x-lo scales of row tid-256
-  const int srow = tid & 255;
-  const int64_t sm_row = min(m0 + srow, M - 1), sn_row = min(n0 + srow, N - 1);
-  const uint8_t *s_src0 = (tid < 256 ? sh : sl) + sm_row * nb;
-  const uint8_t *s_src1 = sw + sn_row * nb;
-
-  auto gload = [&](int step) {
-    const int k0 = step * F_BK;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int c = tid + F_THREADS * j, row = c >> 2, part = c & 3;
-      const int64_t mr = min(m0 + row, M - 1), nr = min(n0 + row, N - 1);
-      ra_h[j] = *(const uint4 *)(xh + mr * K + k0 + part * 16);
-      ra_l[j] = *(const uint4 *)(xl + mr * K + k0 + part * 16);
-      rb[j] = load_stream16(w + nr * K + k0 + part * 16);
-    }
-    rs0 = *(const uint16_t *)(s_src0 + (k0 >> 5));
-    if (tid < 256) rs1 = *(const uint16_t *)(s_src1 + (k0 >> 5));
-  };
-  auto sstore = [&](int buf) {
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int c = tid + F_THREADS * j, row = c >> 2, part = c & 3;
-      *(uint4 *)(sm.a_hi[buf] + row * F_PITCH + part * 16) = ra_h[j];
-      *(uint4 *)(sm.a_lo[buf] + row * F_PITCH + part * 16) = ra_l[j];
-      *(uint4 *)(sm.b[buf] + row * F_PITCH + part * 16) = rb[j];
-    }
-    if (tid < 256) {
-      *(uint16_t *)(sm.s_hi[buf] + srow * 2) = rs0;
-      *(uint16_t *)(sm.s_b[buf] + srow * 2) = rs1;
-    } else {
-      *(uint16_t *)(sm.s_lo[buf] + srow * 2) = rs0;
-    }
-  };
-
-  f32x16_t acc[2][4];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-
-  gload(0);
-  sstore(0);
-  __syncthreads();
-  // Operand layout of v_mfma_scale_f32_32x32x64_f8f6f4 (measured on gfx950): lane l
-  // holds row l%32; its bytes 0-15 are K 16*(l/32)+[0,16) of block 0 and bytes 16-31
-  // the same span of block 1 (K+32).  Its scale byte covers block l/32 of row l%32.
-  const int fr = lane & 31, fh = lane >> 5, fk = fh * 16;
-  for (int s = 0; s < steps; ++s) {
-    const int buf = s & 1;
-    if (s + 1 < steps) gload(s + 1);
-    i32x8_t ah[2], al[2];
-    int shv[2], slv[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int row = wm * 64 + i * 32 + fr;
-      const uint8_t *ph = sm.a_hi[buf] + row * F_PITCH + fk;
-      const uint8_t *pl = sm.a_lo[buf] + row * F_PITCH + fk;
-      const uint4 h0 = *(const uint4 *)ph, h1 = *(const uint4 *)(ph + 32);
-      const uint4 l0 = *(const uint4 *)pl, l1 = *(const uint4 *)(pl + 32);
-      ah[i] = i32x8_t{(int)h0.x, (int)h0.y, (int)h0.z, (int)h0.w, (int)h1.x, (int)h1.y, (int)h1.z, (int)h1.w};
-      al[i] = i32x8_t{(int)l0.x, (int)l0.y, (int)l0.z, (int)l0.w, (int)l1.x, (int)l1.y, (int)l1.z, (int)l1.w};
-      shv[i] = sm.s_hi[buf][row * 2 + fh];
-      slv[i] = sm.s_lo[buf][row * 2 + fh];
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int row = wn * 128 + j * 32 + fr;
-      const uint8_t *p = sm.b[buf] + row * F_PITCH + fk;
-      const uint4 u0 = *(const uint4 *)p, u1 = *(const uint4 *)(p + 32);
-      const i32x8_t bfr = i32x8_t{(int)u0.x, (int)u0.y, (int)u0.z, (int)u0.w, (int)u1.x, (int)u1.y, (int)u1.z, (int)u1.w};
-      const int bsc = sm.s_b[buf][row * 2 + fh];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(ah[i], bfr, acc[i][j], 0, 0, 0, shv[i], 0, bsc);
-        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(al[i], bfr, acc[i][j], 0, 0, 0, slv[i], 0, bsc);
-      }
-    }
-    if (s + 1 < steps) sstore(buf ^ 1);
-    __syncthreads();
+// A block's tile: WM x WN waves of (32 FI) x (32 FJ); LDS rings of SX stages of x (a step
+// each) and SW stages of W and of the scales (two steps each: 128 bytes of a W row, the dword
+// of its four block scales and an x row's two).
+template <int FI_, int FJ_, int WM_, int WN_, int SX_, int SW_>
+struct MxGeom {
+  static constexpr int FI = FI_, FJ = FJ_, WM = WM_, WN = WN_, SX = SX_, SW = SW_;
+  static constexpr int TM = 32 * FI * WM, TN = 32 * FJ * WN, NW = WM * WN, THREADS = 64 * NW;
+  static constexpr int XT = TM * 128, WT = TN * 128;
+  static constexpr int SD = (TN + 2 * TM + 255) / 256;  // scale DMAs of a stage
+  static constexpr int WOFF = SX * XT, SOFF = WOFF + SW * WT, ST = SD * 1024;
+  static constexpr int LDS = SOFF + SW * ST;
+  static constexpr int NX = TM / 8 / NW;       // x DMAs per wave per step
+  static constexpr int NWD = TN / 8 / NW + 1;  // W DMAs and one of the scales' per wave per stage
+  static_assert(TM / 8 % NW == 0 && TN / 8 % NW == 0 && TN % 4 == 0 && NW % 2 == 0 && SD <= NW, "");
+  static_assert(SX >= 2 && SW >= 2 && SX <= 2 * SW - 1, "");
+  static constexpr int REGION = 32 * (64 * FJ + 32);
+  static_assert(NW * REGION <= LDS, "the epilogue regions fit the rings");
+  // DMAs that may be in flight at the barrier of an even (odd) step s: x of step i + SX is
+  // issued in step i, and W stage (i - 1) / 2 + SW after it when i is odd; x of step s + 1
+  // has to be there and, at an odd step, the next W stage.
+  static constexpr int issued(int from, int to) {  // in steps from .. to - 1
+    int n = 0;
+    for (int i = from; i < to; ++i) n += NX + (i & 1 ? NWD : 0);
+    return n;
   }
-
-  // epilogue: 32x32 accumulator element v of lane l is row 8*(v/4) + 4*(l/32) + v%4, col l%32
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int col = n0 + wn * 128 + j * 32 + (lane & 31);
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int row = m0 + wm * 64 + i * 32 + (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3);
-        if (row < M && col < N) y[(int64_t)row * N + col] = f32_to_bf16_rne(acc[i][j][v]);
-      }
-    }
-}
-
-// ---------------------------------------------------------------- pipelined GEMM (K % 128 == 0)
-//
-// Same MFMA and wave layout as above (8 waves, 4 along x rows x 2 along W rows),
-// in two tile sizes: TS = 256 (waves of 64 x 128) for the bulk and TS = 128
-// (waves of 32 x 64) for a last partial round of the chip, split four ways so
-// that it takes a quarter of a round.  The operand traffic is off the VGPRs:
-//   * every operand byte goes global -> LDS directly (global_load_lds: lane i
-//     of a wave writes bytes [16 i, 16 i + 16) of the wave's 1 KiB destination,
-//     [4 i, 4 i + 4) for the dword form), into a 3-stage ring: the loads of step
-//     s + 2 are issued while step s computes;
-//   * the DMA is issued from inline assembly and waited for explicitly
-//     (s_waitcnt vmcnt), so no compiler-inserted wait serialises the ring;
-//   * an operand tile is TS rows x 64 bytes, unpadded; 16-byte slot p of row r is
-//     stored at slot p ^ p_swz(r), so the fragment reads of 8 (or 16) consecutive
-//     rows at one slot hit distinct banks; x hi / lo come pre-tiled in exactly
-//     this order (a 128-row tile is one half of a 256-row block), W row-major;
-//   * scales: per stage, the dword holding each row's 4 E8M0 bytes of the step
-//     pair (the step uses 2 of them) for x hi, x lo and W, from the tile-major
-//     copies;
-//   * each wave issues exactly TS / 32 DMAs per step (3 TS / 128 tile, TS / 128
-//     scale), the count the waits are written for.
-namespace {
-constexpr int P_BK = 64, P_STAGES = 3;
-template <int TS>
-struct PipeGeom {
-  static constexpr int TILE = TS * P_BK;                  // one operand tile (bytes)
-  static constexpr int SCALES = 4 * TS * 4;               // x hi, x lo, W scale dwords + a spare block
-  static constexpr int STAGE = 3 * TILE + SCALES;         // 52 KiB at 256, 26 KiB at 128
-  static constexpr size_t LDS = (size_t)P_STAGES * STAGE;
-  static constexpr int TI = TS / 128;                     // tile DMAs per wave per operand
-  static constexpr int IPT = TS / 64;                     // scale DMAs per scale tensor
-  static constexpr int NDMA = 4 * TI;                     // DMAs per wave per step
-  static constexpr int FI = TS / 128, FJ = TS / 64;       // accumulators per wave
+  static constexpr int in_flight(int s) {
+    const int i0 = s + 1 - SX, nx = (i0 & 1 ? NWD : 0) + issued(i0 + 1, s);
+    const int nw = issued(s + 2 - 2 * SW + 1, s);
+    return (s & 1) && nw < nx ? nw : nx;
+  }
 };
 }  // namespace
 
-__device__ __forceinline__ i32x8_t p_frag(const uint8_t *base, int off) {
-  const uint4 u0 = *(const uint4 *)(base + off), u1 = *(const uint4 *)(base + (off ^ 32));
-  return i32x8_t{(int)u0.x, (int)u0.y, (int)u0.z, (int)u0.w, (int)u1.x, (int)u1.y, (int)u1.z, (int)u1.w};
-}
+// Zeros that stand for the pieces of the last stage past K.
+__device__ const uint4 mx_zero = {0, 0, 0, 0};
 
-// Tile `bid` of the TS x TS tiling of x rows [0, M) and W rows [n_begin, n_end), over the
-// K steps [s_begin, s_end).  With `part` null the tile's bf16 result goes to y; otherwise
-// (a K range of a split tile) the fp32 accumulators go to `part` as they sit in the
-// registers: wave w, accumulator (i, j), elements 4 v4 .. 4 v4 + 3 of lane l as the float4
-// at ((w * FI * FJ + i * FJ + j) * 4 + v4) * 64 + l.
-template <int TS>
-__device__ __forceinline__ void pipe_tile(int bid, const uint8_t *__restrict__ xh, const uint8_t *__restrict__ xl,
-                                          const uint8_t *__restrict__ sh, const uint8_t *__restrict__ sl,
-                                          const uint8_t *__restrict__ w, const uint8_t *__restrict__ sw,
-                                          const YOut yo, int M, int N, int K, int n_begin, int n_end,
-                                          int s_begin, int s_end, float *__restrict__ part) {
-  using G = PipeGeom<TS>;
+// 16-byte piece p of a row's 128 bytes is stored at slot p ^ mx_swz(row).
+__device__ __forceinline__ int mx_swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
+
+// MLP: the tile's W rows are two matrices', 32-row blocks of gate and of up in turn (row
+// block 2 b and 2 b + 1 of a tile are rows 32 b + [0, 32) of the tile's TN / 2), and the
+// result is silu(gate) * up, TN / 2 columns of it per tile.
+template <class G, bool MLP>
+__global__ __launch_bounds__(G::THREADS, G::LDS <= 81920 ? 2 * G::NW / 4 : G::NW / 4) void gemm_mxfp8_kernel(
+    const uint8_t *__restrict__ xs, const uint32_t *__restrict__ sx, const uint8_t *__restrict__ w,
+    const uint8_t *__restrict__ sp, const uint8_t *__restrict__ w_up, const uint8_t *__restrict__ sp_up, const YOut yo,
+    int M, int N, int K, int whole_tiles, int S, float *__restrict__ part) {
+  constexpr int FI = G::FI, FJ = G::FJ, NX = G::NX, NWD = G::NWD, SX = G::SX, SW = G::SW;
+  constexpr int TC = MLP ? G::TN / 2 : G::TN;  // columns of y per tile
+  static_assert(!MLP || FJ % 2 == 0, "a wave holds gate and up of a column");
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const uint32_t lds0 = lds_addr(lds);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 1, wn = wave & 1;  // wave tile: rows wm * TS / 4 + [0, TS / 4), cols wn * TS / 2 + [0, TS / 2)
-  int tm, tn;
-  tile_of(bid, (M + TS - 1) / TS, (n_end - n_begin + TS - 1) / TS, &tm, &tn);
-  const int m0 = tm * TS, n0 = n_begin + tn * TS;
-  const int steps = K / P_BK;
+  const int wm = wave % G::WM, wn = wave / G::WM;
+  const int tiles_m = (M + G::TM - 1) / G::TM, tiles_n = (N + TC - 1) / TC;
+  const int steps = (K + X_BK - 1) / X_BK, stages = (steps + 1) / 2;
+  const GpBlock blk = gp_block(blockIdx.x, tiles_m, tiles_n, whole_tiles, S);
+  const int m0 = blk.tm * G::TM, n0 = blk.tn * TC;
+  const int g_begin = blk.split ? (int)((int64_t)blk.kr * stages / S) : 0;
+  const int g_end = blk.split ? (int)((int64_t)(blk.kr + 1) * stages / S) : stages;
+  const int s_begin = g_begin * 2, s_end = min(g_end * 2, steps);
 
-  // tile DMA: wave-instruction t (< TI) of this wave fills LDS slots q = (8 t + wave) * 64 + lane
-  // (x hi / lo pre-tiled: a 256-row block's step is 1024 contiguous slots, rows m0 % 256 on;
-  // W row-major: slot q holds row q >> 2, 16-byte part (q & 3) ^ swz(row)).  An x instruction
-  // covers tile rows 16 (8 t + wave) + [0, 16); when all 16 are past the last x row (a short
-  // x) it moves 4 bytes per lane instead of 16: the same instruction count (the waits count
-  // them), a quarter of the bytes, and those rows' results are not stored.
-  const uint8_t *ga_h[G::TI], *ga_l[G::TI], *gb[G::TI];
-  bool xdead[G::TI];
+  // A DMA fills 1 KiB: rows 8 q + [0, 8) of a stage of x (or W), q = wave + NW i; lane l the
+  // 16-byte slot l % 8 of row l / 8, which holds piece (l % 8) ^ swz(row) of the row's 128 bytes.
+  const int64_t xrow = (int64_t)steps * 128;
+  const uint8_t *xb = xs + (int64_t)m0 * xrow;
+  const int dr = 8 * wave + (lane >> 3), dp = (lane & 7) ^ mx_swz(dr);  // rows 8 NW apart share a swizzle
+  uint32_t xo[NX], wo[NWD - 1];
+  const uint8_t *wb[MLP ? NWD - 1 : 1];
 #pragma unroll
-  for (int t = 0; t < G::TI; ++t) {
-    const int q = (8 * t + wave) * 64 + lane, row = q >> 2, part = (q & 3) ^ p_swz(row);
-    const int64_t xo = (int64_t)(m0 >> 8) * steps * 16384 + ((m0 & 255) * 4 + q) * 16;
-    ga_h[t] = xh + xo;
-    ga_l[t] = xl + xo;
-    gb[t] = w + (int64_t)min(n0 + row, N - 1) * K + part * 16;
-    xdead[t] = m0 + 16 * (8 * t + wave) >= M;
-  }
-  // scale DMA: wave-instruction t = TI wave + h (h < TI) copies rows (t % IPT) * 64 + lane
-  // of tensor t / IPT (x hi, x lo, W, all tile-major; the 4th re-reads x hi into the spare block)
-  const uint8_t *gs[G::TI];
-  const int pairs = K >> 7;
+  for (int i = 0; i < NX; ++i) xo[i] = (uint32_t)((min(m0 + dr + 8 * G::NW * i, M - 1) - m0) * xrow) + dp * 16;
+  if constexpr (!MLP) wb[0] = w + (int64_t)n0 * K;
 #pragma unroll
-  for (int h = 0; h < G::TI; ++h) {
-    const int t = G::TI * wave + h, tensor = t / G::IPT, row = (t % G::IPT) * 64 + lane;
-    const uint8_t *src = tensor == 1 ? sl : tensor == 2 ? sw : sh;
-    const int base = tensor == 2 ? n0 : m0;
-    gs[h] = src + ((int64_t)(base >> 8) * pairs * 256 + (base & 255) + row) * 4;
-  }
-  auto issue = [&](int s) __attribute__((always_inline)) {
-    const uint32_t st = lds0 + (uint32_t)((s % P_STAGES) * G::STAGE);
-    const int k0 = s * P_BK;
-    const int64_t xs = (int64_t)s * 16384;
-#pragma unroll
-    for (int t = 0; t < G::TI; ++t) {
-      if (xdead[t]) {
-        gp_dma4(ga_h[t] + xs, st + (8 * t + wave) * 1024);
-        gp_dma4(ga_l[t] + xs, st + G::TILE + (8 * t + wave) * 1024);
-      } else {
-        gp_dma16(ga_h[t] + xs, st + (8 * t + wave) * 1024);
-        gp_dma16(ga_l[t] + xs, st + G::TILE + (8 * t + wave) * 1024);
-      }
-      gp_dma16(gb[t] + k0, st + 2 * G::TILE + (8 * t + wave) * 1024);
+  for (int i = 0; i < NWD - 1; ++i) {
+    const int q = wave + G::NW * i, r = dr + 8 * G::NW * i;  // 8 rows of one 32-row block
+    int row = r;
+    if constexpr (MLP) {
+      wb[i] = ((q >> 2) & 1 ? w_up : w) + (int64_t)n0 * K;
+      row = (r >> 6) * 32 + (r & 31);
     }
-    const int so = 1024 * (s >> 1);  // the step pair's block
+    wo[i] = (uint32_t)(min(n0 + row, N - 1) - n0) * (uint32_t)K + dp * 16;
+  }
+  // scales: dword d of a stage's ring slot is W row d's (d < TN), then x row r's of step t at
+  // TN + t TM + r; a DMA moves four dwords per lane, 256 in all, wave v the v % SD-th (lanes past
+  // the last dword repeat it)
+  const int n256 = (N + 255) & ~255, m256 = (M + 255) & ~255;
+  const int sq = min((wave % G::SD) * 256 + 4 * lane, G::TN + 2 * G::TM - 4);
+  const uint8_t *sb;
+  uint32_t sstep;  // bytes from a stage's to the next's
+  if (sq < G::TN) {
+    const int mat = MLP ? (sq >> 5) & 1 : 0, row = min(n0 + (MLP ? (sq >> 6) * 32 + (sq & 31) : sq), n256 - 4);
+    sb = (mat ? sp_up : sp) + ((int64_t)(row >> 8) * stages * 256 + (row & 255)) * 4;
+    sstep = 1024;
+  } else {
+    const int t = (sq - G::TN) / G::TM, row = min(m0 + (sq - G::TN) % G::TM, m256 - 4);
+    sb = (const uint8_t *)sx + (((int64_t)(row >> 8) * stages * 2 + t) * 256 + (row & 255)) * 4;
+    sstep = 2048;
+  }
+
+  auto issue_x = [&](int i, int s) __attribute__((always_inline)) {
+    gp_dma16s(xb + (int64_t)s * 128, xo[i], lds0 + (uint32_t)((s % SX) * G::XT + (wave + G::NW * i) * 1024));
+  };
+  auto w_slot = [&](int i, int g) __attribute__((always_inline)) {
+    return lds0 + (uint32_t)(G::WOFF + (g % SW) * G::WT + (wave + G::NW * i) * 1024);
+  };
+  auto issue_w = [&](int i, int g) __attribute__((always_inline)) {  // the last one: the scales
+    if (i < NWD - 1) gp_dma16s(wb[MLP ? i : 0] + (int64_t)g * 128, wo[i], w_slot(i, g));
+    else gp_dma16(sb + (int64_t)g * sstep, lds0 + (uint32_t)(G::SOFF + (g % SW) * G::ST + (wave % G::SD) * 1024));
+  };
+  // stage g's W, whole or the rows' last, whose pieces past K are zeros
+  auto issue_w_any = [&](int g) __attribute__((always_inline)) {
 #pragma unroll
-    for (int h = 0; h < G::TI; ++h) gp_dma4(gs[h] + so, st + 3 * G::TILE + (G::TI * wave + h) * 256);
+    for (int i = 0; i < NWD; ++i) {
+      if ((g + 1) * 2 * X_BK <= K || i == NWD - 1) {
+        issue_w(i, g);
+      } else {
+        const uint8_t *p = wb[MLP ? i : 0] + wo[i] + (int64_t)g * 128;
+        if (g * 2 * X_BK + 16 * dp >= K) p = (const uint8_t *)&mx_zero;
+        gp_dma16(p, w_slot(i, g));
+      }
+    }
   };
 
-  // fragment geometry (32x32x64 operand layout: lane l holds row l % 32, K bytes 16 (l / 32) + [0, 16) and +32)
+  // Fragments (32x32x64 operands: lane l holds row l % 32, K bytes 16 fh + [0, 16) and 32 + 16 fh
+  // + [0, 16), fh = l / 32, and the scale of block fh): x hi pieces fh and fh + 2 of the row's 128
+  // bytes, lo fh + 4 and fh + 6; W, step t of its stage, 4 t + fh and 4 t + fh + 2.
   const int fr = lane & 31, fh = lane >> 5;
-  int oa[G::FI], ob[G::FJ], osa[G::FI], osb[G::FJ];
-#pragma unroll
-  for (int i = 0; i < G::FI; ++i) {
-    const int r = wm * (TS / 4) + i * 32 + fr;
-    oa[i] = r * P_BK + 16 * (fh ^ p_swz(r));
-    osa[i] = 3 * G::TILE + r * 4 + fh;
-  }
-#pragma unroll
-  for (int j = 0; j < G::FJ; ++j) {
-    const int r = wn * (TS / 2) + j * 32 + fr;
-    ob[j] = r * P_BK + 16 * (fh ^ p_swz(r));
-    osb[j] = 3 * G::TILE + 2 * TS * 4 + r * 4 + fh;
-  }
+  const int ra = wm * 32 * FI + fr, rb = wn * 32 * FJ + fr;
+  const int oa = ra * 128 + 16 * (fh ^ mx_swz(ra));
+  const int ob = G::WOFF + rb * 128 + 16 * (fh ^ mx_swz(rb));
+  const int osw = G::SOFF + rb * 4 + fh, osx = G::SOFF + (G::TN + ra) * 4 + 2 * fh;
 
-  f32x16_t acc[G::FI][G::FJ];
+  f32x16_t acc[FI][FJ];
 #pragma unroll
-  for (int i = 0; i < G::FI; ++i)
+  for (int i = 0; i < FI; ++i)
 #pragma unroll
-    for (int j = 0; j < G::FJ; ++j)
+    for (int j = 0; j < FJ; ++j)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
 
-  // Ping-pong: waves 0-3 (group 0) and 4-7 (group 1) put one wave of each group on
-  // every SIMD.  Barrier intervals alternate: in each, one group runs the MFMAs
-  // of its step while the other issues its DMAs and reads its next fragments, so
-  // the MFMA pipe of every SIMD always has a wave feeding it.  Group 0 computes
-  // step k in interval 2k + 1, group 1 in 2k + 2.  DMA(k + 2) overwrites the
-  // stage group 1 read in interval 2k - 1, and is issued in the loading interval
-  // of step k (2k, 2k + 1); at the barrier that ends interval 2k + 1 every wave
-  // waits for its DMA(k + 1) (only DMA(k + 2), NDMA loads, may remain), so stage
-  // k + 1 is whole before group 0 reads it in interval 2k + 2.
-  const int grp = wave >> 2;
-  issue(s_begin);
-  if (s_end - s_begin > 1) issue(s_begin + 1);
-  if (s_end - s_begin > 1) gp_wait_barrier<G::NDMA>();
+  i32x8_t ah[FI], al[FI], bf[2][FJ];  // W in set s % 2
+  // block scales (x: hi in byte 0, lo in byte 1), also in set s % 2: the MFMA reads its scale
+  // registers after issue, so none is written by the instructions that follow it
+  int sa[2][FI], sbw[2][FJ];
+  auto frag = [&](const uint8_t *p, int o) __attribute__((always_inline)) {
+    const uint4 u0 = *(const uint4 *)(p + o), u1 = *(const uint4 *)(p + (o ^ 32));
+    return i32x8_t{(int)u0.x, (int)u0.y, (int)u0.z, (int)u0.w, (int)u1.x, (int)u1.y, (int)u1.z, (int)u1.w};
+  };
+  auto read_hi = [&](auto t_c, int s, int i) __attribute__((always_inline)) {
+    constexpr int T = decltype(t_c)::value;  // s % 2
+    ah[i] = frag(lds + (s % SX) * G::XT + 4096 * i, oa);
+    sa[T][i] = *(const uint16_t *)(lds + ((s >> 1) % SW) * G::ST + osx + T * (4 * G::TM) + 128 * i);
+  };
+  auto read_lo = [&](int s, int i) __attribute__((always_inline)) {
+    al[i] = frag(lds + (s % SX) * G::XT + 4096 * i, oa ^ 64);
+  };
+  auto read_w = [&](auto t_c, int s, int j) __attribute__((always_inline)) {
+    constexpr int T = decltype(t_c)::value;
+    bf[T][j] = frag(lds + ((s >> 1) % SW) * G::WT + 4096 * j, ob ^ (64 * T));
+    sbw[T][j] = *(lds + ((s >> 1) % SW) * G::ST + osw + 2 * T + 128 * j);
+  };
+  constexpr int NM = FI * FJ;
+  using I0 = std::integral_constant<int, 0>;
+  using I1 = std::integral_constant<int, 1>;
+  using I2 = std::integral_constant<int, 2>;
+  using I3 = std::integral_constant<int, 3>;
+
+  // The DMAs' order: step i brings x of step i + SX and, when odd, then W stage (i - 1) / 2 + SW
+  // (relative to the range's first step); here the steps before the first.
+#pragma unroll 1
+  for (int i = 1 - 2 * SW; i < 0; ++i) {
+    if (i + SX >= 0 && s_begin + i + SX < s_end) {
+#pragma unroll
+      for (int q = 0; q < NX; ++q) issue_x(q, s_begin + i + SX);
+    }
+    if ((i & 1) && g_begin + (i - 1) / 2 + SW < g_end) issue_w_any(g_begin + (i - 1) / 2 + SW);
+  }
+  if (g_end - g_begin >= SW && s_end - s_begin >= SX) gp_wait_barrier<G::in_flight(1)>();
   else gp_wait_barrier<0>();
+#pragma unroll
+  for (int j = 0; j < FJ; ++j) read_w(I0{}, s_begin, j);
+#pragma unroll
+  for (int i = 0; i < FI; ++i) read_hi(I0{}, s_begin, i);
 
-  // one step of a group: loading interval (DMAs of step s + 2 if DMA, fragments of
-  // step s), barrier, computing interval, barrier.  Each call is one basic block, so
-  // the scheduling barriers keep the MFMAs inside their interval.
-  auto pp_step = [&](auto grp_c, auto dma_c, int s) __attribute__((always_inline)) {
-    constexpr int GRP = decltype(grp_c)::value;
-    constexpr bool DMA = decltype(dma_c)::value;
-    if constexpr (DMA) issue(s + 2);
-    const uint8_t *st = lds + (s % P_STAGES) * G::STAGE;
-    const int sb = 2 * (s & 1);  // byte of the pair dword: block fh of this step
-    i32x8_t ah[G::FI], al[G::FI], bf[G::FJ];
-    int shv[G::FI], slv[G::FI], bsc[G::FJ];
+  // Step s = 2 g + T: the products of the hi parts beside the reads of the lo parts; then every
+  // read of the step's stages is done and, after the barrier, every wave's: the products of the
+  // lo parts beside the next step's reads and the DMAs that refill the x stage and, after its
+  // second step, the W stage.
+  // MODE 2: those are whole and in the range; 3: no W stage g + SW; 1: whatever is in the range,
+  // each barrier waiting for every DMA.
+  auto step = [&](auto mode_c, auto t_c, int g) __attribute__((always_inline)) {
+    constexpr int MODE = decltype(mode_c)::value, T = decltype(t_c)::value;
+    const int s = 2 * g + T;
 #pragma unroll
-    for (int i = 0; i < G::FI; ++i) {
-      ah[i] = p_frag(st, oa[i]);
-      al[i] = p_frag(st + G::TILE, oa[i]);
-      shv[i] = st[osa[i] + sb];
-      slv[i] = st[osa[i] + TS * 4 + sb];
-    }
+    for (int m = 0; m < NM; ++m) {
 #pragma unroll
-    for (int j = 0; j < G::FJ; ++j) {
-      bf[j] = p_frag(st + 2 * G::TILE, ob[j]);
-      bsc[j] = st[osb[j] + sb];
+      for (int i = m * FI / NM; i < (m + 1) * FI / NM; ++i) read_lo(s, i);
+      const int j = m / FI, i = m % FI;
+      acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(ah[i], bf[T][j], acc[i][j], 0, 0, 0, sa[T][i], 0,
+                                                                  sbw[T][j]);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    __builtin_amdgcn_sched_barrier(0);
-    if constexpr (GRP == 0) gp_lds_barrier();                // ends interval 2s
-    else if constexpr (DMA) gp_wait_barrier<G::NDMA>();      // ends interval 2s + 1
+    if constexpr (MODE >= 2) gp_wait_barrier<G::in_flight(T)>();
     else gp_wait_barrier<0>();
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (MODE == 1) {
+      if (s + SX < s_end) {
 #pragma unroll
-    for (int j = 0; j < G::FJ; ++j)
-#pragma unroll
-      for (int i = 0; i < G::FI; ++i) {
-        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(ah[i], bf[j], acc[i][j], 0, 0, 0, shv[i], 0, bsc[j]);
-        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(al[i], bf[j], acc[i][j], 0, 0, 0, slv[i], 0, bsc[j]);
+        for (int q = 0; q < NX; ++q) issue_x(q, s + SX);
       }
-    __builtin_amdgcn_sched_barrier(0);
-    if constexpr (GRP == 1) gp_barrier_only();               // ends interval 2s + 2
-    else if constexpr (DMA) gp_wait_barrier<G::NDMA>();      // ends interval 2s + 1
-    else gp_wait_barrier<0>();
-    __builtin_amdgcn_sched_barrier(0);
+      if (T == 1 && g + SW < g_end) issue_w_any(g + SW);
+    }
+    constexpr int NI = MODE == 1 ? 0 : NX + (T == 1 && MODE == 2 ? NWD : 0), NR = FJ + FI;
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+#pragma unroll
+      for (int i = m * NI / NM; i < (m + 1) * NI / NM; ++i) {
+        if (i < NX) issue_x(i, s + SX);
+        else issue_w(i - NX, g + SW);
+      }
+#pragma unroll
+      for (int q = m * NR / NM; q < (m + 1) * NR / NM; ++q) {
+        if (q < FJ) read_w(std::integral_constant<int, 1 - T>{}, s + 1, q);
+        else read_hi(std::integral_constant<int, 1 - T>{}, s + 1, q - FJ);
+      }
+      const int j = m / FI, i = m % FI;
+      acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(al[i], bf[T][j], acc[i][j], 0, 0, 1, sa[T][i], 0,
+                                                                  sbw[T][j]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
   };
-  auto pp_run = [&](auto grp_c) __attribute__((always_inline)) {
-    constexpr int GRP = decltype(grp_c)::value;
-    if constexpr (GRP == 1) gp_barrier_only();  // group 1 starts one interval late
-    int s = s_begin;
-    for (; s + 2 < s_end; ++s) pp_step(grp_c, std::true_type{}, s);
-    for (; s < s_end; ++s) pp_step(grp_c, std::false_type{}, s);
-    if constexpr (GRP == 0) gp_barrier_only();  // matches group 1's extra barrier
-  };
-  if (grp == 0) pp_run(std::integral_constant<int, 0>{});
-  else pp_run(std::integral_constant<int, 1>{});
+  int g = g_begin;
+  const int whole = min(g_end, K / (2 * X_BK));  // the stages that are whole
+#pragma unroll 1
+  for (; g + SW < whole; ++g) {
+    step(I2{}, I0{}, g);
+    step(I2{}, I1{}, g);
+  }
+  if (g + SW == whole && whole == g_end) {
+    step(I3{}, I0{}, g);
+    step(I3{}, I1{}, g);
+    ++g;
+  }
+#pragma unroll 1
+  for (; g < g_end; ++g) {
+    step(I1{}, I0{}, g);
+    if (2 * g + 1 < s_end) step(I1{}, I1{}, g);
+  }
+  gp_lds_barrier();
 
-  if (part) {  // a K range of a split tile: the raw accumulators
-    gp_store_partial<G::FI, G::FJ>(acc, part, wave, lane, M - (m0 + wm * (TS / 4)));
+  const int row0 = m0 + wm * 32 * FI;
+  if (blk.split) {
+    gp_store_partial<FI, FJ, G::NW>(acc, part + (size_t)((blk.t - whole_tiles) * S + blk.kr) * G::TM * G::TN, wave, lane,
+                                    M - row0);
     return;
   }
-  (void)steps;
-
-  // epilogue through LDS (the ring is idle: every wave has passed the last barrier,
-  // after which no fragment read or DMA is outstanding); wave w's region follows w - 1's
-  constexpr int REGION = 32 * G::FI * (64 * G::FJ + 32);
-  static_assert(8 * REGION <= G::LDS, "the epilogue regions fit the ring");
   const bool vec = yout_vec(yo);
-  gp_store_tile_bf16<G::FI, G::FJ, 0, G::FI>(acc, lds + wave * REGION, lane, yo, M, m0 + wm * (TS / 4),
-                                             n0 + wn * (TS / 2), n_end, vec);
-}
-
-// Covers x rows [0, M) and W rows [n_begin, n_end) in TS x TS tiles.
-template <int TS>
-__global__ __launch_bounds__(F_THREADS) void gemm_mxfp8_pipe_kernel(
-    const uint8_t *__restrict__ xh, const uint8_t *__restrict__ xl, const uint8_t *__restrict__ sh,
-    const uint8_t *__restrict__ sl, const uint8_t *__restrict__ w, const uint8_t *__restrict__ sw,
-    const YOut yo, int M, int N, int K, int n_begin, int n_end) {
-  pipe_tile<TS>(blockIdx.x, xh, xl, sh, sl, w, sw, yo, M, N, K, n_begin, n_end, 0, K / P_BK, nullptr);
-}
-
-// Both tilings in one launch: blocks [0, tiles1) are the 256-tiles of W rows [0, n_split),
-// the rest cover W rows [n_split, N) one of two ways:
-//   * S == 0: as 128-tiles;
-//   * S >= 2: as 256-tiles whose K steps are split S ways (split tiles): block tiles1 + u
-//     runs K range u % S of tile u / S and leaves its fp32 accumulators in part[u] (256 KiB
-//     each), which gemm_mxfp8_split_reduce_kernel then sums.
-// Blocks start in index order as CUs free up, so a CU that finishes its last 256-tile
-// early takes a tail block at once instead of waiting for the slowest CU at a kernel
-// boundary.  (The host gives tiles1 as whole rounds, a multiple of the CU count, so on a
-// CU count that is a multiple of 8 both parts keep their XCD-aware tile order; any
-// tiles1 gives the same results.)
-__global__ __launch_bounds__(F_THREADS) void gemm_mxfp8_pipe_split_kernel(
-    const uint8_t *__restrict__ xh, const uint8_t *__restrict__ xl, const uint8_t *__restrict__ sh,
-    const uint8_t *__restrict__ sl, const uint8_t *__restrict__ w, const uint8_t *__restrict__ sw,
-    const YOut yo, int M, int N, int K, int n_split, int tiles1, int S, float *__restrict__ part) {
-  const int b = blockIdx.x, steps = K / P_BK;
-  if (b < tiles1) {
-    pipe_tile<256>(b, xh, xl, sh, sl, w, sw, yo, M, N, K, 0, n_split, 0, steps, nullptr);
-  } else if (S == 0) {
-    pipe_tile<128>(b - tiles1, xh, xl, sh, sl, w, sw, yo, M, N, K, n_split, N, 0, steps, nullptr);
+  uint8_t *region = lds + wave * G::REGION;
+  if constexpr (MLP) {
+    f32x16_t h[FI][FJ / 2];
+    gp_silu_mul<FI, FJ>(acc, h);
+    gp_store_rows<FI, FJ / 2, 0>(h, region, lane, yo, M, row0, n0 + wn * 16 * FJ, N, vec);
   } else {
-    const int u = b - tiles1, t = u / S, k = u - t * S;
-    pipe_tile<256>(t, xh, xl, sh, sl, w, sw, yo, M, N, K, n_split, N, k * steps / S, (k + 1) * steps / S,
-                   part + (size_t)u * 256 * 256);
+    gp_store_rows<FI, FJ, 0>(acc, region, lane, yo, M, row0, n0 + wn * 32 * FJ, N, vec);
   }
 }
 
-// Every 128-tile split S ways along K, two blocks per CU (the 78 KiB ring and at most 128
-// registers per lane): for x of at most 128 rows, whose 256-tiles would be mostly padding.
-// Block b runs K range b % S of tile b / S into slot b of `part` (64 KiB each).
-__global__ __launch_bounds__(F_THREADS, 2) void gemm_mxfp8_pipe_ksplit128_kernel(
-    const uint8_t *__restrict__ xh, const uint8_t *__restrict__ xl, const uint8_t *__restrict__ sh,
-    const uint8_t *__restrict__ sl, const uint8_t *__restrict__ w, const uint8_t *__restrict__ sw,
-    const YOut yo, int M, int N, int K, int S, float *__restrict__ part) {
-  const int b = blockIdx.x, t = b / S, k = b - t * S, steps = K / P_BK;
-  pipe_tile<128>(t, xh, xl, sh, sl, w, sw, yo, M, N, K, 0, N, k * steps / S, (k + 1) * steps / S,
-                 part ? part + (size_t)b * 128 * 128 : nullptr);
+template <class G, bool MLP>
+__global__ __launch_bounds__(256) void gemm_mxfp8_reduce_kernel(const float *__restrict__ part, const YOut yo, int M,
+                                                                int N, int whole_tiles, int S) {
+  gp_reduce_tile<G, MLP>(part, yo, M, N, whole_tiles, S, blockIdx.x * 256 + threadIdx.x);
 }
 
-// The split tiles' results (TS-tiles of W rows [n_split, N)): one thread per float4 of a
-// tile's partial layout (gp_reduce_quad), fp8_reduce_blocks<TS> blocks of 256 per tile.
-template <int TS>
-constexpr int fp8_reduce_blocks() {
-  return 2 * PipeGeom<TS>::FI * PipeGeom<TS>::FJ * 4;
-}
-template <int TS>
-__global__ __launch_bounds__(256) void gemm_mxfp8_split_reduce_kernel(const float *__restrict__ part,
-                                                                       const YOut yo, int M, int N,
-                                                                       int n_split, int S) {
-  using G = PipeGeom<TS>;
-  constexpr int NQ = G::FI * G::FJ * 4;  // float4s per lane per wave
-  static_assert(8 * NQ * 64 == 256 * fp8_reduce_blocks<TS>(), "whole blocks per tile");
-  const int g = blockIdx.x * 256 + threadIdx.x;
-  const int t = g / (8 * NQ * 64), rem = g - t * (8 * NQ * 64);
-  const int wave = rem / (NQ * 64), q = (rem >> 6) % NQ, lane = rem & 63;
-  int tm, tn;
-  tile_of(t, (M + TS - 1) / TS, (N - n_split + TS - 1) / TS, &tm, &tn);
-  const int wm = wave >> 1, wn = wave & 1;
-  gp_reduce_quad<G::FI, G::FJ>(part, yo, M, N, t, S, wave, q, lane, tm * TS + wm * (TS / 4),
-                               n_split + tn * TS + wn * (TS / 2));
+// ---------------------------------------------------------------- the plan
+
+namespace {
+using Mx256 = MxGeom<4, 4, 2, 2, 2, 2>;  // 256 x 256
+using Mx192 = MxGeom<3, 4, 2, 2, 2, 2>;  // 192 x 256
+using MxW = MxGeom<2, 4, 2, 2, 3, 3>;    // 128 x 256
+using Mx128 = MxGeom<2, 2, 2, 2, 2, 2>;  // 128 x 128, two blocks per CU
+using Mx64 = MxGeom<1, 2, 2, 2, 3, 3>;   // 64 x 128, two blocks per CU
+using Mx160 = MxGeom<2, 5, 4, 1, 2, 2>;  // 256 x 160
+using Mx32 = MxGeom<1, 1, 1, 4, 3, 3>;   // 32 x 128, two blocks per CU
+// (fitted to 50 shapes of the declared range with every tile and split, rms error 8%; the
+// plan's choice is 1.01 of the best of them on average, at most 1.18.  The last two have no
+// MLP form: a wave's column blocks are not pairs.)
+constexpr GpCost MX_COST[] = {{256, 256, 1, 13.9f, {1.05f}},        {192, 256, 1, 13.4f, {0.83f}},
+                              {128, 256, 1, 13.6f, {0.61f}},        {128, 128, 2, 12.2f, {0.49f, 0.76f}},
+                              {64, 128, 2, 12.5f, {0.28f, 0.46f}},  {256, 160, 1, 13.7f, {0.72f}},
+                              {32, 128, 2, 11.8f, {0.24f, 0.40f}}};
+constexpr int MX_CONFIGS = sizeof(MX_COST) / sizeof(MX_COST[0]);
+}  // namespace
+
+static GpPlan mx_plan(const QmmArgs &a) {
+  return gp_plan(MX_COST, a.w_up ? MX_CONFIGS - 2 : MX_CONFIGS, a.M, a.w_up ? 2 * (int64_t)a.N : a.N, (a.K + X_BK - 1) / X_BK, 2,
+                 device_cu_count());
 }
 
-// K % 128: whole step pairs (the tile-major scale layout); W rows must be 16-byte
-// aligned for the DMA, and the W scales 4-byte aligned for the repack.
-static bool gemm_mxfp8_pipe_ok(const QmmArgs &a) {
-  return a.K % 128 == 0 && (uintptr_t)a.w % 16 == 0 && (uintptr_t)a.s % 4 == 0;
+// The workspace: the split x, its scales, the repacked W scales that do not come tile-major,
+// and the split tiles' fp32 partial sums; each part a multiple of 256 bytes.
+struct MxWs {
+  size_t xs, sx, sw, part;
+};
+static MxWs mx_ws(const QmmArgs &a, const GpPlan &p) {
+  const size_t steps = (a.K + X_BK - 1) / X_BK, rows = ((size_t)a.M + 255) & ~(size_t)255;
+  MxWs ws;
+  ws.xs = ((size_t)a.M * steps * 128 + 255) & ~(size_t)255;
+  ws.sx = rows * ((steps + 1) / 2 * 2) * 4;
+  ws.sw = tiled_scales_bytes(a.N, a.K / 32);
+  ws.part = (size_t)p.left * p.S * MX_COST[p.cfg].TM * MX_COST[p.cfg].TN * sizeof(float);
+  return ws;
 }
 
-static size_t round256(size_t v) { return (v + 255) & ~(size_t)255; }
+template <class G, bool MLP>
+static hipError_t launch_mx_tiles(const QmmArgs &a, const GpPlan &p, const uint8_t *xs, const uint32_t *sx,
+                                  const uint8_t *sp, const uint8_t *sp_up, float *part, hipStream_t st) {
+  static std::atomic<uint64_t> lds_set{0};
+  hipError_t e = ensure_dynamic_lds(lds_set, (const void *)gemm_mxfp8_kernel<G, MLP>, G::LDS);
+  if (e != hipSuccess) return e;
+  const YOut yo = yout_of(a);  // y, or a grouped call's parts
+  hipLaunchKernelGGL((gemm_mxfp8_kernel<G, MLP>), dim3(p.whole + p.left * p.S), dim3(G::THREADS), G::LDS, st, xs, sx, a.w,
+                     sp, a.w_up, sp_up, yo, a.M, a.N, a.K, p.whole, p.S, part);
+  e = hipGetLastError();
+  if (e != hipSuccess || p.left == 0) return e;
+  constexpr int RB = G::NW * G::FI * (MLP ? G::FJ / 2 : G::FJ);
+  hipLaunchKernelGGL((gemm_mxfp8_reduce_kernel<G, MLP>), dim3(p.left * RB), dim3(256), 0, st, (const float *)part, yo, a.M,
+                     a.N, p.whole, p.S);
+  return hipGetLastError();
+}
 
 hipError_t launch_repack_scales(const uint8_t *s, int64_t N, int nb, uint32_t *out, hipStream_t st) {
   const int dpr = (nb + 3) / 4;
   const bool dwords = nb % 4 == 0 && (uintptr_t)s % 4 == 0, wide = dwords && dpr % 4 == 0 && (uintptr_t)s % 16 == 0;
-  const int64_t threads = (int64_t)round256(N) * dpr / (wide ? 4 : 1);
+  const int64_t threads = ((N + 255) & ~(int64_t)255) * dpr / (wide ? 4 : 1);
   const int64_t blocks = (threads + 255) / 256 < 65536 ? (threads + 255) / 256 : 65536;
   if (wide)
     hipLaunchKernelGGL(repack_scales_kernel<4>, dim3(blocks), dim3(256), 0, st, s, N, nb, out);
@@ -631,169 +480,70 @@ hipError_t launch_repack_scales(const uint8_t *s, int64_t N, int nb, uint32_t *o
   return hipGetLastError();
 }
 
-int gemm_mxfp8_split_layout_of(const QmmArgs &a) { return gemm_mxfp8_pipe_ok(a) ? 1 : 0; }
+size_t tiled_scales_bytes(int64_t N, int nb) { return (((size_t)N + 255) & ~(size_t)255) * (size_t)((nb + 3) / 4 * 4); }
 
+int gemm_tiled_scale_bytes_per_row(const QmmArgs &a) {
+  if (qmm_on_decode(a)) return 0;
+  return gemm_mxfp8_ok(a) ? a.K / 32 : gemm_nvfp4_ok(a) ? a.K / 16 : 0;
+}
+
+// K % 32: whole scale blocks, 16-byte W pieces; x and W rows 16-byte aligned.
 bool gemm_mxfp8_ok(const QmmArgs &a) {
-  return a.mode == MXFP8 && !a.x_f32 && a.K % F_BK == 0 && a.K > 0 && a.M > 0 && a.N > 0;
-}
-
-// Workspace: x hi, x lo (M x K bytes each), x hi / lo scales, and for the pipelined
-// kernel the W scales repacked, each scale array padded to whole 256-row tiles.
-
-// How the pipelined GEMM covers the 256-tiles of a call on `cus` CUs:
-//   * a call of at most half as many tiles as CUs (short prefill chunks, narrow
-//     projections) runs every tile split S ways along K (S >= 2, at most one round of
-//     blocks, each at least 8 K steps): n_split = 0, tail_tiles = all tiles;
-//   * otherwise whole rounds of 256-tiles over W rows [0, n_split), and when the last
-//     partial round is whole W tile-columns and four times as many 128-tiles fit one
-//     round, those columns [n_split, N) run as 128-tiles (S = 0);
-//   * else the last round runs as it falls (n_split = N).
-// (Split tiles for a last partial round of a larger call measured slower at M = 4096,
-// N = 17408, K = 5120: the 64 MiB of partial sums cost more than the 128-tiles lose.)
-// x of at most 128 rows runs 128-tiles instead, two blocks per CU (TS = 128): split S
-// ways along K where they leave block slots idle, whole (S = 1, stored directly) where
-// there are more of them than slots.
-struct Fp8Plan {
-  int n_split, tiles1, tail_tiles, S, TS;
-};
-static int fp8_split_ways(int tiles, int capacity, int steps) {
-  int S = capacity / tiles;
-  if (S > 8) S = 8;
-  if (S > steps / 8) S = steps / 8;
-  return S >= 2 ? S : 0;
-}
-static Fp8Plan fp8_plan(const QmmArgs &a, int cus) {
-  const int tiles_m = (a.M + 255) / 256, tiles_n = (a.N + 255) / 256, steps = a.K / P_BK;
-  const int T = tiles_m * tiles_n;
-  Fp8Plan p{a.N, T, 0, 0, 256};
-  if (cus <= 0) return p;
-  const int T128 = ((a.M + 127) / 128) * ((a.N + 127) / 128);
-  if (a.M <= 128) {
-    const int S = fp8_split_ways(T128, 2 * cus, steps);
-    return Fp8Plan{0, 0, T128, S ? S : 1, 128};
-  }
-  if (2 * T <= cus) {
-    const int S = fp8_split_ways(T, cus, steps);
-    if (S) p = Fp8Plan{0, 0, T, S, 256};
-    return p;
-  }
-  const int rem = T % cus;
-  if (rem == 0 || rem % tiles_m != 0 || 4 * rem > cus || T <= cus) return p;
-  p.n_split = (tiles_n - rem / tiles_m) * 256;
-  p.tiles1 = tiles_m * (tiles_n - rem / tiles_m);
-  return p;
+  return a.mode == MXFP8 && !a.x_f32 && a.K % 32 == 0 && a.K > 0 && a.M > 0 && a.N > 0 && (uintptr_t)a.x % 16 == 0 &&
+         (uintptr_t)a.w % 16 == 0 && (uintptr_t)a.w_up % 16 == 0;
 }
 
 size_t gemm_mxfp8_workspace(const QmmArgs &a) {
-  const size_t mk = round256(a.M) * a.K, nbk = (size_t)a.K / 32;
-  const bool pipe = gemm_mxfp8_pipe_ok(a);
-  const bool repack = pipe && !a.s_tiled;
-  size_t bytes = 2 * mk + 2 * round256(a.M) * nbk + (repack ? round256(a.N) * nbk : 0);
-  if (pipe) {  // the split tiles' fp32 partials, 256 KiB per block, 256-byte aligned
-    const Fp8Plan p = fp8_plan(a, device_cu_count());
-    if (p.S >= 2) bytes = round256(bytes) + (size_t)p.tail_tiles * p.S * p.TS * p.TS * 4;
-  }
-  return bytes + 256;
+  const MxWs ws = mx_ws(a, mx_plan(a));
+  return ws.xs + ws.sx + (a.s_tiled ? 0 : ws.sw) + (a.w_up && !a.s_up_tiled ? ws.sw : 0) + ws.part;
 }
 
-size_t tiled_scales_bytes(int64_t N, int nb) { return (size_t)round256((size_t)N) * (size_t)((nb + 3) / 4 * 4); }
-
-int gemm_tiled_scale_bytes_per_row(const QmmArgs &a) {
-  if (qmm_on_decode(a) || a.x_f32 || a.K <= 0) return 0;
-  if (gemm_mxfp8_ok(a)) return gemm_mxfp8_pipe_ok(a) && (uintptr_t)a.x % 16 == 0 ? a.K / 32 : 0;
-  if (gemm_nvfp4_ok(a)) return a.K / 16;
-  return 0;
-}
-
-hipError_t launch_gemm_mxfp8(const QmmArgs &a, void *ws, hipStream_t st) {
+hipError_t launch_gemm_mxfp8(const QmmArgs &a, void *workspace, hipStream_t st) {
   if (!gemm_mxfp8_ok(a)) return hipErrorInvalidValue;
-  const size_t mk = round256(a.M) * a.K, nbk = (size_t)a.K / 32;
-  uint8_t *xh = (uint8_t *)ws, *xl = xh + mk, *sh = xl + mk, *sl = sh + round256(a.M) * nbk;
-  uint8_t *swp = sl + round256(a.M) * nbk;
-  const bool pipe = gemm_mxfp8_pipe_ok(a);
-  // one thread per (row, 16 elements); the packed form covers rows in groups of 16 and
-  // U steps per thread (4 when K % 256 == 0, else 2: K % 128 == 0 there)
-  const int64_t rows_t = pipe ? ((int64_t)a.M + 15) / 16 * 16 : (int64_t)a.M;
-  const int U = pipe && a.K % 256 == 0 ? 4 : 2;
-  const int64_t total = rows_t * (a.K / 16) / (pipe ? U : 1);
-  if (rows_t * (a.K / 16) >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
-  const unsigned sb = (unsigned)((total + 255) / 256);
-  if (a.x_split_ready)
-    ;  // the previous call on this stream left this x split in this workspace
-  else if (pipe && U == 4)
-    hipLaunchKernelGGL(split_x_packed_kernel<4>, dim3(sb), dim3(256), 0, st, (const uint16_t *)a.x, (uint32_t)total,
-                       a.M, a.K, xh, xl, sh, sl);
-  else if (pipe)
-    hipLaunchKernelGGL(split_x_packed_kernel<2>, dim3(sb), dim3(256), 0, st, (const uint16_t *)a.x, (uint32_t)total,
-                       a.M, a.K, xh, xl, sh, sl);
+  const int steps = (a.K + X_BK - 1) / X_BK;
+  const GpPlan p = mx_plan(a);
+  const MxWs ws = mx_ws(a, p);
+  uint8_t *xs = (uint8_t *)workspace, *next = xs + ws.xs + ws.sx;
+  uint32_t *sx = (uint32_t *)(xs + ws.xs);
+  // U steps per wave: enough waves to fill the chip first, then 4 for the loads in flight
+  const int64_t rg = ((int64_t)a.M + 15) / 16;
+  const int U = rg * steps >= 4 * 4096 ? 4 : 1;
+  const int64_t waves = rg * ((steps + U - 1) / U);
+  if (waves >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
+  if (U == 4)
+    hipLaunchKernelGGL(split_x_kernel<4>, dim3((waves + 3) / 4), dim3(256), 0, st, (const uint16_t *)a.x, a.M, a.K, steps, xs, sx);
   else
-    hipLaunchKernelGGL(split_x_kernel, dim3(sb), dim3(256), 0, st, (const uint16_t *)a.x, (uint32_t)total, a.M, a.K,
-                       xh, xl, sh, sl);
+    hipLaunchKernelGGL(split_x_kernel<1>, dim3((waves + 3) / 4), dim3(256), 0, st, (const uint16_t *)a.x, a.M, a.K, steps, xs, sx);
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  const int tiles = ((a.M + F_BM - 1) / F_BM) * ((a.N + F_BN - 1) / F_BN);
-  if (pipe) {
-    if (a.s_tiled) {
-      swp = (uint8_t *)a.s_tiled;  // already tile-major
-    } else {
-      e = launch_repack_scales(a.s, (int64_t)a.N, a.K / 32, (uint32_t *)swp, st);
-      if (e != hipSuccess) return e;
-    }
-    static std::atomic<uint64_t> lds256{0}, lds_split{0};
-    e = ensure_dynamic_lds(lds256, (const void *)gemm_mxfp8_pipe_kernel<256>, (int)PipeGeom<256>::LDS);
-    if (e == hipSuccess)
-      e = ensure_dynamic_lds(lds_split, (const void *)gemm_mxfp8_pipe_split_kernel, (int)PipeGeom<256>::LDS);
-    if (e != hipSuccess) return e;
-    const int cus = device_cu_count();
-    if (cus <= 0) return hipErrorNoDevice;
-    // One block per CU at a time (the ring fills most of a CU's LDS); see fp8_plan for
-    // how the last partial round runs.
-    const Fp8Plan p = fp8_plan(a, cus);
-    const YOut yo = yout_of(a);  // y, or a grouped call's parts
-    if (p.n_split == a.N) {
-      hipLaunchKernelGGL(gemm_mxfp8_pipe_kernel<256>, dim3(p.tiles1), dim3(F_THREADS), PipeGeom<256>::LDS, st, xh, xl,
-                         sh, sl, a.w, swp, yo, a.M, a.N, a.K, 0, a.N);
-      return hipGetLastError();
-    }
-    if (p.S == 0) {
-      const int tiles2 = ((a.M + 127) / 128) * ((a.N - p.n_split + 127) / 128);
-      hipLaunchKernelGGL(gemm_mxfp8_pipe_split_kernel, dim3(p.tiles1 + tiles2), dim3(F_THREADS), PipeGeom<256>::LDS,
-                         st, xh, xl, sh, sl, a.w, swp, yo, a.M, a.N, a.K, p.n_split, p.tiles1, 0,
-                         (float *)nullptr);
-      return hipGetLastError();
-    }
-    // the partials follow the workspace's x split and (when made here) repacked scales
-    const size_t part_off = round256(2 * mk + 2 * round256(a.M) * nbk + (a.s_tiled ? 0 : round256(a.N) * nbk));
-    float *part = (float *)((uint8_t *)ws + part_off);
-    if (p.TS == 128) {
-      static std::atomic<uint64_t> lds128{0};
-      e = ensure_dynamic_lds(lds128, (const void *)gemm_mxfp8_pipe_ksplit128_kernel, (int)PipeGeom<128>::LDS);
-      if (e != hipSuccess) return e;
-      hipLaunchKernelGGL(gemm_mxfp8_pipe_ksplit128_kernel, dim3(p.tail_tiles * p.S), dim3(F_THREADS),
-                         PipeGeom<128>::LDS, st, xh, xl, sh, sl, a.w, swp, yo, a.M, a.N, a.K, p.S,
-                         p.S >= 2 ? part : (float *)nullptr);
-      e = hipGetLastError();
-      if (e != hipSuccess || p.S < 2) return e;
-      hipLaunchKernelGGL(gemm_mxfp8_split_reduce_kernel<128>, dim3(p.tail_tiles * fp8_reduce_blocks<128>()), dim3(256), 0,
-                         st, (const float *)part, yo, a.M, a.N, 0, p.S);
-      return hipGetLastError();
-    }
-    hipLaunchKernelGGL(gemm_mxfp8_pipe_split_kernel, dim3(p.tiles1 + p.tail_tiles * p.S), dim3(F_THREADS),
-                       PipeGeom<256>::LDS, st, xh, xl, sh, sl, a.w, swp, yo, a.M, a.N, a.K, p.n_split,
-                       p.tiles1, p.S, part);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(gemm_mxfp8_split_reduce_kernel<256>, dim3(p.tail_tiles * fp8_reduce_blocks<256>()), dim3(256), 0,
-                       st, (const float *)part, yo, a.M, a.N, p.n_split, p.S);
-    return hipGetLastError();
+  const uint8_t *sp = (const uint8_t *)a.s_tiled, *sp_up = (const uint8_t *)a.s_up_tiled;
+  if (e == hipSuccess && !sp) {
+    e = launch_repack_scales(a.s, a.N, a.K / 32, (uint32_t *)next, st);
+    sp = next, next += ws.sw;
   }
-  if (a.parts) return hipErrorInvalidValue;  // (grouped calls run the pipelined kernels only)
-  static std::atomic<uint64_t> lds_set{0};
-  e = ensure_dynamic_lds(lds_set, (const void *)gemm_mxfp8_kernel, (int)sizeof(Fp8Smem));
+  if (e == hipSuccess && a.w_up && !sp_up) {
+    e = launch_repack_scales(a.s_up, a.N, a.K / 32, (uint32_t *)next, st);
+    sp_up = next, next += ws.sw;
+  }
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(gemm_mxfp8_kernel, dim3(tiles), dim3(F_THREADS), sizeof(Fp8Smem), st, xh, xl, sh, sl, a.w, a.s,
-                     (uint16_t *)a.y, a.M, a.N, a.K);
-  return hipGetLastError();
+  float *part = (float *)next;
+  if (a.w_up) {
+    switch (p.cfg) {
+      case 0: return launch_mx_tiles<Mx256, true>(a, p, xs, sx, sp, sp_up, part, st);
+      case 1: return launch_mx_tiles<Mx192, true>(a, p, xs, sx, sp, sp_up, part, st);
+      case 2: return launch_mx_tiles<MxW, true>(a, p, xs, sx, sp, sp_up, part, st);
+      case 3: return launch_mx_tiles<Mx128, true>(a, p, xs, sx, sp, sp_up, part, st);
+      default: return launch_mx_tiles<Mx64, true>(a, p, xs, sx, sp, sp_up, part, st);
+    }
+  }
+  switch (p.cfg) {
+    case 0: return launch_mx_tiles<Mx256, false>(a, p, xs, sx, sp, sp_up, part, st);
+    case 1: return launch_mx_tiles<Mx192, false>(a, p, xs, sx, sp, sp_up, part, st);
+    case 2: return launch_mx_tiles<MxW, false>(a, p, xs, sx, sp, sp_up, part, st);
+    case 3: return launch_mx_tiles<Mx128, false>(a, p, xs, sx, sp, sp_up, part, st);
+    case 4: return launch_mx_tiles<Mx64, false>(a, p, xs, sx, sp, sp_up, part, st);
+    case 5: return launch_mx_tiles<Mx160, false>(a, p, xs, sx, sp, sp_up, part, st);
+    default: return launch_mx_tiles<Mx32, false>(a, p, xs, sx, sp, sp_up, part, st);
+  }
 }
 
 }  // namespace qmm

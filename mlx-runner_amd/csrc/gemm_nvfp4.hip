@@ -67,20 +67,26 @@ __device__ const uint4 nv_zero = {0, 0, 0, 0};
 // 16-byte piece p of a row's 128 bytes is stored at slot p ^ nv_swz(row).
 __device__ __forceinline__ int nv_swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 
-template <class G>
+// MLP: the tile's W rows are two matrices', 32-row blocks of gate and of up in turn (row
+// blocks 2 b and 2 b + 1 of a tile are rows 32 b + [0, 32) of the tile's TN / 2), and the
+// result is silu(gate) * up, TN / 2 columns of it per tile.
+template <class G, bool MLP>
 __global__ __launch_bounds__(G::THREADS, G::LDS <= 81920 ? 2 * G::NW / 4 : G::NW / 4) void gemm_nvfp4_kernel(
-    const uint16_t *__restrict__ x, const uint8_t *__restrict__ w, const uint8_t *__restrict__ sp, const YOut yo, int M,
-    int N, int K, int whole_tiles, int S, float *__restrict__ part) {
+    const uint16_t *__restrict__ x, const uint8_t *__restrict__ w, const uint8_t *__restrict__ sp,
+    const uint8_t *__restrict__ w_up, const uint8_t *__restrict__ sp_up, const YOut yo, int M, int N, int K,
+    int whole_tiles, int S, float *__restrict__ part) {
   constexpr int FI = G::FI, FJ = G::FJ, NX = G::NX, NWD = G::NWD, SX = G::SX;
+  constexpr int TC = MLP ? G::TN / 2 : G::TN;  // columns of y per tile
+  static_assert(!MLP || FJ % 2 == 0, "a wave holds gate and up of a column");
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const uint32_t lds0 = lds_addr(lds);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % G::WM, wn = wave / G::WM;
-  const int tiles_m = (M + G::TM - 1) / G::TM, tiles_n = (N + G::TN - 1) / G::TN;
+  const int tiles_m = (M + G::TM - 1) / G::TM, tiles_n = (N + TC - 1) / TC;
   const int steps = (K + V_BK - 1) / V_BK, stages = (steps + V_SS - 1) / V_SS;
   const GpBlock blk = gp_block(blockIdx.x, tiles_m, tiles_n, whole_tiles, S);
-  const int m0 = blk.tm * G::TM, n0 = blk.tn * G::TN;
+  const int m0 = blk.tm * G::TM, n0 = blk.tn * TC;
   // the block's W stages [g_begin, g_end) and steps [s_begin, s_end)
   const int g_begin = blk.split ? (int)((int64_t)blk.kr * stages / S) : 0;
   const int g_end = blk.split ? (int)((int64_t)(blk.kr + 1) * stages / S) : stages;
@@ -89,24 +95,35 @@ __global__ __launch_bounds__(G::THREADS, G::LDS <= 81920 ? 2 * G::NW / 4 : G::NW
   // A DMA fills 1 KiB: rows 8 g + [0, 8) of a stage of x (or W), g = wave + NW i; lane l the
   // 16-byte slot l % 8 of row l / 8, which holds piece (l % 8) ^ swz(row) of the row's 128 bytes.
   const int64_t wrow = K >> 1;
-  const uint8_t *xb = (const uint8_t *)x + (int64_t)m0 * K * 2, *wb = w + (int64_t)n0 * wrow;
+  const uint8_t *xb = (const uint8_t *)x + (int64_t)m0 * K * 2;
   const int dr = 8 * wave + (lane >> 3), dp = (lane & 7) ^ nv_swz(dr);  // rows 8 NW apart share a swizzle
   uint32_t xo[NX], wo[NWD];
+  const uint8_t *wb[MLP ? NWD : 1];
 #pragma unroll
   for (int i = 0; i < NX; ++i) xo[i] = (uint32_t)(min(m0 + dr + 8 * G::NW * i, M - 1) - m0) * (uint32_t)(2 * K) + dp * 16;
+  if constexpr (!MLP) wb[0] = w + (int64_t)n0 * wrow;
 #pragma unroll
-  for (int i = 0; i < NWD; ++i) wo[i] = (uint32_t)((min(n0 + dr + 8 * G::NW * i, N - 1) - n0) * wrow) + dp * 16;
+  for (int i = 0; i < NWD; ++i) {
+    const int q = wave + G::NW * i, r = dr + 8 * G::NW * i;  // 8 rows of one 32-row block
+    int row = r;
+    if constexpr (MLP) {
+      wb[i] = ((q >> 2) & 1 ? w_up : w) + (int64_t)n0 * wrow;
+      row = (r >> 6) * 32 + (r & 31);
+    }
+    wo[i] = (uint32_t)((min(n0 + row, N - 1) - n0) * wrow) + dp * 16;
+  }
   // scales: the tile-major copy holds, per 256 rows and step, 256 dwords; a stage's V_SS x TN
   // dwords take TN / 64 DMAs of four rows per lane, one per wave (the waves past that repeat one)
-  const int sq = (wave % (G::TN / 64)) * 64 + lane, sd = sq / (G::TN / 4), sr = n0 + sq % (G::TN / 4) * 4;
-  const uint8_t *sb = sp + ((int64_t)(sr >> 8) * steps * 256 + (sr & 255)) * 4;
+  const int sq = (wave % (G::TN / 64)) * 64 + lane, sd = sq / (G::TN / 4), st = sq % (G::TN / 4) * 4;
+  const int sr = min(n0 + (MLP ? (st >> 6) * 32 + (st & 31) : st), ((N + 255) & ~255) - 4);
+  const uint8_t *sb = (MLP && (st >> 5) & 1 ? sp_up : sp) + ((int64_t)(sr >> 8) * steps * 256 + (sr & 255)) * 4;
   const uint32_t sl = (uint32_t)(G::SOFF + (wave % (G::TN / 64)) * 1024);
 
   auto issue_x = [&](int i, int s) __attribute__((always_inline)) {
     gp_dma16s(xb + (int64_t)s * 128, xo[i], lds0 + (uint32_t)((s % SX) * G::XT + (wave + G::NW * i) * 1024));
   };
   auto issue_w = [&](int i, int g) __attribute__((always_inline)) {
-    gp_dma16s(wb + (int64_t)g * 128, wo[i], lds0 + (uint32_t)(G::WOFF + (g & 1) * G::WT + (wave + G::NW * i) * 1024));
+    gp_dma16s(wb[MLP ? i : 0] + (int64_t)g * 128, wo[i], lds0 + (uint32_t)(G::WOFF + (g & 1) * G::WT + (wave + G::NW * i) * 1024));
   };
   // (a stage's steps past the last one repeat it)
   auto issue_s = [&](int g) __attribute__((always_inline)) {
@@ -133,7 +150,7 @@ __global__ __launch_bounds__(G::THREADS, G::LDS <= 81920 ? 2 * G::NW / 4 : G::NW
       if ((g + 1) * V_SS * V_BK <= K) {
         issue_w(i, g);
       } else {
-        const uint8_t *p = wb + wo[i] + (int64_t)g * 128;
+        const uint8_t *p = wb[MLP ? i : 0] + wo[i] + (int64_t)g * 128;
         if (g * V_SS * V_BK + 32 * dp >= K) p = (const uint8_t *)&nv_zero;
         gp_dma16(p, lds0 + (uint32_t)(G::WOFF + (g & 1) * G::WT + (wave + G::NW * i) * 1024));
       }
@@ -300,7 +317,7 @@ __global__ __launch_bounds__(G::THREADS, G::LDS <= 81920 ? 2 * G::NW / 4 : G::NW
   }
   gp_lds_barrier();
 
-  const int row0 = m0 + wm * 32 * FI, col0 = n0 + wn * 32 * FJ;
+  const int row0 = m0 + wm * 32 * FI;
   if (blk.split) {
     gp_store_partial<FI, FJ, G::NW>(acc, part + (size_t)((blk.t - whole_tiles) * S + blk.kr) * G::TM * G::TN, wave, lane,
                                     M - row0);
@@ -308,13 +325,19 @@ __global__ __launch_bounds__(G::THREADS, G::LDS <= 81920 ? 2 * G::NW / 4 : G::NW
   }
   const bool vec = yout_vec(yo);
   uint8_t *region = lds + wave * G::REGION;
-  gp_store_rows<FI, FJ, 0>(acc, region, lane, yo, M, row0, col0, N, vec);
+  if constexpr (MLP) {
+    f32x16_t h[FI][FJ / 2];
+    gp_silu_mul<FI, FJ>(acc, h);
+    gp_store_rows<FI, FJ / 2, 0>(h, region, lane, yo, M, row0, n0 + wn * 16 * FJ, N, vec);
+  } else {
+    gp_store_rows<FI, FJ, 0>(acc, region, lane, yo, M, row0, n0 + wn * 32 * FJ, N, vec);
+  }
 }
 
-template <class G>
+template <class G, bool MLP>
 __global__ __launch_bounds__(256) void gemm_nvfp4_reduce_kernel(const float *__restrict__ part, const YOut yo, int M,
                                                                 int N, int whole_tiles, int S) {
-  gp_reduce_tile<G>(part, yo, M, N, whole_tiles, S, blockIdx.x * 256 + threadIdx.x);
+  gp_reduce_tile<G, MLP>(part, yo, M, N, whole_tiles, S, blockIdx.x * 256 + threadIdx.x);
 }
 
 // ---------------------------------------------------------------- the plan
@@ -333,57 +356,81 @@ constexpr GpCost NV_COST[] = {{256, 256, 1, 9.7f, {1.10f}},         {192, 256, 1
                               {64, 128, 2, 8.6f, {0.26f, 0.43f}},   {32, 128, 3, 8.4f, {0.22f, 0.34f, 0.48f}}};
 }  // namespace
 
+// The MLP form needs a wave's column blocks in pairs: at 128 columns, 2 x 2 waves.
+using Nv128M = NvGeom<2, 2, 2, 2, 2>;  // 128 x 128, two blocks per CU
+using Nv64M = NvGeom<1, 2, 2, 2, 4>;   // 64 x 128, two blocks per CU
+
 static GpPlan nv_plan(const QmmArgs &a) {
-  return gp_plan(NV_COST, sizeof(NV_COST) / sizeof(NV_COST[0]), a.M, a.N, (a.K + V_BK - 1) / V_BK, V_SS,
+  const int n = sizeof(NV_COST) / sizeof(NV_COST[0]);
+  return gp_plan(NV_COST, a.w_up ? n - 1 : n, a.M, a.w_up ? 2 * (int64_t)a.N : a.N, (a.K + V_BK - 1) / V_BK, V_SS,
                  device_cu_count());
 }
 
-template <class G>
-static hipError_t launch_nv(const QmmArgs &a, const GpPlan &p, const uint8_t *tiled, float *part, hipStream_t st) {
+template <class G, bool MLP>
+static hipError_t launch_nv(const QmmArgs &a, const GpPlan &p, const uint8_t *sp, const uint8_t *sp_up, float *part,
+                            hipStream_t st) {
   static std::atomic<uint64_t> lds_set{0};
-  hipError_t e = ensure_dynamic_lds(lds_set, (const void *)gemm_nvfp4_kernel<G>, G::LDS);
+  hipError_t e = ensure_dynamic_lds(lds_set, (const void *)gemm_nvfp4_kernel<G, MLP>, G::LDS);
   if (e != hipSuccess) return e;
   const YOut yo = yout_of(a);  // y, or a grouped call's parts
-  hipLaunchKernelGGL((gemm_nvfp4_kernel<G>), dim3(p.whole + p.left * p.S), dim3(G::THREADS), G::LDS, st,
-                     (const uint16_t *)a.x, a.w, tiled, yo, a.M, a.N, a.K, p.whole, p.S, part);
+  hipLaunchKernelGGL((gemm_nvfp4_kernel<G, MLP>), dim3(p.whole + p.left * p.S), dim3(G::THREADS), G::LDS, st,
+                     (const uint16_t *)a.x, a.w, sp, a.w_up, sp_up, yo, a.M, a.N, a.K, p.whole, p.S, part);
   e = hipGetLastError();
   if (e != hipSuccess || p.left == 0) return e;
-  hipLaunchKernelGGL((gemm_nvfp4_reduce_kernel<G>), dim3(p.left * (G::NW * G::FI * G::FJ)), dim3(256), 0, st,
-                     (const float *)part, yo, a.M, a.N, p.whole, p.S);
+  constexpr int RB = G::NW * G::FI * (MLP ? G::FJ / 2 : G::FJ);
+  hipLaunchKernelGGL((gemm_nvfp4_reduce_kernel<G, MLP>), dim3(p.left * RB), dim3(256), 0, st, (const float *)part, yo,
+                     a.M, a.N, p.whole, p.S);
   return hipGetLastError();
 }
 
 // K % 32: 16-byte W pieces; x and W rows 16-byte aligned for the DMA.
 bool gemm_nvfp4_ok(const QmmArgs &a) {
   return a.mode == NVFP4 && !a.x_f32 && a.K % 32 == 0 && a.K > 0 && a.M > 0 && a.N > 0 && (uintptr_t)a.x % 16 == 0 &&
-         (uintptr_t)a.w % 16 == 0;
+         (uintptr_t)a.w % 16 == 0 && (uintptr_t)a.w_up % 16 == 0;
 }
 
-// Workspace: the scales repacked tile-major, unless they come so (a.s_tiled), then the split
-// tiles' fp32 partial sums.
-static size_t nv_scales_bytes(const QmmArgs &a) { return a.s_tiled ? 0 : tiled_scales_bytes(a.N, a.K / 16); }
+// Workspace: the scales repacked tile-major, unless they come so, then the split tiles' fp32
+// partial sums.
 size_t gemm_nvfp4_workspace(const QmmArgs &a) {
   const GpPlan p = nv_plan(a);
-  return nv_scales_bytes(a) + (size_t)p.left * p.S * NV_COST[p.cfg].TM * NV_COST[p.cfg].TN * sizeof(float);
+  const size_t sw = tiled_scales_bytes(a.N, a.K / 16);
+  return (a.s_tiled ? 0 : sw) + (a.w_up && !a.s_up_tiled ? sw : 0) +
+         (size_t)p.left * p.S * NV_COST[p.cfg].TM * NV_COST[p.cfg].TN * sizeof(float);
 }
 
 hipError_t launch_gemm_nvfp4(const QmmArgs &a, void *ws, hipStream_t st) {
   if (!gemm_nvfp4_ok(a)) return hipErrorInvalidValue;
-  const uint8_t *tiled = (const uint8_t *)a.s_tiled;
-  if (!tiled) {
-    const hipError_t e = launch_repack_scales(a.s, (int64_t)a.N, a.K / 16, (uint32_t *)ws, st);
-    if (e != hipSuccess) return e;
-    tiled = (const uint8_t *)ws;
+  const uint8_t *sp = (const uint8_t *)a.s_tiled, *sp_up = (const uint8_t *)a.s_up_tiled;
+  uint8_t *next = (uint8_t *)ws;
+  const size_t sw = tiled_scales_bytes(a.N, a.K / 16);  // (a multiple of 1 KiB)
+  hipError_t e = hipSuccess;
+  if (!sp) {
+    e = launch_repack_scales(a.s, a.N, a.K / 16, (uint32_t *)next, st);
+    sp = next, next += sw;
   }
-  float *part = (float *)((uint8_t *)ws + nv_scales_bytes(a));  // (a multiple of 1 KiB)
+  if (e == hipSuccess && a.w_up && !sp_up) {
+    e = launch_repack_scales(a.s_up, a.N, a.K / 16, (uint32_t *)next, st);
+    sp_up = next, next += sw;
+  }
+  if (e != hipSuccess) return e;
+  float *part = (float *)next;
   const GpPlan p = nv_plan(a);
+  if (a.w_up) {
+    switch (p.cfg) {
+      case 0: return launch_nv<Nv256, true>(a, p, sp, sp_up, part, st);
+      case 1: return launch_nv<Nv192, true>(a, p, sp, sp_up, part, st);
+      case 2: return launch_nv<NvW, true>(a, p, sp, sp_up, part, st);
+      case 3: return launch_nv<Nv128M, true>(a, p, sp, sp_up, part, st);
+      default: return launch_nv<Nv64M, true>(a, p, sp, sp_up, part, st);
+    }
+  }
   switch (p.cfg) {
-    case 0: return launch_nv<Nv256>(a, p, tiled, part, st);
-    case 1: return launch_nv<Nv192>(a, p, tiled, part, st);
-    case 2: return launch_nv<NvW>(a, p, tiled, part, st);
-    case 3: return launch_nv<Nv128>(a, p, tiled, part, st);
-    case 4: return launch_nv<Nv64>(a, p, tiled, part, st);
-    default: return launch_nv<Nv32>(a, p, tiled, part, st);
+    case 0: return launch_nv<Nv256, false>(a, p, sp, sp_up, part, st);
+    case 1: return launch_nv<Nv192, false>(a, p, sp, sp_up, part, st);
+    case 2: return launch_nv<NvW, false>(a, p, sp, sp_up, part, st);
+    case 3: return launch_nv<Nv128, false>(a, p, sp, sp_up, part, st);
+    case 4: return launch_nv<Nv64, false>(a, p, sp, sp_up, part, st);
+    default: return launch_nv<Nv32, false>(a, p, sp, sp_up, part, st);
   }
 }
 

@@ -8,27 +8,11 @@
 
 namespace qmm {
 
-// Tile order: the hardware hands workgroup b to XCD b % 8.  Each XCD gets a
-// contiguous run of tile indices, and tiles are numbered in groups of 4 M-tiles
-// walked down M first, so the ~32 blocks resident on one XCD cover a 4 x 8
-// patch of (x rows, W rows) and share those operand slabs in that XCD's L2.
-__device__ __forceinline__ void tile_of(int b, int tiles_m, int tiles_n, int *tm, int *tn) {
-  const int T = tiles_m * tiles_n;
-  const int base = T / 8, rem = T % 8;
-  const int x = b % 8, local = b / 8;
-  const int t = x * base + (x < rem ? x : rem) + local;
-  constexpr int G = 4;
-  const int group = t / (G * tiles_n);
-  const int first_m = group * G;
-  const int gm = (tiles_m - first_m) < G ? (tiles_m - first_m) : G;
-  const int idx = t - group * G * tiles_n;
-  *tm = first_m + idx % gm;
-  *tn = idx / gm;
-}
-
 // A call's blocks: [0, whole_tiles) run whole tiles, the others the S K-ranges of the tiles
-// that are left (whole_tiles on).  Tiles are numbered in tile_of's order; each XCD (block %
-// 8) takes a contiguous run, and of a call that is all split, at few x tiles, the x tiles of
+// that are left (whole_tiles on).  Tiles are numbered in groups of 4 x tiles walked down x
+// tiles first, and each XCD (the hardware hands it the blocks b with b % 8 = its number)
+// takes a contiguous run of them, so the ~32 blocks resident on one XCD cover a 4 x 8 patch of
+// (x rows, W rows) and share those operands in that XCD's L2.  Of a call that is all split, at few x tiles, the x tiles of
 // one W range of one K range run next to each other, so that they share its W.
 struct GpBlock {
   int t, tm, tn, kr;
@@ -62,22 +46,15 @@ __device__ __forceinline__ GpBlock gp_block(int b, int tiles_m, int tiles_n, int
 
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
-// LDS DMA: lane i's 16 (4) bytes at g land at LDS byte l + 16 i (4 i); l must be
+// LDS DMA: lane i's 16 bytes at g land at LDS byte l + 16 i; l must be
 // wave-uniform.  Issued from assembly so that the compiler inserts no waits of
 // its own for it: every user waits explicitly with s_waitcnt vmcnt.
 __device__ __forceinline__ void gp_dma16(const void *g, uint32_t l) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(l), "v"(g) : "memory", "m0");
 }
-__device__ __forceinline__ void gp_dma4(const void *g, uint32_t l) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(l), "v"(g) : "memory", "m0");
-}
 // The same with the source as a wave-uniform base (SGPRs) plus a 32-bit lane offset.
 __device__ __forceinline__ void gp_dma16s(const void *base, uint32_t off, uint32_t l) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(l), "v"(off), "s"(base)
-               : "memory", "m0");
-}
-__device__ __forceinline__ void gp_dma4s(const void *base, uint32_t off, uint32_t l) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(l), "v"(off), "s"(base)
                : "memory", "m0");
 }
 #pragma clang diagnostic pop
@@ -89,7 +66,6 @@ __device__ __forceinline__ void gp_wait_barrier() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 __device__ __forceinline__ void gp_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-__device__ __forceinline__ void gp_barrier_only() { asm volatile("s_barrier" ::: "memory"); }
 
 __device__ __forceinline__ uint32_t lds_addr(const void *p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t *)p;
@@ -195,48 +171,65 @@ __device__ __forceinline__ void gp_store_partial(const f32x16_t (&acc)[FI][FJ], 
   }
 }
 
-// The split-tile reduce, one thread per float4 of the partial layout: float4 (wave, q, lane)
-// of split tile t, q = (i FJ + j) 4 + v4, is summed over the tile's S <= GP_MAX_SPLIT slots
-// (t S .. t S + S - 1) in K order, the same order whichever block finished first, so the
-// result is deterministic.  Its four values are rows 32 i + 8 v4 + 4 (lane / 32) + [0, 4),
-// column 32 j + lane % 32 of the wave's region at (row0, col0) of y (yo.at); they are rounded to bf16
-// as the tile epilogue rounds (rows from M on and columns from col_end on are not stored).
+// The split-tile reduce: the float4 at p is summed over the tile's S <= GP_MAX_SPLIT slots in
+// K order, the same order whichever block finished first, so the result is deterministic.
 // All S loads are issued before the first add, so a thread waits for one round trip, not S.
 constexpr int GP_MAX_SPLIT = 8;
-template <int FI, int FJ, int NW = 8>
-__device__ __forceinline__ void gp_reduce_quad(const float *__restrict__ part, const YOut yo, int M, int col_end,
-                                               int t, int S, int wave, int q, int lane, int row0, int col0) {
-  const int i = q / (FJ * 4), j = (q / 4) % FJ, v4 = q % 4;
-  const int r = row0 + 32 * i + 8 * v4 + 4 * (lane >> 5), c = col0 + 32 * j + (lane & 31);
-  if (r >= M || c >= col_end) return;  // not stored by the split blocks either (rows past M)
-  const float4 *pw = (const float4 *)part + ((size_t)t * S * NW + wave) * FI * FJ * 4 * 64 + q * 64 + lane;
-  const size_t slot = (size_t)NW * FI * FJ * 4 * 64;  // float4s per slot
+__device__ __forceinline__ float4 gp_sum_slots(const float4 *__restrict__ p, size_t slot, int S) {
   float4 f[GP_MAX_SPLIT];
 #pragma unroll
-  for (int k = 0; k < GP_MAX_SPLIT; ++k) f[k] = pw[(k < S ? k : S - 1) * slot];
+  for (int k = 0; k < GP_MAX_SPLIT; ++k) f[k] = p[(k < S ? k : S - 1) * slot];
   float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
   for (int k = 0; k < GP_MAX_SPLIT; ++k)
     if (k < S) s.x += f[k].x, s.y += f[k].y, s.z += f[k].z, s.w += f[k].w;
-  const float v[4] = {s.x, s.y, s.z, s.w};
+  return s;
+}
+
+// The reduce of a kernel of geometry G (tiles of TM x TN, WM x WN waves of 32 FI x 32 FJ), one
+// thread per float4 of the partial layout that is stored, thread i of the call: the tiles
+// whole_tiles on, in gp_tile_at's order.  A float4 is four rows of one column; it is rounded to
+// bf16 as the tile epilogue rounds (rows from M on and columns from N on are not stored).
+// MLP: column blocks
+// 2 j and 2 j + 1 of a wave are gate and up of the same 32 columns, and silu(gate) * up is
+// stored, TN / 2 columns per tile.
+template <class G, bool MLP = false>
+__device__ __forceinline__ void gp_reduce_tile(const float *__restrict__ part, const YOut yo, int M, int N,
+                                               int whole_tiles, int S, int i) {
+  constexpr int OJ = MLP ? G::FJ / 2 : G::FJ, NQ = G::FI * OJ * 4, TILE = G::NW * NQ * 64;
+  static_assert(TILE % 256 == 0, "whole blocks per tile");
+  const int t = i / TILE, rem = i - t * TILE;
+  const int wave = rem / (NQ * 64), q = (rem >> 6) % NQ, lane = rem & 63;
+  int tm, tn;
+  gp_tile_at(whole_tiles + t, (M + G::TM - 1) / G::TM, (N + 32 * OJ * G::WN - 1) / (32 * OJ * G::WN), &tm, &tn);
+  const int row0 = tm * G::TM + (wave % G::WM) * 32 * G::FI, col0 = (tn * G::WN + wave / G::WM) * 32 * OJ;
+  const int fi = q / (OJ * 4), j = (q / 4) % OJ, v4 = q % 4;
+  const int r = row0 + 32 * fi + 8 * v4 + 4 * (lane >> 5), c = col0 + 32 * j + (lane & 31);
+  if (r >= M || c >= N) return;  // not stored by the split blocks either (rows past M)
+  const size_t slot = (size_t)G::NW * G::FI * G::FJ * 4 * 64;  // float4s per slot
+  const float4 *p = (const float4 *)part + (size_t)t * S * slot +
+                    ((size_t)(wave * G::FI + fi) * G::FJ + (MLP ? 2 * j : j)) * 4 * 64 + v4 * 64 + lane;
+  const float4 a = gp_sum_slots(p, slot, S);
+  float v[4] = {a.x, a.y, a.z, a.w};
+  if constexpr (MLP) {
+    const float4 u = gp_sum_slots(p + 4 * 64, slot, S);
+    v[0] = silu_mul_bf16(v[0], u.x), v[1] = silu_mul_bf16(v[1], u.y);
+    v[2] = silu_mul_bf16(v[2], u.z), v[3] = silu_mul_bf16(v[3], u.w);
+  }
 #pragma unroll
   for (int e = 0; e < 4; ++e)
     if (r + e < M) *yo.at(r + e, c) = __builtin_bit_cast(uint16_t, (__bf16)v[e]);
 }
 
-// The same for a kernel of geometry G (tiles of TM x TN, WM x WN waves of 32 FI x 32 FJ),
-// thread i of the call: the tiles whole_tiles on, in gp_tile_at's order.
-template <class G>
-__device__ __forceinline__ void gp_reduce_tile(const float *__restrict__ part, const YOut yo, int M, int N,
-                                               int whole_tiles, int S, int i) {
-  constexpr int NQ = G::FI * G::FJ * 4, TILE = G::NW * NQ * 64;
-  static_assert(TILE % 256 == 0, "whole blocks per tile");
-  const int t = i / TILE, rem = i - t * TILE;
-  const int wave = rem / (NQ * 64), q = (rem >> 6) % NQ, lane = rem & 63;
-  int tm, tn;
-  gp_tile_at(whole_tiles + t, (M + G::TM - 1) / G::TM, (N + G::TN - 1) / G::TN, &tm, &tn);
-  gp_reduce_quad<G::FI, G::FJ, G::NW>(part, yo, M, N, t, S, wave, q, lane, tm * G::TM + (wave % G::WM) * 32 * G::FI,
-                                      tn * G::TN + (wave / G::WM) * 32 * G::FJ);
+// silu(gate) * up of a wave's accumulators, column blocks 2 j gate and 2 j + 1 up.
+template <int FI, int FJ>
+__device__ __forceinline__ void gp_silu_mul(const f32x16_t (&acc)[FI][FJ], f32x16_t (&h)[FI][FJ / 2]) {
+#pragma unroll
+  for (int i = 0; i < FI; ++i)
+#pragma unroll
+    for (int j = 0; j < FJ / 2; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) h[i][j][v] = silu_mul_bf16(acc[i][2 * j][v], acc[i][2 * j + 1][v]);
 }
 
 // gp_store_tile_bf16 of all FI accumulator rows, one at a time.
@@ -298,26 +291,33 @@ struct GpPlan {
 };
 // The least estimated time over every tile size and every split of the tiles left after the
 // whole rounds (at most GP_MAX_SPLIT ways, one round of blocks, at least 4 K steps each, in
-// units of `unit` steps).  A split adds the reduce: its launch and its partial sums' traffic.
-inline GpPlan gp_plan(const GpCost *costs, int n, int M, int N, int steps, int unit, int cus) {
+// units of `unit` steps).  Where several blocks share a CU, the last round may instead give
+// every CU `more` whole tiles and the split ones run beside them.  A split adds the reduce: its
+// launch and its partial sums' traffic.
+inline GpPlan gp_plan(const GpCost *costs, int n, int M, int64_t N, int steps, int unit, int cus) {
   if (cus <= 0) cus = 256;  // (no device answers: the launch reports it)
   GpPlan best{0, 0, 0, 1};
   float best_us = 1e30f;
+  const int units = (steps + unit - 1) / unit;
   for (int c = 0; c < n; ++c) {
     const GpCost &d = costs[c];
     const int64_t T = (int64_t)((M + d.TM - 1) / d.TM) * ((N + d.TN - 1) / d.TN);
-    const int64_t slots = (int64_t)cus * d.per_cu, whole = T / slots * slots, left = T - whole;
-    const float base = (float)(whole / slots) * ((float)steps * d.step[d.per_cu - 1] + d.round);
-    const int units = (steps + unit - 1) / unit;
-    for (int S = 1; S <= GP_MAX_SPLIT; ++S) {
-      if (S > 1 && (left == 0 || left * S > slots || units < S || steps < 4 * S)) break;
-      float us = base;
-      if (left) {
-        const int per = (int)((left * S + cus - 1) / cus), mine = (units + S - 1) / S * unit;
-        us += (float)(mine < steps ? mine : steps) * d.step[(per < d.per_cu ? per : d.per_cu) - 1] + d.round;
+    const int64_t slots = (int64_t)cus * d.per_cu, rounds = T / slots;
+    for (int more = 0; more < d.per_cu; ++more) {
+      const int64_t whole = rounds * slots + (int64_t)more * cus, left = T - whole;
+      if (left < 0) break;
+      for (int S = 1; S <= GP_MAX_SPLIT; ++S) {
+        if (S > 1 && (left == 0 || left * S > slots - (int64_t)more * cus || units < S || steps < 4 * S)) break;
+        if (more && left && S == 1) continue;  // (the same blocks as more = 0)
+        const int mine = (units + S - 1) / S * unit, split_steps = mine < steps ? mine : steps;
+        int per = more + (int)((left * S + cus - 1) / cus);  // blocks on a CU in the last round
+        if (per > d.per_cu) per = d.per_cu;
+        float us = (float)rounds * ((float)steps * d.step[d.per_cu - 1] + d.round);
+        if (more) us += (float)(steps - split_steps) * d.step[more - 1];
+        if (per) us += (float)split_steps * d.step[per - 1] + d.round;
+        if (S > 1) us += 1.5f + (float)left * S * (M < d.TM ? M : d.TM) * d.TN * 8.f / 6.6e6f;
+        if (us < best_us) best_us = us, best = GpPlan{c, (int)whole, (int)left, S};
       }
-      if (S > 1) us += 1.5f + (float)left * S * (M < d.TM ? M : d.TM) * d.TN * 8.f / 6.6e6f;
-      if (us < best_us) best_us = us, best = GpPlan{c, (int)whole, (int)left, S};
     }
   }
   if (best.S == 1) best.whole += best.left, best.left = 0;

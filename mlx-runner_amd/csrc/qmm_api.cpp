@@ -571,12 +571,8 @@ static int tiled_scales(Arr *sa, const QmmArgs &a, hipStream_t st, const uint32_
 }
 
 // Whether a grouped call's stacked matrices can run as one prefill GEMM: the pipelined
-// kernels (mxfp8: K % 128, scales 4-byte aligned), whose epilogues store to parts.
-static bool gemm_parts_ok(const QmmArgs &a) {
-  if (a.x_f32 || (((uintptr_t)a.x | (uintptr_t)a.w) & 15) != 0) return false;
-  if (a.mode == MXFP8) return gemm_mxfp8_ok(a) && a.K % 128 == 0 && ((uintptr_t)a.s & 3) == 0;
-  return gemm_nvfp4_ok(a);
-}
+// kernels, whose epilogues store to parts.
+static bool gemm_parts_ok(const QmmArgs &a) { return gemm_mxfp8_ok(a) || gemm_nvfp4_ok(a); }
 
 // Workspace bytes run_qmm needs for these arguments (0 for the decode kernels).
 static size_t qmm_workspace(const QmmArgs &a) {
@@ -976,14 +972,27 @@ int qmm_mlp_gate_up_silu(qmm_array *res, qmm_array x, qmm_array w_gate, qmm_arra
     if (e != hipSuccess) return finish(fail_hip(e, op));
     return finish(0);
   }
-  // prefill shapes: the two projections, then the activation; the gate and up results
-  // and the projections' own workspace in the stream's workspace
-  const size_t bytes = (ha->nbytes() + 255) & ~(size_t)255;
   QmmArgs b = a;
   b.w = wu;
   b.s = su;
   if (tiled_scales((Arr *)s_gate.ctx, a, st, &a.s_tiled) || tiled_scales((Arr *)s_up.ctx, b, st, &b.s_tiled))
     return finish(1);
+  // prefill shapes of the pipelined GEMMs: both projections and the activation in one
+  // (rounded as three calls would; the fp32 sums of a tile split along K can differ from
+  // those of the projections alone, whose splits are their own)
+  if (K > 0 && !qmm_on_decode(a)) {
+    QmmArgs f = a;
+    f.w_up = wu;
+    f.s_up = su;
+    f.s_up_tiled = b.s_tiled;
+    if (gemm_mxfp8_ok(f) || gemm_nvfp4_ok(f)) {
+      if (run_qmm(f, ha->nbytes(), st, op)) return finish(1);
+      return finish(0);
+    }
+  }
+  // others: the two projections, then the activation; the gate and up results
+  // and the projections' own workspace in the stream's workspace
+  const size_t bytes = (ha->nbytes() + 255) & ~(size_t)255;
   const size_t gemm_ws = std::max(qmm_workspace(a), qmm_workspace(b));
   void *ws = nullptr;
   bool transient = false;
@@ -991,11 +1000,6 @@ int qmm_mlp_gate_up_silu(qmm_array *res, qmm_array x, qmm_array w_gate, qmm_arra
   void *g = ws, *u = (char *)ws + bytes, *gws = gemm_ws ? (char *)ws + 2 * bytes : nullptr;
   a.y = g;
   b.y = u;
-  // mxfp8: the up projection reuses the x split the gate projection made in the shared
-  // workspace (same x, M, K and split layout; the two launches are stream-ordered)
-  const bool aligned_x = (((uintptr_t)a.x | (uintptr_t)a.w | (uintptr_t)b.w) & 15) == 0;
-  b.x_split_ready = gws && aligned_x && gemm_mxfp8_ok(a) && gemm_mxfp8_ok(b) &&
-                    gemm_mxfp8_split_layout_of(a) == gemm_mxfp8_split_layout_of(b);
   int rc = run_qmm(a, bytes, st, op, gws);
   if (!rc) rc = run_qmm(b, bytes, st, op, gws);
   if (!rc) {

@@ -46,10 +46,10 @@ struct QmmArgs {
   // The scales already in the prefill GEMMs' tile-major layout (the repack of
   // launch_repack_scales), or null: the GEMM then repacks them into its workspace.
   const uint32_t *s_tiled = nullptr;
-  // mxfp8 prefill: x is already split into this call's workspace (the previous call on the
-  // stream split the same x with the same M and K into the same workspace, for the same
-  // kernel family: gemm_mxfp8_split_layout_of of both calls agree), so the split is skipped.
-  bool x_split_ready = false;
+  // An MLP's prefill: the up projection's weights and scales beside the gate's (w, s); the GEMM
+  // then computes silu(gate) * up into y.  Null otherwise.
+  const uint8_t *w_up = nullptr, *s_up = nullptr;
+  const uint32_t *s_up_tiled = nullptr;
 };
 
 // The output descriptor of a call: y as one part, or the grouped call's parts.
@@ -94,16 +94,14 @@ hipError_t launch_gemm(const QmmArgs &a, hipStream_t st);
 // mxfp8 prefill on the scaled fp8 MFMA (bf16 x split into E4M3 hi + lo).
 bool gemm_mxfp8_ok(const QmmArgs &a);
 size_t gemm_mxfp8_workspace(const QmmArgs &a);
-// The layout launch_gemm_mxfp8 splits x into (0: row-major, 1: pre-tiled for the pipelined
-// kernel); two calls may share one split only where this agrees.
-int gemm_mxfp8_split_layout_of(const QmmArgs &a);
 hipError_t launch_gemm_mxfp8(const QmmArgs &a, void *workspace, hipStream_t st);
 bool gemm_nvfp4_ok(const QmmArgs &a);
 size_t gemm_nvfp4_workspace(const QmmArgs &a);
 hipError_t launch_gemm_nvfp4(const QmmArgs &a, void *workspace, hipStream_t st);
 
 // The prefill GEMMs' scale layout: for each 256-row tile and each dword d of a row's
-// nb scale bytes, 256 consecutive dwords (one per row).  tiled_scales_bytes(N, nb) bytes.
+// nb scale bytes (zeros past them), 256 consecutive dwords (one per row).
+// tiled_scales_bytes(N, nb) bytes.
 size_t tiled_scales_bytes(int64_t N, int nb);
 hipError_t launch_repack_scales(const uint8_t *s, int64_t N, int nb, uint32_t *out, hipStream_t st);
 // Whether the prefill GEMM for these arguments reads tile-major scales (and how many
@@ -122,8 +120,7 @@ inline bool qmm_on_decode(const QmmArgs &a) {
   // (x of 9-16 rows on the MFMA decode kernels, where they take the shape)
   if (a.M > QMV_MAX_M) return a.M <= 16 && qmv_mfma_ok(a);
   if (a.M <= 4 || a.N < 4096 || qmv_mfma_ok(a) || ((uintptr_t)a.x | (uintptr_t)a.w) & 15) return true;
-  if (a.mode == MXFP8) return !(gemm_mxfp8_ok(a) && a.K % 128 == 0 && ((uintptr_t)a.s & 3) == 0);
-  return !gemm_nvfp4_ok(a);
+  return !gemm_mxfp8_ok(a) && !gemm_nvfp4_ok(a);
 }
 
 // dequant: out [N, K] float32 (out_f32) or bfloat16.

@@ -353,7 +353,7 @@ def gdn_recurrence_noalloc(q: Array, k: Array, v: Array, g: Array, beta: Array, 
 
 def mlp_gate_up_silu(x: Array, w_gate: Array, s_gate: Array, w_up: Array, s_up: Array, mode: str, *,
                      group_size=None, bits=None, out: Array | None = None, stream: Stream | None = None) -> Array:
-    """silu(x @ deq(Wg).T) * (x @ deq(Wu).T) (src/model.zig:905-913), fused for decode shapes."""
+    """silu(x @ deq(Wg).T) * (x @ deq(Wu).T) (src/model.zig:905-913), one launch at decode and prefill shapes."""
     res = out if out is not None else Array()
     s = _stream(stream)
     check(lib.qmm_mlp_gate_up_silu(byref(res.h), x.h, w_gate.h, s_gate.h, w_up.h, s_up.h, opt_int(group_size),

@@ -563,6 +563,28 @@ def test_decode_mfma_other_k_match_oracle(K, mode, M, N, xkind):
     assert np.array_equal(run_qmm(mode, xb, wq, s), y)
 
 
+@pytest.mark.parametrize("mode", ["mxfp8", "nvfp4"])
+@pytest.mark.parametrize("M,N,K", [(17, 33, 96), (64, 65, 224), (130, 129, 288), (200, 1000, 512), (383, 2000, 992),
+                                   (520, 5000, 288), (2049, 8300, 544)])
+def test_mlp_prefill_tiles(mode, M, N, K):
+    """The one-launch prefill MLP at the edges of its tiles and splits: each output within the
+    activation's roundings of the projections' results.  The projections alone may sum in
+    another order, so gate and up may differ by a bf16 rounding (2^-8); through silu and the
+    product that is at most 2^-5 of the value, and 2^-8 of |gate| |up| where silu's slope
+    counts, and nearly all outputs are equal."""
+    rng = np.random.default_rng(M + N + K)
+    wg, sg = rand_w(rng, mode, N, K)
+    wu, su = rand_w(rng, mode, N, K)
+    x = Q.Array.from_numpy(bf16(rng.standard_normal((M, K))), Q.BFLOAT16)
+    A = lambda a, d: Q.Array.from_numpy(a, d)  # noqa: E731
+    gate, up = (A(wg, Q.UINT32), A(sg, Q.UINT8)), (A(wu, Q.UINT32), A(su, Q.UINT8))
+    h = f32(Q.mlp_gate_up_silu(x, *gate, *up, mode).numpy())
+    g, u = Q.quantized_matmul(x, *gate, mode), Q.quantized_matmul(x, *up, mode)
+    h2, gu = f32(Q.silu_mul(g, u).numpy()), np.abs(f32(g.numpy()) * f32(u.numpy()))
+    assert np.all(np.abs(h - h2) <= np.abs(h2) * 2.0 ** -5 + gu * 2.0 ** -8 + 1e-30)
+    assert np.mean(h == h2) > 0.99
+
+
 @pytest.mark.parametrize("mode,M,N", [("nvfp4", 1, 16400), ("nvfp4", 2, 4099), ("nvfp4", 3, 4099),
                                       ("nvfp4", 4, 16400), ("mxfp8", 3, 4101), ("mxfp8", 4, 70001),
                                       ("mxfp8", 6, 4101), ("nvfp4", 5, 4099), ("nvfp4", 1, 17408),
