@@ -18,6 +18,7 @@ struct Arr {
   void *data = nullptr;
   bool owned = false;                   // free the buffer with the handle
   hipStream_t alloc_stream = nullptr;   // stream the buffer was allocated on (stream-ordered free)
+  int device = -1;                      // device current when the handle was made (-1: none)
   int ndim = 0;
   int shape[QMM_MAX_DIM] = {0};
   qmm_dtype dtype = QMM_BOOL;

@@ -136,6 +136,30 @@ def test_convert_ragged_bit_exact(mode, src, N, K):
     assert np.array_equal(d, ref)
 
 
+def test_freed_results_are_reused_in_stream_order():
+    """Results freed on the null stream are handed to its next allocations of their size:
+    live results never share memory, and a reused buffer holds the new result whatever the
+    earlier one still queued."""
+    rng = np.random.default_rng(5)
+    ws = [O.quantize("nvfp4", f32(bf16(rng.standard_normal((n, 512)) * 0.02))) for n in (64, 64, 96, 2048)]
+    refs = [O.dequant_bf16("nvfp4", w, s, 512) for w, s in ws]
+    arrs = [(Q.Array.from_numpy(w, Q.UINT32), Q.Array.from_numpy(s, Q.UINT8)) for w, s in ws]
+    for _ in range(3):
+        live = [Q.dequantize(*a, "nvfp4") for a in arrs]
+        spans = sorted((d.ptr, d.ptr + r.nbytes) for d, r in zip(live, refs))
+        assert all(x[1] <= y[0] for x, y in zip(spans, spans[1:]))
+        first = live[0].ptr
+        live[0].free()
+        again = Q.dequantize(*arrs[1], "nvfp4")  # the size just freed
+        assert again.ptr == first
+        for d, r in zip([again] + live[1:], [refs[1]] + refs[1:]):
+            assert np.array_equal(d.numpy(), r)
+    for n in range(1, 200):  # more sizes than are kept
+        d = Q.dequantize(Q.Array.from_numpy(ws[3][0][:n], Q.UINT32), Q.Array.from_numpy(ws[3][1][:n], Q.UINT8), "nvfp4")
+        if n % 50 == 0:
+            assert np.array_equal(d.numpy(), refs[3][:n])
+
+
 @pytest.mark.parametrize("mode", ["mxfp8", "nvfp4"])
 def test_reference_qmm_case_exact(mode):
     """src/model.zig:1561-1609 restated: integer W, x -> closed-form integer y (tighter than tol 0.05)."""
