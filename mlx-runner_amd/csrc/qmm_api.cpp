@@ -666,6 +666,8 @@ static int run_qmm(QmmArgs &a, size_t ybytes, hipStream_t st, const char *op, vo
   } else if (qmm_on_decode(a)) {
     if (qmv_mfma_ok(a))
       e = launch_qmv_mfma(a, st);
+    else if (qmv_any_ok(a))
+      e = launch_qmv_any(a, st);
     else
       e = (aligned && qmv_fast_ok(a)) ? launch_qmv(a, st) : launch_qmv_generic(a, st);
   } else if (aligned && (gemm_mxfp8_ok(a) || gemm_nvfp4_ok(a))) {
@@ -813,8 +815,10 @@ int qmm_quantized_matmul_group(qmm_array *res, size_t n, qmm_array x, const qmm_
     a.s = s0;
     a.y = nullptr;
     a.parts = &parts;
-    if (qmv_parts_ok(a)) {
-      const hipError_t e = qmv_mfma_ok(a) ? launch_qmv_mfma(a, st) : launch_qmv(a, st);
+    // (x of 5-8 rows whose members qmv_any takes alone would run those; together they are one)
+    const bool any = !qmv_mfma_ok(a) && qmv_any_ok(a);
+    if (any || qmv_parts_ok(a)) {
+      const hipError_t e = any ? launch_qmv_any(a, st) : qmv_mfma_ok(a) ? launch_qmv_mfma(a, st) : launch_qmv(a, st);
       if (e != hipSuccess) return finish(fail_hip(e, op));
       g_group_launches.fetch_add(1, std::memory_order_relaxed);
       return finish(0);
@@ -1032,7 +1036,16 @@ int qmm_mlp_gate_up_silu(qmm_array *res, qmm_array x, qmm_array w_gate, qmm_arra
   // decode shapes: one kernel for both projections and the activation.  Each
   // fused kernel computes the same per-row sums as the kernel run_qmm picks
   // for the shape, so the fused result equals the unfused one.
-  if (K > 0 && qmv_mfma_ok(a)) {
+  QmmArgs fused = a;
+  fused.w_up = wu;
+  fused.s_up = su;
+  if (K > 0 && !qmv_mfma_ok(a) && qmv_any_ok(a)) {
+    if (qmv_any_ok(fused)) {
+      hipError_t e = launch_qmv_any(fused, st);
+      if (e != hipSuccess) return finish(fail_hip(e, op));
+      return finish(0);
+    }
+  } else if (K > 0 && qmv_mfma_ok(a)) {
     if (qmv_mfma_mlp_ok(a, wu, su)) {
       hipError_t e = launch_qmv_mfma_mlp(a, wu, su, st);
       if (e != hipSuccess) return finish(fail_hip(e, op));
@@ -1052,12 +1065,10 @@ int qmm_mlp_gate_up_silu(qmm_array *res, qmm_array x, qmm_array w_gate, qmm_arra
   // (rounded as three calls would; the fp32 sums of a tile split along K can differ from
   // those of the projections alone, whose splits are their own)
   if (K > 0 && !qmm_on_decode(a)) {
-    QmmArgs f = a;
-    f.w_up = wu;
-    f.s_up = su;
-    f.s_up_tiled = b.s_tiled;
-    if (gemm_mxfp8_ok(f) || gemm_nvfp4_ok(f)) {
-      if (run_qmm(f, ha->nbytes(), st, op)) return finish(1);
+    fused.s_tiled = a.s_tiled;
+    fused.s_up_tiled = b.s_tiled;
+    if (gemm_mxfp8_ok(fused) || gemm_nvfp4_ok(fused)) {
+      if (run_qmm(fused, ha->nbytes(), st, op)) return finish(1);
       return finish(0);
     }
   }

@@ -91,6 +91,11 @@ hipError_t launch_silu_mul(const void *g, const void *u, void *h, int64_t n, boo
 bool gemm_ok(const QmmArgs &a);
 hipError_t launch_gemm(const QmmArgs &a, hipStream_t st);
 
+// nvfp4 decode matmul (x of 3-8 rows; also grouped, and an MLP: w_up) at any K % 128 = 0, where
+// qmv_mfma_ok does not take it.
+bool qmv_any_ok(const QmmArgs &a);
+hipError_t launch_qmv_any(const QmmArgs &a, hipStream_t st);
+
 // mxfp8 prefill on the scaled fp8 MFMA (bf16 x split into E4M3 hi + lo).
 bool gemm_mxfp8_ok(const QmmArgs &a);
 size_t gemm_mxfp8_workspace(const QmmArgs &a);
@@ -119,7 +124,7 @@ int gemm_tiled_scale_bytes_per_row(const QmmArgs &a);
 inline bool qmm_on_decode(const QmmArgs &a) {
   // (x of 9-16 rows on the MFMA decode kernels, where they take the shape)
   if (a.M > QMV_MAX_M) return a.M <= 16 && qmv_mfma_ok(a);
-  if (a.M <= 4 || a.N < 4096 || qmv_mfma_ok(a) || ((uintptr_t)a.x | (uintptr_t)a.w) & 15) return true;
+  if (a.M <= 4 || a.N < 4096 || qmv_mfma_ok(a) || qmv_any_ok(a) || ((uintptr_t)a.x | (uintptr_t)a.w) & 15) return true;
   return !gemm_mxfp8_ok(a) && !gemm_nvfp4_ok(a);
 }
 

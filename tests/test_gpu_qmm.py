@@ -587,6 +587,32 @@ def test_decode_mfma_other_k_match_oracle(K, mode, M, N, xkind):
     assert np.array_equal(run_qmm(mode, xb, wq, s), y)
 
 
+@pytest.mark.parametrize("M,N,K", [(3, 5120, 128), (4, 5121, 1152), (5, 4096, 4096), (6, 4111, 3968), (8, 16384, 384),
+                                   (3, 8200, 2944), (4, 4097, 4224), (3, 4100, 12288), (4, 20000, 8320)])
+def test_qmv_any_k(M, N, K):
+    """x of 3-8 rows at row lengths of any multiple of 128: whole and half last slices, one and
+    several passes, ranges that end in partial row blocks; plain, grouped and as an MLP.  A
+    row's sums do not depend on the call, so grouped and fused results equal the plain ones."""
+    rng = np.random.default_rng(M + N + K)
+    wq, s = rand_packed(rng, "nvfp4", N, K)
+    xb = make_x(rng, M, K, "edge")
+    y = run_qmm("nvfp4", xb, wq, s)
+    cols = np.unique(np.concatenate([np.arange(0, N, 37), np.arange(N - 20, N)]))
+    ok, fro, worst = O.check_tolerance(f32(y[:, cols]), f32(O.qmm("nvfp4", xb, wq, s, cols=cols)), **TOL)
+    assert ok, (fro, worst)
+    x, A = Q.Array.from_numpy(xb, Q.BFLOAT16), Q.Array.from_numpy
+    wu, su = rand_packed(rng, "nvfp4", N, K)
+    gate, up = (A(wq, Q.UINT32), A(s, Q.UINT8)), (A(wu, Q.UINT32), A(su, Q.UINT8))
+    h = Q.mlp_gate_up_silu(x, *gate, *up, "nvfp4").numpy()
+    g, u = Q.quantized_matmul(x, *gate, "nvfp4"), Q.quantized_matmul(x, *up, "nvfp4")
+    assert np.array_equal(h, Q.silu_mul(g, u).numpy())
+    tw, ts = torch.tensor(wq.view(np.int32)).cuda(), torch.tensor(s).cuda()
+    n0 = N - 1000
+    outs = Q.quantized_matmul_group(x, [Q.Array.from_torch(tw[:n0]), Q.Array.from_torch(tw[n0:])],
+                                    [Q.Array.from_torch(ts[:n0]), Q.Array.from_torch(ts[n0:])], "nvfp4")
+    assert np.array_equal(np.concatenate([o.numpy() for o in outs], 1), y)
+
+
 @pytest.mark.parametrize("mode", ["mxfp8", "nvfp4"])
 @pytest.mark.parametrize("M,N,K", [(17, 33, 96), (64, 65, 224), (130, 129, 288), (200, 1000, 512), (383, 2000, 992),
                                    (520, 5000, 288), (2049, 8300, 544)])
