@@ -1,6 +1,6 @@
 // Dense bf16 linear y[M, N] = x[M, K] @ w[N, K].T (linear, src/model.zig:200-211): bf16
-// operands, fp32 accumulation, bf16 out (RNE).  x of at most 8 rows runs a GEMV
-// (gemv_bf16_kernel), taller x a pipelined GEMM on v_mfma_f32_32x32x16_bf16.
+// operands, fp32 accumulation, bf16 out (RNE).  x of a few rows runs a GEMV
+// (gemv_bf16_kernel; linear_gemv), taller x a pipelined GEMM on v_mfma_f32_32x32x16_bf16.
 //
 // The GEMM.  What bounds it: at tall x the matrix cores at the clock the power limit leaves
 // (a large library product reaches ~1.45 PFLOP/s here, not 2.5), and before that the time a
@@ -31,14 +31,20 @@
 
 namespace qmm {
 
-// ---------------------------------------------------------------- x of at most 8 rows
+// ---------------------------------------------------------------- x of a few rows
 
-// One wave per 4 W rows, lanes over 16-byte (8-element) chunks.
-template <int M>
-__global__ __launch_bounds__(64) void gemv_bf16_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w,
-                                                       uint16_t *__restrict__ y, int N, int K) {
+// A workgroup of W waves per 4 W rows, its lanes over 16-byte (8-element) chunks of them, U chunks
+// in flight per lane; the waves' sums are added in wave order.  Bound by the weight stream, so by
+// the bytes in flight: with one wave per 4 rows and one chunk each, a CU had 20 KiB of 5120 rows
+// in flight, and short matrices left most CUs without a wave (us,
+// before and now: 5120 x 17408 at 2 rows 30.6 -> 28.9, 1024 x 5120 at 1 row 7.1 -> 3.9, 703 x
+// 6912 at 4 rows 11.4 -> 6.3).
+template <int M, int W, int U>
+__global__ __launch_bounds__(64 * W) void gemv_bf16_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w,
+                                                           uint16_t *__restrict__ y, int N, int K) {
   constexpr int R = 4;
-  const int lane = threadIdx.x;
+  __shared__ float part[W][R * M];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int n0 = blockIdx.x * R;
   const int C = K >> 3;
   float acc[R][M];
@@ -46,39 +52,82 @@ __global__ __launch_bounds__(64) void gemv_bf16_kernel(const uint16_t *__restric
   for (int r = 0; r < R; ++r)
 #pragma unroll
     for (int m = 0; m < M; ++m) acc[r][m] = 0.f;
-  for (int c = lane; c < C; c += 64) {
-    uint4 q[R];
+  // chunk c + 64 W u of the rows, u < U
+  auto chunks = [&](auto u_c, int c) __attribute__((always_inline)) {
+    constexpr int UU = decltype(u_c)::value;
+    uint4 q[UU][R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int n = n0 + r < N ? n0 + r : N - 1;
-      q[r] = load_stream16((const uint4 *)(w + (int64_t)n * K) + c);
-    }
-#pragma unroll
-    for (int m = 0; m < M; ++m) {
-      const uint4 xv = ((const uint4 *)(x + (int64_t)m * K))[c];
+    for (int u = 0; u < UU; ++u)
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        float t = acc[r][m];
-        t = dot2_bf16(__builtin_bit_cast(bf16x2_t, q[r].x), xv.x, t);
-        t = dot2_bf16(__builtin_bit_cast(bf16x2_t, q[r].y), xv.y, t);
-        t = dot2_bf16(__builtin_bit_cast(bf16x2_t, q[r].z), xv.z, t);
-        t = dot2_bf16(__builtin_bit_cast(bf16x2_t, q[r].w), xv.w, t);
-        acc[r][m] = t;
+        const int n = n0 + r < N ? n0 + r : N - 1;
+        q[u][r] = load_stream16((const uint4 *)(w + (int64_t)n * K) + c + 64 * W * u);
       }
-    }
-  }
+#pragma unroll
+    for (int u = 0; u < UU; ++u)
+#pragma unroll
+      for (int m = 0; m < M; ++m) {
+        const uint4 xv = ((const uint4 *)(x + (int64_t)m * K))[c + 64 * W * u];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          float t = acc[r][m];
+          t = dot2_bf16(__builtin_bit_cast(bf16x2_t, q[u][r].x), xv.x, t);
+          t = dot2_bf16(__builtin_bit_cast(bf16x2_t, q[u][r].y), xv.y, t);
+          t = dot2_bf16(__builtin_bit_cast(bf16x2_t, q[u][r].z), xv.z, t);
+          t = dot2_bf16(__builtin_bit_cast(bf16x2_t, q[u][r].w), xv.w, t);
+          acc[r][m] = t;
+        }
+      }
+  };
+  int c = tid;
+  if constexpr (U > 1)
+    for (; c + 64 * W * (U - 1) < C; c += 64 * W * U) chunks(std::integral_constant<int, U>{}, c);
+  for (; c < C; c += 64 * W) chunks(std::integral_constant<int, 1>{}, c);
   float out = 0.f;
 #pragma unroll
   for (int r = 0; r < R; ++r)
 #pragma unroll
     for (int m = 0; m < M; ++m) {
-      float t = wave_sum(acc[r][m]);
+      const float t = wave_sum(acc[r][m]);
       out = (lane == r * M + m) ? t : out;
     }
+  if constexpr (W > 1) {
+    if (lane < R * M) part[wave][lane] = out;
+    __syncthreads();
+    if (wave) return;
+    out = 0.f;
+    if (lane < R * M) {
+#pragma unroll
+      for (int v = 0; v < W; ++v) out += part[v][lane];
+    }
+  }
   if (lane < R * M) {
     const int r = lane / M, m = lane % M;
     if (n0 + r < N) y[(int64_t)m * N + n0 + r] = f32_to_bf16_rne(out);
   }
+}
+
+template <int M>
+static void launch_gemv(const uint16_t *x, const uint16_t *w, uint16_t *y, int N, int K, hipStream_t st) {
+  // Several waves per row group where the groups alone give a CU under 6 waves and every lane
+  // still has a chunk; from there on one wave and one chunk each (at 12288 x 5120 four waves and
+  // two chunks measured 22.4 -> 23.9 us at 4 rows, 300 x 1024 eight waves 4.0 -> 5.2).
+  const int groups = (N + 3) / 4, cus = device_cu_count(), chunks = K >> 3;
+  const dim3 grid(groups);
+  if (groups < 2 * cus && chunks >= 512) hipLaunchKernelGGL((gemv_bf16_kernel<M, 8, 2>), grid, dim3(512), 0, st, x, w, y, N, K);
+  else if (groups < 6 * cus && chunks >= (M <= 4 ? 256 : 512)) hipLaunchKernelGGL((gemv_bf16_kernel<M, 4, 2>), grid, dim3(256), 0, st, x, w, y, N, K);
+  else if (groups < 4 * cus && chunks >= 128) hipLaunchKernelGGL((gemv_bf16_kernel<M, 2, 1>), grid, dim3(128), 0, st, x, w, y, N, K);
+  else hipLaunchKernelGGL((gemv_bf16_kernel<M, 1, 1>), grid, dim3(64), 0, st, x, w, y, N, K);
+}
+
+// x of up to 5 rows runs the GEMV, and up to 8 rows on matrices whose row groups are fewer than
+// two per CU: its work grows with every row, the GEMM's does not (us at 6 rows, GEMV / GEMM:
+// 10240 x 5120 28 / 21, 5120 x 6144 20 / 16, 2000 x 4096 10.9 / 8.9; 1024 x 5120 7.3 / 8.4; at 5
+// rows 10240 x 5120 23.5 / 21.4, 4000 x 2560 8.2 / 9.9), unless K is short too (2288 x 1216 7.2 /
+// 8.1).
+static bool linear_gemv(int M, int N, int K) {
+  const int groups = (N + 3) / 4, cus = device_cu_count();
+  return M <= 5 || (M <= QMV_MAX_M && (groups < 2 * cus || (groups < 4 * cus && K < 2048)));
 }
 
 // ---------------------------------------------------------------- taller x
@@ -305,7 +354,7 @@ static hipError_t launch_dense_plan(const uint16_t *x, const uint16_t *w, uint16
 }
 
 size_t linear_bf16_workspace(int M, int N, int K) {
-  if (M <= QMV_MAX_M) return 0;
+  if (linear_gemv(M, N, K)) return 0;
   const GpPlan p = dense_plan(M, N, K);
   return (size_t)p.left * p.S * DN_COST[p.cfg].TM * DN_COST[p.cfg].TN * sizeof(float);
 }
@@ -313,11 +362,10 @@ size_t linear_bf16_workspace(int M, int N, int K) {
 hipError_t launch_linear_bf16(const uint16_t *x, const uint16_t *w, uint16_t *y, int M, int N, int K, void *ws,
                               hipStream_t st) {
   if (K % 16 != 0 || M <= 0 || N <= 0) return hipErrorInvalidValue;
-  if (M > QMV_MAX_M) return launch_dense_plan(x, w, y, M, N, K, dense_plan(M, N, K), (float *)ws, st);
-  dim3 grid((N + 3) / 4);
+  if (!linear_gemv(M, N, K)) return launch_dense_plan(x, w, y, M, N, K, dense_plan(M, N, K), (float *)ws, st);
   switch (M) {
 #define QMM_GEMV_CASE(MM) \
-  case MM: hipLaunchKernelGGL((gemv_bf16_kernel<MM>), grid, dim3(64), 0, st, x, w, y, N, K); break;
+  case MM: launch_gemv<MM>(x, w, y, N, K, st); break;
     QMM_GEMV_CASE(1) QMM_GEMV_CASE(2) QMM_GEMV_CASE(3) QMM_GEMV_CASE(4)
     QMM_GEMV_CASE(5) QMM_GEMV_CASE(6) QMM_GEMV_CASE(7) QMM_GEMV_CASE(8)
 #undef QMM_GEMV_CASE

@@ -367,13 +367,15 @@ def test_dense_linear_matches_fp32_reference(M):
 
 
 @pytest.mark.parametrize("M,N,K", [
+    (1, 3, 16), (2, 2049, 1040), (5, 700, 4112), (8, 2047, 2064), (3, 4100, 2064), (4, 6146, 4096),  # the GEMV's forms
+    (6, 2048, 1040), (8, 5000, 528),                              # a few rows on the GEMM
     (9, 1, 16), (10, 65, 48), (64, 63, 64), (65, 129, 1040),      # one partial tile, K ends inside a step
     (33, 1000, 1040), (129, 273, 3328), (548, 256, 3584),         # tiles split along K
     (1030, 492, 2848), (700, 2500, 1296),                         # 128-row tiles, whole and left over
     (1000, 10240, 272), (1000, 10239, 288), (1300, 16400, 528),   # 256-row tiles: one round, and tiles left over
 ])
 def test_dense_linear_tiles(M, N, K):
-    """The dense GEMM at the edges of its tiles, K steps and splits, against float64 on the
+    """The dense GEMV and GEMM at the edges of their tiles, K steps and splits, against float64 on the
     GPU: within the one bf16 rounding (2^-8 of the value) and the fp32 sums' error, which is
     below 2^-24 K of sum |x| |w|."""
     gen = torch.Generator(device="cuda")
