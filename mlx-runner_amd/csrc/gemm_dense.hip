@@ -314,6 +314,9 @@ using DnH = DnGeom<4, 2, 2, 2, 2, 4>;     // 256 x 128
 using Dn128 = DnGeom<2, 2, 2, 2, 2, 3>;   // 128 x 128, two blocks per CU
 using Dn64 = DnGeom<2, 1, 1, 4, 2, 4>;    // 64 x 128, two blocks per CU
 using DnS = DnGeom<1, 1, 2, 2, 2, 4>;     // 64 x 64, three blocks per CU
+// Measured on calls of whole rounds and of one block per CU, weights cold: on 39 shapes the plan's
+// choice takes 1.05 times the best configuration's time on average, at most 1.35 (1000 x 10240 x
+// 5120: 256 x 160 tiles fill one round of 256 CUs, 95 us; 256 x 256 ones, 160 of them, 99).
 constexpr GpCost DN_COST[] = {{256, 256, 1, 3.f, {1.24f}},         {256, 160, 1, 3.f, {1.10f}},
                               {192, 256, 1, 3.f, {1.20f}},         {256, 128, 1, 3.f, {0.91f}},
                               {128, 128, 2, 3.f, {0.64f, 0.90f}},  {64, 128, 2, 3.f, {0.56f, 0.74f}},

@@ -14,8 +14,8 @@
 // the weight tile is loaded once, the MFMA work doubles.
 //
 // What bounds it: at tall x the matrix cores at the clock the power limit leaves (a large
-// fp8 library product reaches ~3.07 PFLOP/s here; 2048 x 34816 x 5120 runs at 2.93, hi and lo
-// both counted), at short x the latency of a step.  So:
+// fp8 library product reaches ~3.07 PFLOP/s here; 2048 x 34816 x 5120 runs at 2.8-2.9, hi and
+// lo both counted), at short x the latency of a step.  So:
 //   * K steps of 64: a row's hi and lo bytes of a step lie together, 128 bytes, a cache line;
 //     W moves in stages of two steps, 128 bytes per row too (64 wasted half of each line).
 //   * x and W go to LDS rings by DMA; the lo fragments are read beside the products of the
@@ -24,8 +24,8 @@
 //     split along K over the idle CUs, fp32 partial sums reduced in K order (deterministic) by
 //     a second kernel.
 // Measured, us per call with the split, weights cold (M x N x K; the former kernel, two groups
-// of waves in turns, two barriers per step, in brackets): 2048 x 5120 x 17408  272 (322),
-// 2048 x 17408 x 5120  269 (282), 200 x 5120 x 17408  54 (61), 48 x 17408 x 5120  35 (46),
+// of waves in turns, two barriers per step, in brackets): 2048 x 5120 x 17408  272-287 (320),
+// 2048 x 17408 x 5120  269 (282), 200 x 5120 x 17408  54 (61), 48 x 17408 x 5120  28-35 (37-46),
 // 385 x 4129 x 1280  20 (32); K % 128 != 0, which ran unpipelined kernels: 68 x 27408 x 3392
 // 41 (199), 147 x 2181 x 8672  25 (325).
 // gate, up and silu(gate) * up of an MLP in one launch (MLP below), 2048 x (2 x 17408) x 5120:

@@ -21,8 +21,8 @@
 //     (deterministic) by a second kernel.
 // Measured, us per call, weights cold (M x N x K; the former kernel, two groups of waves in
 // turns with W moved 32 bytes per row and step, in brackets): 2048 x 16480 x 5120  271 (318,
-// 1.28 PFLOP/s now), 500 x 10240 x 5120  57 (63), 48 x 17408 x 5120  26 (30), 200 x 6144 x
-// 5120  26 (32).  256 x 256 tiles in 8 waves of 128 x 64, which dequantize every element
+// 1.28 PFLOP/s now), 2048 x 34816 x 5120  544 (567), 500 x 10240 x 5120  57 (63), 48 x 17408 x
+// 5120  23-26 (26-30), 200 x 6144 x 5120  26-31 (32).  256 x 256 tiles in 8 waves of 128 x 64, which dequantize every element
 // twice: 276 in the first.  K that is not a multiple of 64, which ran gemm.hip's kernel:
 // 33 x 1000 x 1056 28 -> 9.4.
 #include <type_traits>
@@ -349,7 +349,7 @@ using NvW = NvGeom<4, 2, 1, 4, 2>;    // 128 x 256
 using Nv128 = NvGeom<4, 1, 1, 4, 2>;  // 128 x 128, two blocks per CU
 using Nv64 = NvGeom<2, 1, 1, 4, 4>;   // 64 x 128, two blocks per CU
 using Nv32 = NvGeom<1, 1, 1, 4, 4>;   // 32 x 128, three blocks per CU
-// (fitted to 45 shapes of the declared range with every tile and split, rms error 7%; the
+// (fitted to 45 shapes with every tile and split, rms error 7%; the
 // plan's choice is 1.01 of the best of them on average, at most 1.26)
 constexpr GpCost NV_COST[] = {{256, 256, 1, 9.7f, {1.10f}},         {192, 256, 1, 8.9f, {0.86f}},
                               {128, 256, 1, 9.7f, {0.58f}},         {128, 128, 2, 7.8f, {0.42f, 0.69f}},

@@ -1,6 +1,6 @@
-// Pieces shared by the pipelined prefill GEMMs (mxfp8 on the scaled fp8 MFMA,
-// nvfp4 on the bf16 MFMA): tile order, LDS DMA, barrier/wait helpers and the
-// weight-scale repack.
+// Pieces shared by the pipelined GEMMs (mxfp8 on the scaled fp8 MFMA, nvfp4 and
+// dense bf16 on the bf16 MFMA): tile order, LDS DMA, barrier/wait helpers, the
+// epilogues, the split tiles' reduce, the weight-scale repack and the plan.
 #pragma once
 
 #include "qmm_device.h"

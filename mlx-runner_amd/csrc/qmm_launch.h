@@ -78,7 +78,7 @@ bool qmv_mfma_parts_ok(const QmmArgs &a);
 bool qmv_fast_ok(const QmmArgs &a);
 hipError_t launch_qmv(const QmmArgs &a, hipStream_t st);
 hipError_t launch_qmv_generic(const QmmArgs &a, hipStream_t st);
-// Decode GEMV on the scaled MFMA (K = 5120; nvfp4 M <= 2, mxfp8 M <= 4, bf16 x).
+// Decode matmul on the MFMA (bf16 x of up to 16 rows; K = 5120, 6144, 10240, 17408).
 bool qmv_mfma_ok(const QmmArgs &a);
 hipError_t launch_qmv_mfma(const QmmArgs &a, hipStream_t st);
 bool qmv_mfma_mlp_ok(const QmmArgs &a, const uint8_t *w_up, const uint8_t *s_up);
@@ -87,7 +87,7 @@ bool qmv_mlp_ok(const QmmArgs &a);
 hipError_t launch_qmv_mlp(const QmmArgs &a, const uint8_t *w_up, const uint8_t *s_up, hipStream_t st);
 hipError_t launch_silu_mul(const void *g, const void *u, void *h, int64_t n, bool f32, hipStream_t st);
 
-// Prefill GEMM (M > QMV_MAX_M, and 5-8 rows the decode MFMA kernels do not take: qmm_on_decode).
+// nvfp4 prefill at K % 32 = 16, which the pipelined GEMM below does not take.
 bool gemm_ok(const QmmArgs &a);
 hipError_t launch_gemm(const QmmArgs &a, hipStream_t st);
 
@@ -116,11 +116,10 @@ int gemm_tiled_scale_bytes_per_row(const QmmArgs &a);
 // Whether a call runs on the decode kernels (x of at most QMV_MAX_M rows, and x of up to
 // 16 rows where the MFMA decode kernels take it: mxfp8 on the scaled MFMA, nvfp4 at
 // K = 5120 / 6144 from 5 rows on the dequantizing bf16-MFMA kernel) rather than a prefill GEMM.  x of
-// 5-8 rows that the MFMA decode kernels do not take (nvfp4 at K = 10240 / 17408; mxfp8 at
-// K = 17408 from 6 rows) runs on the pipelined GEMM's split tiles when the matrix is tall:
-// the other decode kernel is the unpacking GEMV, whose work grows with every row
-// (N = 17408, K = 5120, nvfp4: 40-62 us at 5-8 rows against 25 us; N = 5120, K = 17408,
-// mxfp8: 50-61 us against 47 us).
+// 5-8 rows that no MFMA decode kernel takes (mxfp8 at K = 17408 from 6 rows and at other K;
+// nvfp4 where qmv_any_ok says no) runs on the pipelined GEMM's split tiles when the matrix is
+// tall: the other decode kernel is the unpacking GEMV, whose work grows with every row
+// (N = 5120, K = 17408, mxfp8: 50-61 us at 6-8 rows; the GEMM 23 us).
 inline bool qmm_on_decode(const QmmArgs &a) {
   // (x of 9-16 rows on the MFMA decode kernels, where they take the shape)
   if (a.M > QMV_MAX_M) return a.M <= 16 && qmv_mfma_ok(a);
