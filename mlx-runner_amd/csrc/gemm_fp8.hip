@@ -26,8 +26,8 @@
 // Measured, us per call with the split, weights cold (M x N x K; the former kernel, two groups
 // of waves in turns, two barriers per step, in brackets): 2048 x 5120 x 17408  272-287 (320),
 // 2048 x 17408 x 5120  269 (282), 200 x 5120 x 17408  54 (61), 48 x 17408 x 5120  28-35 (37-46),
-// 385 x 4129 x 1280  20 (32); K % 128 != 0, which ran unpipelined kernels: 68 x 27408 x 3392
-// 41 (199), 147 x 2181 x 8672  25 (325).
+// 385 x 4129 x 1280  20 (32); K % 128 = 64, which ran an unpipelined kernel: 68 x 27408 x 3392
+// 41 (199).
 // gate, up and silu(gate) * up of an MLP in one launch (MLP below), 2048 x (2 x 17408) x 5120:
 // 556 us and a reduce of 13, against 268 + 268 and 78 for silu * mul over memory.
 #include <type_traits>
@@ -487,9 +487,12 @@ int gemm_tiled_scale_bytes_per_row(const QmmArgs &a) {
   return gemm_mxfp8_ok(a) ? a.K / 32 : gemm_nvfp4_ok(a) ? a.K / 16 : 0;
 }
 
-// K % 32: whole scale blocks, 16-byte W pieces; x and W rows 16-byte aligned.
+// K % 64: the row lengths whose results the split of x has always served; an odd number of 32-blocks
+// runs gemm.hip's kernel, whose products are exact (a padded half step here would be ten times
+// faster, but of its outputs 1.2% round the other way than the exact sums, of that kernel's 0.01%).
+// x and W rows 16-byte aligned.
 bool gemm_mxfp8_ok(const QmmArgs &a) {
-  return a.mode == MXFP8 && !a.x_f32 && a.K % 32 == 0 && a.K > 0 && a.M > 0 && a.N > 0 && (uintptr_t)a.x % 16 == 0 &&
+  return a.mode == MXFP8 && !a.x_f32 && a.K % X_BK == 0 && a.K > 0 && a.M > 0 && a.N > 0 && (uintptr_t)a.x % 16 == 0 &&
          (uintptr_t)a.w % 16 == 0 && (uintptr_t)a.w_up % 16 == 0;
 }
 

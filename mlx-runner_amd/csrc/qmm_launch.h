@@ -87,7 +87,7 @@ bool qmv_mlp_ok(const QmmArgs &a);
 hipError_t launch_qmv_mlp(const QmmArgs &a, const uint8_t *w_up, const uint8_t *s_up, hipStream_t st);
 hipError_t launch_silu_mul(const void *g, const void *u, void *h, int64_t n, bool f32, hipStream_t st);
 
-// nvfp4 prefill at K % 32 = 16, which the pipelined GEMM below does not take.
+// Prefill at the K that the pipelined GEMMs below do not take (nvfp4 K % 32 = 16, mxfp8 K % 64 = 32).
 bool gemm_ok(const QmmArgs &a);
 hipError_t launch_gemm(const QmmArgs &a, hipStream_t st);
 
@@ -116,15 +116,18 @@ int gemm_tiled_scale_bytes_per_row(const QmmArgs &a);
 // Whether a call runs on the decode kernels (x of at most QMV_MAX_M rows, and x of up to
 // 16 rows where the MFMA decode kernels take it: mxfp8 on the scaled MFMA, nvfp4 at
 // K = 5120 / 6144 from 5 rows on the dequantizing bf16-MFMA kernel) rather than a prefill GEMM.  x of
-// 5-8 rows that no MFMA decode kernel takes (mxfp8 at K = 17408 from 6 rows and at other K;
+// 5-8 rows that no MFMA decode kernel takes (mxfp8 at K = 17408 from 6 rows and at other K % 128 = 0;
 // nvfp4 where qmv_any_ok says no) runs on the pipelined GEMM's split tiles when the matrix is
 // tall: the other decode kernel is the unpacking GEMV, whose work grows with every row
-// (N = 5120, K = 17408, mxfp8: 50-61 us at 6-8 rows; the GEMM 23 us).
+// (N = 5120, K = 17408, mxfp8: 50-61 us at 6-8 rows; the GEMM 23 us).  mxfp8 at K % 128 != 0 stays
+// on the GEMV, whose products are exact: the GEMM splits x into two 8-bit parts for the fp8 MFMA,
+// and 1.2% of its outputs round the other way than the exact sums (of the GEMV's 0.003-0.012%).
 inline bool qmm_on_decode(const QmmArgs &a) {
   // (x of 9-16 rows on the MFMA decode kernels, where they take the shape)
   if (a.M > QMV_MAX_M) return a.M <= 16 && qmv_mfma_ok(a);
   if (a.M <= 4 || a.N < 4096 || qmv_mfma_ok(a) || qmv_any_ok(a) || ((uintptr_t)a.x | (uintptr_t)a.w) & 15) return true;
-  return !gemm_mxfp8_ok(a) && !gemm_nvfp4_ok(a);
+  if (a.mode == MXFP8) return !(gemm_mxfp8_ok(a) && a.K % 128 == 0 && ((uintptr_t)a.s & 3) == 0);
+  return !gemm_nvfp4_ok(a);
 }
 
 // dequant: out [N, K] float32 (out_f32) or bfloat16.

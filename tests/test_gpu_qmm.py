@@ -421,6 +421,32 @@ def test_prefill_tiles(mode, M, N, K):
     assert torch.all((y.double() - ref).abs() <= bound)
 
 
+@pytest.mark.parametrize("M,N,K", [(9, 300, 96), (27, 4672, 1376), (200, 1000, 1056), (147, 2181, 8672),
+                                   (5, 4672, 1344), (7, 4096, 1376), (8, 5000, 192)])
+def test_mxfp8_exact_products_off_the_fp8_gemm(M, N, K):
+    """mxfp8 at K % 64 = 32, and x of 5-8 rows at K % 128 != 0, multiplies x itself, not its two-part
+    8-bit split: nearly every output is the exact sum's bf16.  fp32 sums of K terms are off by
+    a few 2^-24 sqrt(K) of the output's rms, against a rounding step of 2^-8 of the value: at
+    most 2^-14 sqrt(K) of the outputs may round the other way (K = 8672: 0.6%; a split x gives
+    1.2% at every K).  The same through the MLP's projections and in a group."""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + N + K)
+    x = torch.randn((M, K), generator=gen, device="cuda").to(torch.bfloat16)
+    W = (torch.randn((N, K), generator=gen, device="cuda") * 0.02).to(torch.bfloat16)
+    st = Q.Stream.torch_current()
+    wq, sc = Q.quantize(Q.Array.from_torch(W), "mxfp8", stream=st)
+    Wd = torch.from_numpy(Q.dequantize(wq, sc, "mxfp8", dtype=Q.FLOAT32, stream=st).numpy(st)).cuda().double()
+    ref = (x.double() @ Wd.t()).to(torch.bfloat16)
+    xa = Q.Array.from_torch(x)
+    y = Q.quantized_matmul(xa, wq, sc, "mxfp8", stream=st)
+    yg = Q.quantized_matmul_group(xa, [wq], [sc], "mxfp8", stream=st)[0]
+    h = Q.mlp_gate_up_silu(xa, wq, sc, wq, sc, "mxfp8", stream=st)
+    assert np.array_equal(h.numpy(st), Q.silu_mul(y, y, stream=st).numpy(st))
+    assert np.array_equal(yg.numpy(st), y.numpy(st))
+    other = np.mean(y.numpy(st) != ref.view(torch.int16).cpu().numpy().view(np.uint16))
+    assert other <= min(2.0 ** -14 * K ** 0.5, 0.006), other
+
+
 # ---------------------------------------------------------------- MLP activation and the fused gate/up
 def test_silu_mul_matches_oracle():
     """src/model.zig:405-415 / :451-456 on the GPU: bf16 chain within one ulp of the
