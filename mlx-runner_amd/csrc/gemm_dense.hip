@@ -1,6 +1,6 @@
 // Dense bf16 linear y[M, N] = x[M, K] @ w[N, K].T (linear, src/model.zig:200-211): bf16
-// operands, fp32 accumulation, bf16 out (RNE).  x of a few rows runs a GEMV
-// (gemv_bf16_kernel; linear_gemv), taller x a pipelined GEMM on v_mfma_f32_32x32x16_bf16.
+// operands, fp32 accumulation, bf16 out (RNE).  x of up to 8 rows runs a GEMV
+// (gemv_bf16_kernel), taller x a pipelined GEMM on v_mfma_f32_32x32x16_bf16.
 //
 // The GEMM.  What bounds it: at tall x the matrix cores at the clock the power limit leaves
 // (a large library product reaches ~1.45 PFLOP/s here, not 2.5), and before that the time a
@@ -18,11 +18,14 @@
 //   * The tile is chosen per call (dense_plan below): the sizes differ in operand bytes per
 //     MFMA, in how they divide M x N, and in rounds of the chip.  Tiles left over after the
 //     whole rounds are split along K over the idle CUs in the same launch, fp32 partial
-//     sums reduced in K order (deterministic) by a second kernel.
+//     sums reduced in K order (deterministic) by a second kernel.  Without scratch for
+//     them (a call that is being captured: a replay may run beside other calls of the
+//     stream) every tile is whole.
 // Measured, us per call, inputs changing from call to call (M x N x K; the former
 // kernel, 128 x 128 tiles through registers without a pipeline, in brackets):
 //   1000 x 10240 x 5120  92 (172), 2048 x 34816 x 5120  570 = 1.28 PFLOP/s,
-//   512 x 6144 x 5120  45, 64 x 10240 x 5120  27 (110), 16 x 17408 x 5120  39.
+//   512 x 6144 x 5120  45, 64 x 10240 x 5120  27 (110; without scratch 40),
+//   16 x 17408 x 5120  39 (131; 53).
 #include <type_traits>
 
 #include "gemm_pipe.h"
@@ -52,37 +55,47 @@ __global__ __launch_bounds__(64 * W) void gemv_bf16_kernel(const uint16_t *__res
   for (int r = 0; r < R; ++r)
 #pragma unroll
     for (int m = 0; m < M; ++m) acc[r][m] = 0.f;
-  // chunk c + 64 W u of the rows, u < U
-  auto chunks = [&](auto u_c, int c) __attribute__((always_inline)) {
-    constexpr int UU = decltype(u_c)::value;
-    uint4 q[UU][R];
-#pragma unroll
-    for (int u = 0; u < UU; ++u)
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const int n = n0 + r < N ? n0 + r : N - 1;
-        q[u][r] = load_stream16((const uint4 *)(w + (int64_t)n * K) + c + 64 * W * u);
-      }
-#pragma unroll
-    for (int u = 0; u < UU; ++u)
-#pragma unroll
-      for (int m = 0; m < M; ++m) {
-        const uint4 xv = ((const uint4 *)(x + (int64_t)m * K))[c + 64 * W * u];
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-          float t = acc[r][m];
-          t = dot2_bf16(__builtin_bit_cast(bf16x2_t, q[u][r].x), xv.x, t);
-          t = dot2_bf16(__builtin_bit_cast(bf16x2_t, q[u][r].y), xv.y, t);
-          t = dot2_bf16(__builtin_bit_cast(bf16x2_t, q[u][r].z), xv.z, t);
-          t = dot2_bf16(__builtin_bit_cast(bf16x2_t, q[u][r].w), xv.w, t);
-          acc[r][m] = t;
-        }
-      }
+  auto dot8 = [](float t, uint4 q, uint4 xv) __attribute__((always_inline)) {
+    t = dot2_bf16(__builtin_bit_cast(bf16x2_t, q.x), xv.x, t);
+    t = dot2_bf16(__builtin_bit_cast(bf16x2_t, q.y), xv.y, t);
+    t = dot2_bf16(__builtin_bit_cast(bf16x2_t, q.z), xv.z, t);
+    return dot2_bf16(__builtin_bit_cast(bf16x2_t, q.w), xv.w, t);
   };
   int c = tid;
+  // chunks c + 64 W u of the rows, u < U
   if constexpr (U > 1)
-    for (; c + 64 * W * (U - 1) < C; c += 64 * W * U) chunks(std::integral_constant<int, U>{}, c);
-  for (; c < C; c += 64 * W) chunks(std::integral_constant<int, 1>{}, c);
+    for (; c + 64 * W * (U - 1) < C; c += 64 * W * U) {
+      uint4 q[U][R];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const int n = n0 + r < N ? n0 + r : N - 1;
+          q[u][r] = load_stream16((const uint4 *)(w + (int64_t)n * K) + c + 64 * W * u);
+        }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+          const uint4 xv = ((const uint4 *)(x + (int64_t)m * K))[c + 64 * W * u];
+#pragma unroll
+          for (int r = 0; r < R; ++r) acc[r][m] = dot8(acc[r][m], q[u][r], xv);
+        }
+    }
+  for (; c < C; c += 64 * W) {
+    uint4 q[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int n = n0 + r < N ? n0 + r : N - 1;
+      q[r] = load_stream16((const uint4 *)(w + (int64_t)n * K) + c);
+    }
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      const uint4 xv = ((const uint4 *)(x + (int64_t)m * K))[c];
+#pragma unroll
+      for (int r = 0; r < R; ++r) acc[r][m] = dot8(acc[r][m], q[r], xv);
+    }
+  }
   float out = 0.f;
 #pragma unroll
   for (int r = 0; r < R; ++r)
@@ -120,15 +133,11 @@ static void launch_gemv(const uint16_t *x, const uint16_t *w, uint16_t *y, int N
   else hipLaunchKernelGGL((gemv_bf16_kernel<M, 1, 1>), grid, dim3(64), 0, st, x, w, y, N, K);
 }
 
-// x of up to 5 rows runs the GEMV, and up to 8 rows on matrices whose row groups are fewer than
-// two per CU: its work grows with every row, the GEMM's does not (us at 6 rows, GEMV / GEMM:
-// 10240 x 5120 28 / 21, 5120 x 6144 20 / 16, 2000 x 4096 10.9 / 8.9; 1024 x 5120 7.3 / 8.4; at 5
-// rows 10240 x 5120 23.5 / 21.4, 4000 x 2560 8.2 / 9.9), unless K is short too (2288 x 1216 7.2 /
-// 8.1).
-static bool linear_gemv(int M, int N, int K) {
-  const int groups = (N + 3) / 4, cus = device_cu_count();
-  return M <= 5 || (M <= QMV_MAX_M && (groups < 2 * cus || (groups < 4 * cus && K < 2048)));
-}
+// x of up to 8 rows, the sizes of decode calls, runs the GEMV, which needs no scratch: a program
+// may capture those calls, forbid allocation around them and issue them from several threads.
+// (At 6-8 rows the GEMM's split tiles are faster, GEMV / GEMM in us: 10240 x 5120 at 6 rows 29 / 25,
+// 5120 x 17408 at 8 rows 47 / 38; but their partial sums are scratch of the stream.)
+static bool linear_gemv(int M) { return M <= QMV_MAX_M; }
 
 // ---------------------------------------------------------------- taller x
 
@@ -323,8 +332,10 @@ constexpr GpCost DN_COST[] = {{256, 256, 1, 3.f, {1.24f}},         {256, 160, 1,
                               {64, 64, 3, 3.f, {0.42f, 0.57f, 0.72f}}};
 }  // namespace
 
-static GpPlan dense_plan(int M, int N, int K) {
-  return gp_plan(DN_COST, sizeof(DN_COST) / sizeof(DN_COST[0]), M, N, (K + D_BK - 1) / D_BK, 1, device_cu_count());
+// (split: with scratch for the partial sums of tiles split along K)
+static GpPlan dense_plan(int M, int N, int K, bool split) {
+  return gp_plan(DN_COST, sizeof(DN_COST) / sizeof(DN_COST[0]), M, N, (K + D_BK - 1) / D_BK, 1, device_cu_count(),
+                 split ? GP_MAX_SPLIT : 1);
 }
 
 template <class G>
@@ -357,15 +368,15 @@ static hipError_t launch_dense_plan(const uint16_t *x, const uint16_t *w, uint16
 }
 
 size_t linear_bf16_workspace(int M, int N, int K) {
-  if (linear_gemv(M, N, K)) return 0;
-  const GpPlan p = dense_plan(M, N, K);
+  if (linear_gemv(M)) return 0;
+  const GpPlan p = dense_plan(M, N, K, true);
   return (size_t)p.left * p.S * DN_COST[p.cfg].TM * DN_COST[p.cfg].TN * sizeof(float);
 }
 
 hipError_t launch_linear_bf16(const uint16_t *x, const uint16_t *w, uint16_t *y, int M, int N, int K, void *ws,
                               hipStream_t st) {
   if (K % 16 != 0 || M <= 0 || N <= 0) return hipErrorInvalidValue;
-  if (!linear_gemv(M, N, K)) return launch_dense_plan(x, w, y, M, N, K, dense_plan(M, N, K), (float *)ws, st);
+  if (!linear_gemv(M)) return launch_dense_plan(x, w, y, M, N, K, dense_plan(M, N, K, ws != nullptr), (float *)ws, st);
   switch (M) {
 #define QMM_GEMV_CASE(MM) \
   case MM: launch_gemv<MM>(x, w, y, N, K, st); break;

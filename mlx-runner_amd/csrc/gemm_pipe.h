@@ -290,11 +290,12 @@ struct GpPlan {
   int cfg, whole, left, S;  // whole tiles, then `left` tiles split S ways along K
 };
 // The least estimated time over every tile size and every split of the tiles left after the
-// whole rounds (at most GP_MAX_SPLIT ways, one round of blocks, at least 4 K steps each, in
+// whole rounds (at most max_split ways, one round of blocks, at least 4 K steps each, in
 // units of `unit` steps).  Where several blocks share a CU, the last round may instead give
 // every CU `more` whole tiles and the split ones run beside them.  A split adds the reduce: its
 // launch and its partial sums' traffic.
-inline GpPlan gp_plan(const GpCost *costs, int n, int M, int64_t N, int steps, int unit, int cus) {
+inline GpPlan gp_plan(const GpCost *costs, int n, int M, int64_t N, int steps, int unit, int cus,
+                      int max_split = GP_MAX_SPLIT) {
   if (cus <= 0) cus = 256;  // (no device answers: the launch reports it)
   GpPlan best{0, 0, 0, 1};
   float best_us = 1e30f;
@@ -306,7 +307,7 @@ inline GpPlan gp_plan(const GpCost *costs, int n, int M, int64_t N, int steps, i
     for (int more = 0; more < d.per_cu; ++more) {
       const int64_t whole = rounds * slots + (int64_t)more * cus, left = T - whole;
       if (left < 0) break;
-      for (int S = 1; S <= GP_MAX_SPLIT; ++S) {
+      for (int S = 1; S <= max_split; ++S) {
         if (S > 1 && (left == 0 || left * S > slots - (int64_t)more * cus || units < S || steps < 4 * S)) break;
         if (more && left && S == 1) continue;  // (the same blocks as more = 0)
         const int mine = (units + S - 1) / S * unit, split_steps = mine < steps ? mine : steps;

@@ -191,8 +191,8 @@ void give_back(FreeList &l, size_t keep_bytes, size_t keep_count) {
 }  // namespace
 
 // Stream-ordered HBM allocation (cached by the device's default pool, and above it for the
-// null stream).
-int alloc_device(void **p, size_t bytes, hipStream_t st) {
+// null stream); the runtime's record of a failure is cleared.
+static hipError_t try_alloc_device(void **p, size_t bytes, hipStream_t st) {
   pool_init();
   *p = nullptr;
   const size_t cap = capacity_of(bytes);
@@ -205,7 +205,7 @@ int alloc_device(void **p, size_t bytes, hipStream_t st) {
         *p = l.bufs[i].second;
         l.bytes -= cap;
         l.bufs.erase(l.bufs.begin() + (ptrdiff_t)i);
-        return 0;
+        return hipSuccess;
       }
   }
   hipError_t e = hipMallocAsync(p, cap, st);
@@ -217,10 +217,14 @@ int alloc_device(void **p, size_t bytes, hipStream_t st) {
     }
     e = hipMallocAsync(p, cap, st);
   }
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e;
+}
+
+int alloc_device(void **p, size_t bytes, hipStream_t st) {
+  const hipError_t e = try_alloc_device(p, bytes, st);
+  if (e != hipSuccess)
     return fail("[qmm::malloc] Unable to allocate %zu bytes: %s (out of memory)", bytes, hipGetErrorName(e));
-  }
   return 0;
 }
 
@@ -250,35 +254,49 @@ std::mutex g_ws_mtx;
 std::map<std::pair<int, uintptr_t>, std::pair<void *, size_t>> g_ws;
 }  // namespace
 
-int workspace(hipStream_t st, size_t bytes, void **out, bool *transient) {
+// Whether the stream is being captured into a graph (or cannot say).
+static bool capturing(hipStream_t st) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
+static hipError_t try_workspace(hipStream_t st, size_t bytes, void **out, bool *transient) {
   *transient = false;
   *out = nullptr;
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return fail_hip(e, "qmm::workspace");
+  if (e != hipSuccess) return e;
   std::lock_guard<std::mutex> lk(g_ws_mtx);
   auto &ent = g_ws[{dev, (uintptr_t)st}];
   if (ent.first && ent.second >= bytes) {
     *out = ent.first;
-    return 0;
+    return hipSuccess;
   }
   // While the stream is being captured, growing would record an allocation into the
   // graph that the cache then keeps: take a transient allocation instead.
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(st, &cs) != hipSuccess) {
-    (void)hipGetLastError();
-    cs = hipStreamCaptureStatusActive;  // unknown: the transient path is safe either way
-  }
-  if (cs != hipStreamCaptureStatusNone) {
+  if (capturing(st)) {  // (unknown: the transient path is safe either way)
     *transient = true;
-    return alloc_device(out, bytes, st);
+    return try_alloc_device(out, bytes, st);
   }
   size_t cap = (size_t)1 << 20;
   while (cap < bytes) cap <<= 1;
   void *p = nullptr;
-  if (alloc_device(&p, cap, st)) return 1;
+  e = try_alloc_device(&p, cap, st);
+  if (e != hipSuccess) return e;
   ent = {p, cap};
   *out = p;
+  return hipSuccess;
+}
+
+int workspace(hipStream_t st, size_t bytes, void **out, bool *transient) {
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return fail_hip(e, "qmm::workspace");
+  e = try_workspace(st, bytes, out, transient);
+  if (e != hipSuccess)
+    return fail("[qmm::workspace] Unable to allocate %zu bytes: %s (out of memory)", bytes, hipGetErrorName(e));
   return 0;
 }
 
@@ -1178,8 +1196,13 @@ int qmm_linear(qmm_array *res, qmm_array x, qmm_array w, qmm_stream s) {
   if (M == 0 || N == 0) return finish(0);
   void *ws = nullptr;
   bool transient = false;
+  // scratch only for eager calls (a graph's replays may overlap the stream's other calls), and
+  // a call that gets none runs without: the same result but for the order of the fp32 sums
   const size_t need = linear_bf16_workspace((int)M, N, K);
-  if (need && workspace(st, need, &ws, &transient)) return finish(1);
+  if (need && !capturing(st) && try_workspace(st, need, &ws, &transient) != hipSuccess) {
+    (void)hipGetLastError();
+    ws = nullptr;
+  }
   hipError_t e = launch_linear_bf16((const uint16_t *)xa->data, (const uint16_t *)wa->data, (uint16_t *)ya->data,
                                     (int)M, N, K, ws, st);
   if (transient) (void)hipFreeAsync(ws, st);  // stream-ordered: released after the kernels that use it

@@ -175,7 +175,7 @@ int device_cu_count();
 hipError_t ensure_dynamic_lds(std::atomic<uint64_t> &done, const void *kernel, int bytes);
 
 // Dense bf16 y[M, N] = x[M, K] @ w[N, K].T (fp32 accumulate, RNE), with a workspace of
-// linear_bf16_workspace bytes (0: none).
+// linear_bf16_workspace bytes (0: none); without it (null) the call splits no tile along K.
 size_t linear_bf16_workspace(int M, int N, int K);
 hipError_t launch_linear_bf16(const uint16_t *x, const uint16_t *w, uint16_t *y, int M, int N, int K, void *ws,
                               hipStream_t st);

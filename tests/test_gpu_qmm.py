@@ -391,6 +391,81 @@ def test_dense_linear_tiles(M, N, K):
     assert torch.all((y.double() - ref).abs() <= bound)
 
 
+class _RawStream:
+    """A HIP stream of its own (torch hands out pooled ones), seen by torch and by the library."""
+
+    def __init__(self):
+        self.hip = ctypes.CDLL("libamdhip64.so")
+        self.ptr = ctypes.c_void_p()
+        assert self.hip.hipStreamCreate(ctypes.byref(self.ptr)) == 0
+        self.torch = torch.cuda.ExternalStream(self.ptr.value)
+
+    def pool_used(self):
+        """Bytes in use of the device's default memory pool, where the library's scratch lives."""
+        pool, used = ctypes.c_void_p(), ctypes.c_uint64()
+        assert self.hip.hipDeviceGetDefaultMemPool(ctypes.byref(pool), 0) == 0
+        assert self.hip.hipMemPoolGetAttribute(pool, 7, ctypes.byref(used)) == 0  # hipMemPoolAttrUsedMemCurrent
+        return used.value
+
+
+def _dense(M, N, K, seed):
+    """x, w, x @ w.T in float64 and its bound: one bf16 rounding and the fp32 sums' error."""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(seed)
+    x = torch.randn((M, K), generator=gen, device="cuda").to(torch.bfloat16)
+    w = (torch.randn((N, K), generator=gen, device="cuda") * 0.02).to(torch.bfloat16)
+    ref = x.double() @ w.double().t()
+    bound = ref.abs() * 2.0 ** -8 + (x.double().abs() @ w.double().abs().t()) * (K * 2.0 ** -24) + 1e-30
+    return x, w, ref, bound
+
+
+@pytest.mark.parametrize("M", [6, 7, 8, 16])
+def test_dense_linear_takes_no_scratch_at_decode_or_in_a_graph(M):
+    """x of up to 8 rows allocates nothing on a stream that has no workspace yet, and neither
+    does a captured call of any size, whose tiles are then whole; replays on another stream
+    beside eager calls of the capture stream, whose split tiles use that stream's workspace,
+    leave both results right."""
+    N, K = 10240, 5120
+    x, w, ref, bound = _dense(M, N, K, M)
+    x2, w2, ref2, bound2 = _dense(64, N, K, M + 100)
+    y, y2 = (torch.full((m, N), float("nan"), dtype=torch.bfloat16, device="cuda") for m in (M, 64))
+    xa, wa, x2a, w2a, ya, y2a = (Q.Array.from_torch(t) for t in (x, w, x2, w2, y, y2))
+    s = _RawStream()
+    torch.cuda.synchronize()
+    used = s.pool_used()
+    with torch.cuda.stream(s.torch):
+        if M <= 8:
+            Q.linear(xa, wa, out=ya, stream=Q.Stream.torch_current())
+            torch.cuda.synchronize()
+            assert s.pool_used() == used
+            assert torch.all((y.double() - ref).abs() <= bound)
+        Q.linear(x2a, w2a, out=y2a, stream=Q.Stream.torch_current())  # the stream's workspace is there from now on
+    torch.cuda.synchronize()
+    used = s.pool_used()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph, stream=s.torch):
+        Q.linear(xa, wa, out=ya, stream=Q.Stream.torch_current())
+    nodes = ctypes.c_size_t()
+    assert s.hip.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(nodes)) == 0
+    assert nodes.value == 1  # one kernel: no partial sums, no memory node
+    graph.instantiate()
+    other = torch.cuda.Stream()
+    for _ in range(20):
+        y.fill_(float("nan"))
+        y2.fill_(float("nan"))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(other):
+            graph.replay()
+            graph.replay()
+        with torch.cuda.stream(s.torch):
+            for _ in range(3):
+                Q.linear(x2a, w2a, out=y2a, stream=Q.Stream.torch_current())
+        torch.cuda.synchronize()
+        assert torch.all((y.double() - ref).abs() <= bound)
+        assert torch.all((y2.double() - ref2).abs() <= bound2)
+    assert s.pool_used() == used
+
+
 @pytest.mark.parametrize("mode", ["nvfp4", "mxfp8"])
 @pytest.mark.parametrize("M,N,K", [
     (17, 1, 32), (33, 129, 96), (64, 257, 224), (65, 300, 288),       # K ends inside a step or a stage of W
