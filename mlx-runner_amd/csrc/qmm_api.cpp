@@ -245,13 +245,23 @@ static void free_device(void *p, size_t bytes, hipStream_t st, int dev) {
 // ---------------------------------------------------------------- workspaces
 // One grow-only workspace per (device, stream), for the per-call scratch of the
 // prefill GEMMs and the chunked GDN form.  Calls on one stream are ordered, so they
-// can share it; calls on different streams get different ones.  A buffer the stream
-// outgrows stays allocated until the process ends: a graph captured earlier may
-// still point at it.  Sizes are powers of two from 1 MiB, so what is kept is under
-// twice the largest request.
+// can share it; calls on different streams get different ones.  A call of several launches
+// holds the workspace until all of them are enqueued: another host thread's call on the
+// same stream (the null stream is one for all threads) then comes after them all, not
+// between a GEMM and its reduce.  A buffer the stream outgrows stays allocated until the
+// process ends: a graph captured earlier may still point at it.  Sizes are powers of two
+// from 1 MiB, so what is kept is under twice the largest request.
 namespace {
+struct Workspace {
+  std::mutex mtx;
+  void *p = nullptr;
+  size_t cap = 0;
+};
 std::mutex g_ws_mtx;
-std::map<std::pair<int, uintptr_t>, std::pair<void *, size_t>> g_ws;
+std::map<std::pair<int, uintptr_t>, Workspace> &workspaces() {
+  static auto *m = new std::map<std::pair<int, uintptr_t>, Workspace>();  // (entries stay where they are)
+  return *m;
+}
 }  // namespace
 
 // Whether the stream is being captured into a graph (or cannot say).
@@ -262,42 +272,49 @@ static bool capturing(hipStream_t st) {
   return true;
 }
 
-static hipError_t try_workspace(hipStream_t st, size_t bytes, void **out, bool *transient) {
-  *transient = false;
-  *out = nullptr;
+hipError_t Scratch::try_take(hipStream_t st, size_t bytes) {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
-  std::lock_guard<std::mutex> lk(g_ws_mtx);
-  auto &ent = g_ws[{dev, (uintptr_t)st}];
-  if (ent.first && ent.second >= bytes) {
-    *out = ent.first;
-    return hipSuccess;
+  Workspace *ws;
+  {
+    std::lock_guard<std::mutex> lk(g_ws_mtx);
+    ws = &workspaces()[{dev, (uintptr_t)st}];
   }
-  // While the stream is being captured, growing would record an allocation into the
-  // graph that the cache then keeps: take a transient allocation instead.
-  if (capturing(st)) {  // (unknown: the transient path is safe either way)
-    *transient = true;
-    return try_alloc_device(out, bytes, st);
+  std::unique_lock<std::mutex> lk(ws->mtx);
+  if (!ws->p || ws->cap < bytes) {
+    // While the stream is being captured, growing would record an allocation into the
+    // graph that the cache then keeps: take a transient allocation instead.
+    if (capturing(st)) {  // (unknown: the transient path is safe either way)
+      void *p = nullptr;
+      e = try_alloc_device(&p, bytes, st);
+      if (e == hipSuccess) ptr_ = p, transient_ = true, st_ = st;
+      return e;
+    }
+    size_t cap = (size_t)1 << 20;
+    while (cap < bytes) cap <<= 1;
+    void *p = nullptr;
+    e = try_alloc_device(&p, cap, st);
+    if (e != hipSuccess) return e;
+    ws->p = p, ws->cap = cap;
   }
-  size_t cap = (size_t)1 << 20;
-  while (cap < bytes) cap <<= 1;
-  void *p = nullptr;
-  e = try_alloc_device(&p, cap, st);
-  if (e != hipSuccess) return e;
-  ent = {p, cap};
-  *out = p;
+  ptr_ = ws->p;
+  lk_ = std::move(lk);
   return hipSuccess;
 }
 
-int workspace(hipStream_t st, size_t bytes, void **out, bool *transient) {
+int Scratch::take(hipStream_t st, size_t bytes) {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return fail_hip(e, "qmm::workspace");
-  e = try_workspace(st, bytes, out, transient);
+  e = try_take(st, bytes);
   if (e != hipSuccess)
     return fail("[qmm::workspace] Unable to allocate %zu bytes: %s (out of memory)", bytes, hipGetErrorName(e));
   return 0;
+}
+
+Scratch::~Scratch() {
+  if (transient_) (void)hipFreeAsync(ptr_, st_);  // stream-ordered: released after the kernels that use it
 }
 
 Arr *new_arr(const int *shape, int dim, qmm_dtype dtype) {
@@ -692,11 +709,10 @@ static int run_qmm(QmmArgs &a, size_t ybytes, hipStream_t st, const char *op, vo
     const bool fp8 = gemm_mxfp8_ok(a);
     if (!a.s_tiled && tiled_scales(scales_arr, a, st, &a.s_tiled)) return 1;
     const size_t need = fp8 ? gemm_mxfp8_workspace(a) : gemm_nvfp4_workspace(a);
-    void *ws = ws_given;
-    bool transient = false;
-    if (!ws && workspace(st, need, &ws, &transient)) return 1;
+    Scratch scratch;
+    if (!ws_given && need && scratch.take(st, need)) return 1;
+    void *ws = ws_given ? ws_given : scratch.get();
     e = fp8 ? launch_gemm_mxfp8(a, ws, st) : launch_gemm_nvfp4(a, ws, st);
-    if (transient) (void)hipFreeAsync(ws, st);  // stream-ordered: released after the kernels that use it
   } else if (aligned && gemm_ok(a)) {
     e = launch_gemm(a, st);
   } else {
@@ -955,11 +971,9 @@ int qmm_gdn_recurrence(qmm_array *y, qmm_array *state_out, qmm_array q, qmm_arra
   if (a.T == 0) {
     e = gdn_no_steps(a, st);
   } else if (gdn_chunked_ok(a)) {  // long T: the chunked form, its per-chunk matrices in the stream's workspace
-    void *ws = nullptr;
-    bool transient = false;
-    if (workspace(st, gdn_chunked_workspace(a), &ws, &transient)) return finish(1);
-    e = launch_gdn_chunked(a, ws, st);
-    if (transient) (void)hipFreeAsync(ws, st);  // stream-ordered: released after the kernels that use it
+    Scratch scratch;
+    if (scratch.take(st, gdn_chunked_workspace(a))) return finish(1);
+    e = launch_gdn_chunked(a, scratch.get(), st);
   } else {
     e = launch_gdn(a, st);
   }
@@ -1094,10 +1108,9 @@ int qmm_mlp_gate_up_silu(qmm_array *res, qmm_array x, qmm_array w_gate, qmm_arra
   // and the projections' own workspace in the stream's workspace
   const size_t bytes = (ha->nbytes() + 255) & ~(size_t)255;
   const size_t gemm_ws = std::max(qmm_workspace(a), qmm_workspace(b));
-  void *ws = nullptr;
-  bool transient = false;
-  if (workspace(st, 2 * bytes + gemm_ws, &ws, &transient)) return finish(1);
-  void *g = ws, *u = (char *)ws + bytes, *gws = gemm_ws ? (char *)ws + 2 * bytes : nullptr;
+  Scratch scratch;
+  if (scratch.take(st, 2 * bytes + gemm_ws)) return finish(1);
+  void *g = scratch.get(), *u = (char *)g + bytes, *gws = gemm_ws ? (char *)g + 2 * bytes : nullptr;
   a.y = g;
   b.y = u;
   int rc = run_qmm(a, bytes, st, op, gws);
@@ -1106,7 +1119,6 @@ int qmm_mlp_gate_up_silu(qmm_array *res, qmm_array x, qmm_array w_gate, qmm_arra
     hipError_t e = launch_silu_mul(g, u, ha->data, (int64_t)M * N, a.x_f32, st);
     if (e != hipSuccess) rc = fail_hip(e, op);
   }
-  if (transient) (void)hipFreeAsync(ws, st);  // stream-ordered: released after the kernels that use it
   return finish(rc ? 1 : 0);
 }
 
@@ -1194,18 +1206,16 @@ int qmm_linear(qmm_array *res, qmm_array x, qmm_array w, qmm_stream s) {
   Arr *ya;
   if (alloc_arr(res, oshape, QMM_BFLOAT16, st, &ya)) return finish(1);
   if (M == 0 || N == 0) return finish(0);
-  void *ws = nullptr;
-  bool transient = false;
-  // scratch only for eager calls (a graph's replays may overlap the stream's other calls), and
-  // a call that gets none runs without: the same result but for the order of the fp32 sums
-  const size_t need = linear_bf16_workspace((int)M, N, K);
-  if (need && !capturing(st) && try_workspace(st, need, &ws, &transient) != hipSuccess) {
-    (void)hipGetLastError();
-    ws = nullptr;
+  hipError_t e;
+  {
+    // scratch only for eager calls (a graph's replays may overlap the stream's other calls), and
+    // a call that gets none runs without: the same result but for the order of the fp32 sums
+    Scratch scratch;
+    const size_t need = linear_bf16_workspace((int)M, N, K);
+    if (need && !capturing(st) && scratch.try_take(st, need) != hipSuccess) (void)hipGetLastError();
+    e = launch_linear_bf16((const uint16_t *)xa->data, (const uint16_t *)wa->data, (uint16_t *)ya->data, (int)M, N, K,
+                           scratch.get(), st);
   }
-  hipError_t e = launch_linear_bf16((const uint16_t *)xa->data, (const uint16_t *)wa->data, (uint16_t *)ya->data,
-                                    (int)M, N, K, ws, st);
-  if (transient) (void)hipFreeAsync(ws, st);  // stream-ordered: released after the kernels that use it
   if (e != hipSuccess) return finish(fail_hip(e, op));
   return finish(0);
 }

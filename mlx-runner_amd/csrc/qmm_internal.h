@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -47,10 +48,26 @@ int finish(int rc);
 // start of every op that launches work).
 void begin_op();
 int alloc_device(void **p, size_t bytes, hipStream_t st);
-// Scratch for work enqueued on `st` (at least `bytes`): the stream's grow-only
-// workspace, or while the stream is being captured and that is too small, a
-// transient allocation (*transient) the caller releases after its kernels.
-int workspace(hipStream_t st, size_t bytes, void **out, bool *transient);
+// Scratch for the work that one call enqueues on `st`, kept until the object goes: the
+// stream's grow-only workspace, which no other call gets meanwhile, or while the stream is
+// being captured and that is too small, a transient allocation released (stream-ordered)
+// after the call's kernels.  At most one per call: the workspace's lock is not recursive.
+class Scratch {
+ public:
+  Scratch() = default;
+  Scratch(const Scratch &) = delete;
+  Scratch &operator=(const Scratch &) = delete;
+  ~Scratch();
+  int take(hipStream_t st, size_t bytes);             // non-zero, with the error latched, if there is none
+  hipError_t try_take(hipStream_t st, size_t bytes);  // the same without latching
+  void *get() const { return ptr_; }                  // null before a successful take
+
+ private:
+  void *ptr_ = nullptr;
+  bool transient_ = false;
+  hipStream_t st_ = nullptr;
+  std::unique_lock<std::mutex> lk_;
+};
 Arr *new_arr(const int *shape, int dim, qmm_dtype dtype);
 int alloc_arr(qmm_array *res, const std::vector<int> &shape, qmm_dtype dtype, hipStream_t st, Arr **out);
 void release_arr(Arr *a);

@@ -893,6 +893,65 @@ def test_calls_from_several_host_threads():
     assert Q.take_error() is None
 
 
+def test_calls_from_several_host_threads_on_one_stream():
+    """Four host threads issue the same calls on the null stream, each with its own x and its own
+    results: calls of several launches (split tiles and their reduce, the split of x, the
+    chunked recurrence) share the stream's workspace, and no thread's launches come between
+    another's, so every output equals the call run alone, bit for bit."""
+    import threading
+
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(92)
+    rn = lambda *s: torch.randn(s, generator=gen, device="cuda")  # noqa: E731
+    st, A, M, N, K, T = Q.Stream(), Q.Array.from_torch, 24, 2048, 4128, 130
+    wd = (rn(N, K) * 0.02).to(torch.bfloat16)
+    quant = {mode: Q.quantize(A(wd), mode) for mode in ("mxfp8", "nvfp4")}
+    k = rn(1, T, 2, 128) / 128 ** 0.5
+    gdn = [A(t) for t in (k.to(torch.bfloat16), torch.exp(-0.7 * torch.rand((1, T, 2), generator=gen, device="cuda")),
+                          torch.sigmoid(rn(1, T, 2)).to(torch.bfloat16), rn(1, 2, 128, 128) * 0.1)]
+    xs = [rn(M, K).to(torch.bfloat16) for _ in range(4)]
+    vs = [rn(1, T, 2, 128).to(torch.bfloat16) for _ in range(4)]
+    empty = lambda *s, dt=torch.bfloat16: torch.full(s, float("nan"), dtype=dt, device="cuda")  # noqa: E731
+    outs = [dict(d=empty(M, N), q=empty(M, N), f=empty(M, N), h=empty(M, N), y=empty(1, T, 2, 128),
+                 s=empty(1, 2, 128, 128, dt=torch.float32)) for _ in range(4)]
+
+    def calls(t):
+        x, o = A(xs[t]), {n: A(v) for n, v in outs[t].items()}
+        Q.linear(x, A(wd), out=o["d"], stream=st)
+        Q.quantized_matmul(x, *quant["nvfp4"], "nvfp4", out=o["q"], stream=st)
+        Q.quantized_matmul(x, *quant["mxfp8"], "mxfp8", out=o["f"], stream=st)
+        Q.mlp_gate_up_silu(x, *quant["nvfp4"], *quant["nvfp4"], "nvfp4", out=o["h"], stream=st)
+        Q.gdn_recurrence(gdn[0], gdn[0], A(vs[t]), *gdn[1:], y=o["y"], state_out=o["s"], stream=st)
+
+    refs = []
+    for t in range(4):
+        calls(t)
+        torch.cuda.synchronize()
+        refs.append({n: v.clone() for n, v in outs[t].items()})
+    bad, errors = [], []
+
+    def worker(t, barrier):
+        try:
+            for _ in range(10):
+                barrier.wait()
+                calls(t)
+        except Exception as e:  # reported by the main thread
+            errors.append(repr(e))
+
+    for rep in range(20):
+        barrier = threading.Barrier(4)
+        threads = [threading.Thread(target=worker, args=(t, barrier)) for t in range(4)]
+        for th in threads:
+            th.start()
+        for th in threads:
+            th.join()
+        torch.cuda.synchronize()
+        bad += [(rep, t, n) for t in range(4) for n, v in outs[t].items() if not torch.equal(v, refs[t][n])]
+    assert not errors, errors
+    assert not bad, bad
+    assert Q.take_error() is None
+
+
 @functools.lru_cache(maxsize=2)
 def _nf_weights(mode, N, K):
     return rand_w(np.random.default_rng(4242), mode, N, K)
