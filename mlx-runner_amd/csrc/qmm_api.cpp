@@ -164,79 +164,117 @@ void pool_init() {
 // pass).  As with the pool, a buffer's next user is ordered after its last one by the stream
 // itself; only the null stream's are kept, which is one stream for every thread and is never
 // destroyed (another stream's handle can come back as a different stream).  Per device at most
-// FREE_BYTES in FREE_COUNT buffers, the oldest given back to the pool first, all of them when
-// an allocation fails.
+// FREE_BYTES in FREE_COUNT buffers, the oldest given back to the pool first; all of them when
+// any allocation of the library fails, on whatever stream (give_back_all).
 namespace {
-constexpr size_t FREE_BYTES = (size_t)1 << 30, FREE_COUNT = 64;
-struct FreeList {
-  std::vector<std::pair<size_t, void *>> bufs;  // oldest first
+constexpr size_t FREE_BYTES = (size_t)1 << 30;
+constexpr int FREE_COUNT = 64, FREE_DEVICES = 64;
+struct FreeList {  // oldest first
+  size_t cap[FREE_COUNT + 1];
+  void *buf[FREE_COUNT + 1];
+  int n = 0;
   size_t bytes = 0;
+  void remove(int i) {
+    bytes -= cap[i];
+    for (--n; i < n; ++i) cap[i] = cap[i + 1], buf[i] = buf[i + 1];
+  }
 };
 std::mutex g_free_mtx;
-std::map<int, FreeList> &free_lists() {
-  static auto *m = new std::map<int, FreeList>();  // never destroyed: arrays can outlive static destructors
-  return *m;
-}
+FreeList g_free[FREE_DEVICES];
+bool listed(int dev) { return dev >= 0 && dev < FREE_DEVICES; }
 // (a capacity is what alloc_device took for `bytes`)
 size_t capacity_of(size_t bytes) { return ((bytes ? bytes : 1) + 255) & ~(size_t)255; }
 
-void give_back(FreeList &l, size_t keep_bytes, size_t keep_count) {
-  size_t n = 0;
-  while (n < l.bufs.size() && (l.bytes > keep_bytes || l.bufs.size() - n > keep_count)) {
-    (void)hipFreeAsync(l.bufs[n].second, (hipStream_t)0);
-    l.bytes -= l.bufs[n++].first;
+// A device made current (its null stream is the one meant by 0), the caller's afterwards.
+class DeviceScope {
+ public:
+  explicit DeviceScope(int dev) {
+    if (hipGetDevice(&was_) != hipSuccess || was_ == dev || hipSetDevice(dev) != hipSuccess) was_ = -1;
   }
-  l.bufs.erase(l.bufs.begin(), l.bufs.begin() + (ptrdiff_t)n);
+  ~DeviceScope() {
+    if (was_ >= 0) (void)hipSetDevice(was_);
+  }
+
+ private:
+  int was_ = -1;
+};
+
+// The oldest buffers of the current device's list, until at most these are left.
+void give_back(FreeList &l, size_t keep_bytes, int keep_count) {
+  while (l.n > 0 && (l.bytes > keep_bytes || l.n > keep_count)) {
+    (void)hipFreeAsync(l.buf[0], (hipStream_t)0);
+    l.remove(0);
+  }
 }
+
+// After a failed allocation for `st` (current device `dev`): the kept buffers back to the pool,
+// and their frees completed, so that any stream can have the memory.  False: there were none,
+// or the stream is being captured, when neither may be done.
+bool give_back_all(int dev, hipStream_t st);
 }  // namespace
 
 // Stream-ordered HBM allocation (cached by the device's default pool, and above it for the
-// null stream); the runtime's record of a failure is cleared.
-static hipError_t try_alloc_device(void **p, size_t bytes, hipStream_t st) {
+// null stream); the runtime's record of a failure is cleared.  *dev_out: the buffer's device.
+static hipError_t try_alloc_device(void **p, size_t bytes, hipStream_t st, int *dev_out = nullptr) {
   pool_init();
   *p = nullptr;
   const size_t cap = capacity_of(bytes);
   int dev = -1;
-  if (!st && hipGetDevice(&dev) == hipSuccess) {
+  hipError_t e = hipGetDevice(&dev);
+  if (dev_out) *dev_out = dev;
+  if (e == hipSuccess && !st && listed(dev)) {
     std::lock_guard<std::mutex> lk(g_free_mtx);
-    FreeList &l = free_lists()[dev];
-    for (size_t i = l.bufs.size(); i-- > 0;)  // the latest first: its lines may still be cached
-      if (l.bufs[i].first == cap) {
-        *p = l.bufs[i].second;
-        l.bytes -= cap;
-        l.bufs.erase(l.bufs.begin() + (ptrdiff_t)i);
+    FreeList &l = g_free[dev];
+    for (int i = l.n; i-- > 0;)  // the latest first: its lines may still be cached
+      if (l.cap[i] == cap) {
+        *p = l.buf[i];
+        l.remove(i);
         return hipSuccess;
       }
   }
-  hipError_t e = hipMallocAsync(p, cap, st);
-  if (e != hipSuccess && !st && dev >= 0) {
+  if (e == hipSuccess) e = hipMallocAsync(p, cap, st);
+  if (e != hipSuccess) {
     (void)hipGetLastError();
-    {
-      std::lock_guard<std::mutex> lk(g_free_mtx);
-      give_back(free_lists()[dev], 0, 0);
+    if (give_back_all(dev, st)) {
+      e = hipMallocAsync(p, cap, st);
+      if (e != hipSuccess) (void)hipGetLastError();
     }
-    e = hipMallocAsync(p, cap, st);
   }
-  if (e != hipSuccess) (void)hipGetLastError();
   return e;
 }
 
-int alloc_device(void **p, size_t bytes, hipStream_t st) {
-  const hipError_t e = try_alloc_device(p, bytes, st);
+int alloc_device(void **p, size_t bytes, hipStream_t st, int *dev_out) {
+  const hipError_t e = try_alloc_device(p, bytes, st, dev_out);
   if (e != hipSuccess)
     return fail("[qmm::malloc] Unable to allocate %zu bytes: %s (out of memory)", bytes, hipGetErrorName(e));
   return 0;
 }
 
+hipError_t malloc_plain(void **p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipSuccess) return e;
+  (void)hipGetLastError();
+  int dev = -1;
+  if (hipGetDevice(&dev) == hipSuccess && give_back_all(dev, (hipStream_t)0)) {
+    hipMemPool_t pool;  // (a plain allocation does not take the pool's free memory)
+    if (hipDeviceGetDefaultMemPool(&pool, dev) == hipSuccess) (void)hipMemPoolTrimTo(pool, 0);
+    e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
+  }
+  return e;
+}
+
 // Frees an alloc_device buffer of `bytes` in the order of the stream it was allocated on.
 static void free_device(void *p, size_t bytes, hipStream_t st, int dev) {
   const size_t cap = capacity_of(bytes);
-  if (!st && dev >= 0 && cap <= FREE_BYTES / 2) {
+  if (!st && listed(dev) && cap <= FREE_BYTES / 2) {
     std::lock_guard<std::mutex> lk(g_free_mtx);
-    FreeList &l = free_lists()[dev];
-    l.bufs.emplace_back(cap, p);
-    l.bytes += cap;
-    give_back(l, FREE_BYTES, FREE_COUNT);
+    FreeList &l = g_free[dev];
+    l.cap[l.n] = cap, l.buf[l.n++] = p, l.bytes += cap;
+    if (l.n > FREE_COUNT || l.bytes > FREE_BYTES) {
+      DeviceScope on(dev);
+      give_back(l, FREE_BYTES, FREE_COUNT);
+    }
     return;
   }
   (void)hipFreeAsync(p, st);
@@ -271,6 +309,19 @@ static bool capturing(hipStream_t st) {
   (void)hipGetLastError();
   return true;
 }
+
+namespace {
+bool give_back_all(int dev, hipStream_t st) {
+  if (!listed(dev) || capturing(st)) return false;
+  {
+    std::lock_guard<std::mutex> lk(g_free_mtx);
+    if (g_free[dev].n == 0) return false;
+    give_back(g_free[dev], 0, 0);
+  }
+  if (hipStreamSynchronize((hipStream_t)0) != hipSuccess) (void)hipGetLastError();
+  return true;
+}
+}  // namespace
 
 hipError_t Scratch::try_take(hipStream_t st, size_t bytes) {
   int dev = 0;
@@ -320,10 +371,6 @@ Scratch::~Scratch() {
 Arr *new_arr(const int *shape, int dim, qmm_dtype dtype) {
   if (dim < 0 || dim > QMM_MAX_DIM) return nullptr;
   Arr *a = new Arr();
-  if (hipGetDevice(&a->device) != hipSuccess) {
-    (void)hipGetLastError();
-    a->device = -1;
-  }
   a->ndim = dim;
   for (int i = 0; i < dim; ++i) a->shape[i] = shape[i];
   a->dtype = dtype;
@@ -343,7 +390,7 @@ int alloc_arr(qmm_array *res, const std::vector<int> &shape, qmm_dtype dtype, hi
   }
   Arr *a = new_arr(shape.data(), (int)shape.size(), dtype);
   if (!a) return fail("[qmm] array rank %zu exceeds %d", shape.size(), QMM_MAX_DIM);
-  if (alloc_device(&a->data, a->nbytes(), st)) {
+  if (alloc_device(&a->data, a->nbytes(), st, &a->device)) {
     delete a;
     return 1;
   }
@@ -411,7 +458,7 @@ qmm_array qmm_array_new_data(const void *data, const int *shape, int dim, qmm_dt
     fail("[qmm_array_new_data] bad rank or dtype");
     return qmm_array{nullptr};
   }
-  if (alloc_device(&a->data, a->nbytes(), (hipStream_t)0)) {
+  if (alloc_device(&a->data, a->nbytes(), (hipStream_t)0, &a->device)) {
     delete a;
     return qmm_array{nullptr};
   }
@@ -659,10 +706,7 @@ static int tiled_scales(Arr *sa, const QmmArgs &a, hipStream_t st, const uint32_
   }
   const size_t bytes = tiled_scales_bytes(a.N, nb);
   void *p = nullptr;
-  if (hipMalloc(&p, bytes) != hipSuccess) {
-    (void)hipGetLastError();
-    return 0;
-  }
+  if (malloc_plain(&p, bytes) != hipSuccess) return 0;
   hipError_t e = launch_repack_scales(a.s, (int64_t)a.N, nb, (uint32_t *)p, st);
   if (e == hipSuccess) e = hipStreamSynchronize(st);
   if (e != hipSuccess) {
@@ -1168,7 +1212,7 @@ int qmm_quantize(qmm_vector_array *res, qmm_array w, qmm_optional_int group_size
   for (Arr *a : v->items) {
     a->owned = true;
     a->alloc_stream = st;
-    if (alloc_device(&a->data, a->nbytes(), st)) {
+    if (alloc_device(&a->data, a->nbytes(), st, &a->device)) {
       qmm_vector_array_free(qmm_vector_array{v});
       return finish(1);
     }

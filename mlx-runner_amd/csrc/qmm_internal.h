@@ -19,7 +19,7 @@ struct Arr {
   void *data = nullptr;
   bool owned = false;                   // free the buffer with the handle
   hipStream_t alloc_stream = nullptr;   // stream the buffer was allocated on (stream-ordered free)
-  int device = -1;                      // device current when the handle was made (-1: none)
+  int device = -1;                      // an owned buffer's device
   int ndim = 0;
   int shape[QMM_MAX_DIM] = {0};
   qmm_dtype dtype = QMM_BOOL;
@@ -47,7 +47,10 @@ int finish(int rc);
 // Clears an error the HIP runtime holds for this thread from outside the library (at the
 // start of every op that launches work).
 void begin_op();
-int alloc_device(void **p, size_t bytes, hipStream_t st);
+int alloc_device(void **p, size_t bytes, hipStream_t st, int *dev_out = nullptr);
+// hipMalloc, tried once more after the library's kept buffers are given back; the runtime's
+// record of a failure is cleared.
+hipError_t malloc_plain(void **p, size_t bytes);
 // Scratch for the work that one call enqueues on `st`, kept until the object goes: the
 // stream's grow-only workspace, which no other call gets meanwhile, or while the stream is
 // being captured and that is too small, a transient allocation released (stream-ordered)

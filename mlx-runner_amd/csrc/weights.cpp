@@ -64,9 +64,7 @@ int load_weights(const std::string &dir, hipStream_t st, WeightMap **out) {
   auto alloc = [&](void **p, size_t bytes, const std::string &what) -> int {
     *p = nullptr;
     if (!bytes) return 0;
-    hipError_t e = hipMalloc(p, bytes);
-    if (e != hipSuccess) {
-      (void)hipGetLastError();
+    if (malloc_plain(p, bytes) != hipSuccess) {
       fail("[qmm_weights_load] Unable to allocate %zu bytes for %s (out of memory)", bytes, what.c_str());
       return QMM_WE_IO;
     }

@@ -42,6 +42,51 @@ def test_failed_allocation_reports_out_of_memory():
         Q.lib.qmm_array_free(s)
 
 
+@pytest.mark.parametrize("where", ["null stream", "own stream"])
+def test_failed_allocation_gives_back_the_kept_buffers(where):
+    """Results freed on the null stream are kept for its next ones; an allocation that fails, on
+    that stream or any other, returns them to the device's pool before it is reported."""
+    import ctypes
+
+    hip = ctypes.CDLL("libamdhip64.so.7")  # the runtime torch and the library share
+
+    def pool_used():
+        pool, used = c_void_p(), ctypes.c_uint64()
+        assert hip.hipDeviceGetDefaultMemPool(byref(pool), 0) == 0
+        assert hip.hipMemPoolGetAttribute(pool, 7, byref(used)) == 0  # hipMemPoolAttrUsedMemCurrent
+        return used.value
+
+    def dequantize(N, K, dtype, stream):
+        """(rc, result) of packed nvfp4 [N, K] over a buffer that holds it only if it is small."""
+        w = Q.lib.qmm_array_new_device(c_void_p(buf.data_ptr()), (c_int * 2)(N, K // 8), 2, Q.UINT32)
+        s = Q.lib.qmm_array_new_device(c_void_p(buf.data_ptr()), (c_int * 2)(N, K // 16), 2, Q.UINT8)
+        res = Q.qmm_array(None)
+        rc = Q.lib.qmm_dequantize(byref(res), w, s, Q.qmm_array(None), Q.opt_int(), Q.opt_int(), b"nvfp4",
+                                  Q.qmm_array(None), Q.qmm_optional_dtype(dtype, True), stream.h)
+        Q.lib.qmm_array_free(w)
+        Q.lib.qmm_array_free(s)
+        return rc, res
+
+    N, K = 2048, 8192
+    buf = torch.zeros(N * K // 2, dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    Q.lib.qmm_reset_faults_for_test()
+    rc, res = dequantize(N, K, Q.FLOAT32, Q.Stream())
+    assert rc == 0
+    Q.lib.qmm_array_free(res)  # 64 MiB kept
+    torch.cuda.synchronize()
+    used = pool_used()
+    with torch.cuda.stream(torch.cuda.Stream()):
+        stream = Q.Stream.torch_current() if where == "own stream" else Q.Stream()
+        rc, res = dequantize(1 << 20, 1 << 22, Q.FLOAT32, stream)  # 16 TiB: nothing is launched
+    assert rc != 0 and not res.ctx
+    assert Q.lib.qmm_check_error() == Q.ERR_OOM
+    assert pool_used() <= used - N * K * 4
+    rc, res = dequantize(N, K, Q.FLOAT32, Q.Stream())  # and the library goes on as before
+    assert rc == 0 and Q.lib.qmm_check_error() == 0
+    Q.lib.qmm_array_free(res)
+
+
 @pytest.mark.parametrize("mode,M", [("nvfp4", 1), ("mxfp8", 3), ("nvfp4", 40), ("mxfp8", 300)])
 def test_error_left_by_other_code_is_not_an_op_failure(mode, M):
     """A HIP error the caller's own code left in the runtime (here hipSetDevice on a device

@@ -395,7 +395,7 @@ class _RawStream:
     """A HIP stream of its own (torch hands out pooled ones), seen by torch and by the library."""
 
     def __init__(self):
-        self.hip = ctypes.CDLL("libamdhip64.so")
+        self.hip = ctypes.CDLL("libamdhip64.so.7")  # the runtime torch and the library share
         self.ptr = ctypes.c_void_p()
         assert self.hip.hipStreamCreate(ctypes.byref(self.ptr)) == 0
         self.torch = torch.cuda.ExternalStream(self.ptr.value)
