@@ -182,8 +182,8 @@ int qmm_silu_mul(qmm_array *res, qmm_array g, qmm_array u, qmm_stream s);
  * each projection.  Decode shapes (M <= 4) run one fused kernel (the gate and up
  * rows of an output in one wave, the activation in its epilogue); the result
  * equals quantized_matmul x 2 + silu_mul.  Prefill shapes run one GEMM over both
- * matrices, rounded in the same places; its fp32 sums can be in another order
- * (where a call splits tiles along K). */
+ * matrices, rounded in the same places and summed in the same order: the result equals
+ * quantized_matmul x 2 + silu_mul there too. */
 int qmm_mlp_gate_up_silu(qmm_array *res, qmm_array x, qmm_array w_gate, qmm_array s_gate, qmm_array w_up,
                          qmm_array s_up, qmm_optional_int group_size, qmm_optional_int bits, const char *mode,
                          qmm_stream s);

@@ -28,8 +28,9 @@
 // 2048 x 17408 x 5120  269 (282), 200 x 5120 x 17408  54 (61), 48 x 17408 x 5120  28-35 (37-46),
 // 385 x 4129 x 1280  20 (32); K % 128 = 64, which ran an unpipelined kernel: 68 x 27408 x 3392
 // 41 (199).
-// gate, up and silu(gate) * up of an MLP in one launch (MLP below), 2048 x (2 x 17408) x 5120:
-// 556 us and a reduce of 13, against 268 + 268 and 78 for silu * mul over memory.
+// gate, up and silu(gate) * up of an MLP in one launch (MLP below), 2048 x (2 x 17408) x 5120 with
+// the split of x: 572 us, against 614 for the three calls, whose result it gives bit for bit
+// (gp_plan_pair; splitting the last tiles as suits one launch best took 550).
 #include <type_traits>
 
 #include "gemm_pipe.h"
@@ -190,10 +191,11 @@ __global__ __launch_bounds__(G::THREADS, G::LDS <= 81920 ? 2 * G::NW / 4 : G::NW
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % G::WM, wn = wave / G::WM;
-  const int tiles_m = (M + G::TM - 1) / G::TM, tiles_n = (N + TC - 1) / TC;
+  const int tiles_m = (M + G::TM - 1) / G::TM, tiles_n = (N + G::TN - 1) / G::TN;
   const int steps = (K + X_BK - 1) / X_BK, stages = (steps + 1) / 2;
-  const GpBlock blk = gp_block(blockIdx.x, tiles_m, tiles_n, whole_tiles, S);
+  const GpBlock blk = gp_block<MLP>(blockIdx.x, tiles_m, tiles_n, whole_tiles, S);
   const int m0 = blk.tm * G::TM, n0 = blk.tn * TC;
+  if (MLP && n0 >= N) return;  // the second half of the last pair (its partial sums are not read either)
   const int g_begin = blk.split ? (int)((int64_t)blk.kr * stages / S) : 0;
   const int g_end = blk.split ? (int)((int64_t)(blk.kr + 1) * stages / S) : stages;
   const int s_begin = g_begin * 2, s_end = min(g_end * 2, steps);
@@ -430,8 +432,9 @@ constexpr int MX_CONFIGS = sizeof(MX_COST) / sizeof(MX_COST[0]);
 }  // namespace
 
 static GpPlan mx_plan(const QmmArgs &a) {
-  return gp_plan(MX_COST, a.w_up ? MX_CONFIGS - 2 : MX_CONFIGS, a.M, a.w_up ? 2 * (int64_t)a.N : a.N, (a.K + X_BK - 1) / X_BK, 2,
-                 device_cu_count());
+  const int steps = (a.K + X_BK - 1) / X_BK, cus = device_cu_count();
+  const GpPlan one = gp_plan(MX_COST, MX_CONFIGS, a.M, a.N, steps, 2, cus);
+  return a.w_up ? gp_plan_pair(MX_COST, MX_CONFIGS - 2, one, a.M, a.N, steps, 2, cus) : one;
 }
 
 // The workspace: the split x, its scales, the repacked W scales that do not come tile-major,
@@ -493,7 +496,7 @@ int gemm_tiled_scale_bytes_per_row(const QmmArgs &a) {
 // x and W rows 16-byte aligned.
 bool gemm_mxfp8_ok(const QmmArgs &a) {
   return a.mode == MXFP8 && !a.x_f32 && a.K % X_BK == 0 && a.K > 0 && a.M > 0 && a.N > 0 && (uintptr_t)a.x % 16 == 0 &&
-         (uintptr_t)a.w % 16 == 0 && (uintptr_t)a.w_up % 16 == 0;
+         (uintptr_t)a.w % 16 == 0 && (uintptr_t)a.w_up % 16 == 0 && (!a.w_up || mx_plan(a).cfg >= 0);
 }
 
 size_t gemm_mxfp8_workspace(const QmmArgs &a) {

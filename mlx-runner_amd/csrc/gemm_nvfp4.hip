@@ -83,10 +83,11 @@ __global__ __launch_bounds__(G::THREADS, G::LDS <= 81920 ? 2 * G::NW / 4 : G::NW
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % G::WM, wn = wave / G::WM;
-  const int tiles_m = (M + G::TM - 1) / G::TM, tiles_n = (N + TC - 1) / TC;
+  const int tiles_m = (M + G::TM - 1) / G::TM, tiles_n = (N + G::TN - 1) / G::TN;
   const int steps = (K + V_BK - 1) / V_BK, stages = (steps + V_SS - 1) / V_SS;
-  const GpBlock blk = gp_block(blockIdx.x, tiles_m, tiles_n, whole_tiles, S);
+  const GpBlock blk = gp_block<MLP>(blockIdx.x, tiles_m, tiles_n, whole_tiles, S);
   const int m0 = blk.tm * G::TM, n0 = blk.tn * TC;
+  if (MLP && n0 >= N) return;  // the second half of the last pair (its partial sums are not read either)
   // the block's W stages [g_begin, g_end) and steps [s_begin, s_end)
   const int g_begin = blk.split ? (int)((int64_t)blk.kr * stages / S) : 0;
   const int g_end = blk.split ? (int)((int64_t)(blk.kr + 1) * stages / S) : stages;
@@ -361,9 +362,9 @@ using Nv128M = NvGeom<2, 2, 2, 2, 2>;  // 128 x 128, two blocks per CU
 using Nv64M = NvGeom<1, 2, 2, 2, 4>;   // 64 x 128, two blocks per CU
 
 static GpPlan nv_plan(const QmmArgs &a) {
-  const int n = sizeof(NV_COST) / sizeof(NV_COST[0]);
-  return gp_plan(NV_COST, a.w_up ? n - 1 : n, a.M, a.w_up ? 2 * (int64_t)a.N : a.N, (a.K + V_BK - 1) / V_BK, V_SS,
-                 device_cu_count());
+  const int n = sizeof(NV_COST) / sizeof(NV_COST[0]), steps = (a.K + V_BK - 1) / V_BK, cus = device_cu_count();
+  const GpPlan one = gp_plan(NV_COST, n, a.M, a.N, steps, V_SS, cus);
+  return a.w_up ? gp_plan_pair(NV_COST, n - 1, one, a.M, a.N, steps, V_SS, cus) : one;
 }
 
 template <class G, bool MLP>
@@ -386,7 +387,7 @@ static hipError_t launch_nv(const QmmArgs &a, const GpPlan &p, const uint8_t *sp
 // K % 32: 16-byte W pieces; x and W rows 16-byte aligned for the DMA.
 bool gemm_nvfp4_ok(const QmmArgs &a) {
   return a.mode == NVFP4 && !a.x_f32 && a.K % 32 == 0 && a.K > 0 && a.M > 0 && a.N > 0 && (uintptr_t)a.x % 16 == 0 &&
-         (uintptr_t)a.w % 16 == 0 && (uintptr_t)a.w_up % 16 == 0;
+         (uintptr_t)a.w % 16 == 0 && (uintptr_t)a.w_up % 16 == 0 && (!a.w_up || nv_plan(a).cfg >= 0);
 }
 
 // Workspace: the scales repacked tile-major, unless they come so, then the split tiles' fp32

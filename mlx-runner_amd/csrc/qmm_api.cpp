@@ -1137,9 +1137,8 @@ int qmm_mlp_gate_up_silu(qmm_array *res, qmm_array x, qmm_array w_gate, qmm_arra
   b.s = su;
   if (tiled_scales((Arr *)s_gate.ctx, a, st, &a.s_tiled) || tiled_scales((Arr *)s_up.ctx, b, st, &b.s_tiled))
     return finish(1);
-  // prefill shapes of the pipelined GEMMs: both projections and the activation in one
-  // (rounded as three calls would; the fp32 sums of a tile split along K can differ from
-  // those of the projections alone, whose splits are their own)
+  // prefill shapes of the pipelined GEMMs: both projections and the activation in one, rounded
+  // and summed as the three calls would be (gp_plan_pair)
   if (K > 0 && !qmm_on_decode(a)) {
     fused.s_tiled = a.s_tiled;
     fused.s_up_tiled = b.s_tiled;

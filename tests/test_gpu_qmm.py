@@ -6,6 +6,7 @@ double sum once to bf16); f32 outputs within the same bound.
 """
 import ctypes
 import functools
+import re
 
 import numpy as np
 import pytest
@@ -716,26 +717,109 @@ def test_qmv_any_k(M, N, K):
     assert np.array_equal(np.concatenate([o.numpy() for o in outs], 1), y)
 
 
-@pytest.mark.parametrize("mode", ["mxfp8", "nvfp4"])
-@pytest.mark.parametrize("M,N,K", [(17, 33, 96), (64, 65, 224), (130, 129, 288), (200, 1000, 512), (383, 2000, 992),
-                                   (520, 5000, 288), (2049, 8300, 544)])
-def test_mlp_prefill_tiles(mode, M, N, K):
-    """The one-launch prefill MLP at the edges of its tiles and splits: each output within the
-    activation's roundings of the projections' results.  The projections alone may sum in
-    another order, so gate and up may differ by a bf16 rounding (2^-8); through silu and the
-    product that is at most 2^-5 of the value, and 2^-8 of |gate| |up| where silu's slope
-    counts, and nearly all outputs are equal."""
-    rng = np.random.default_rng(M + N + K)
-    wg, sg = rand_w(rng, mode, N, K)
-    wu, su = rand_w(rng, mode, N, K)
-    x = Q.Array.from_numpy(bf16(rng.standard_normal((M, K))), Q.BFLOAT16)
-    A = lambda a, d: Q.Array.from_numpy(a, d)  # noqa: E731
-    gate, up = (A(wg, Q.UINT32), A(sg, Q.UINT8)), (A(wu, Q.UINT32), A(su, Q.UINT8))
-    h = f32(Q.mlp_gate_up_silu(x, *gate, *up, mode).numpy())
-    g, u = Q.quantized_matmul(x, *gate, mode), Q.quantized_matmul(x, *up, mode)
-    h2, gu = f32(Q.silu_mul(g, u).numpy()), np.abs(f32(g.numpy()) * f32(u.numpy()))
-    assert np.all(np.abs(h - h2) <= np.abs(h2) * 2.0 ** -5 + gu * 2.0 ** -8 + 1e-30)
-    assert np.mean(h == h2) > 0.99
+class _KernelNode(ctypes.Structure):
+    """hipKernelNodeParams."""
+    _fields_ = [("block", ctypes.c_uint * 3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p),
+                ("grid", ctypes.c_uint * 3), ("args", ctypes.c_void_p), ("lds", ctypes.c_uint)]
+
+
+def kernels_of(call):
+    """[(mangled name, blocks)] of the kernels that call(stream) launches, in some order."""
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    hip.hipKernelNameRefByPtr.restype = ctypes.c_char_p
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call(Q.Stream.torch_current())  # the stream's workspace and the scale copies are there after it
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph, stream=side):
+        call(Q.Stream.torch_current())
+    raw, n, kind, node = ctypes.c_void_p(graph.raw_cuda_graph()), ctypes.c_size_t(), ctypes.c_int(), _KernelNode()
+    assert hip.hipGraphGetNodes(raw, None, ctypes.byref(n)) == 0
+    nodes, out = (ctypes.c_void_p * n.value)(), []
+    assert hip.hipGraphGetNodes(raw, nodes, ctypes.byref(n)) == 0
+    for v in nodes:
+        assert hip.hipGraphNodeGetType(ctypes.c_void_p(v), ctypes.byref(kind)) == 0
+        if kind.value == 0:  # hipGraphNodeTypeKernel
+            assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(v), ctypes.byref(node)) == 0
+            out.append((hip.hipKernelNameRefByPtr(ctypes.c_void_p(node.func), None).decode(), node.grid[0]))
+    return out
+
+
+def tiles_of(call, M, N, mlp=False):
+    """("TM x TN", "whole", "split" or "both") of the one pipelined GEMM that call(stream) launches:
+    its tiles, and whether they run whole, all split along K, or the last ones split."""
+    ks = [(n, g) for n, g in kernels_of(call) if "Geom" in n]
+    (name, blocks), = [k for k in ks if "reduce" not in k[0]]
+    fi, fj, wm, wn = (int(v) for v in re.search(r"GeomILi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)E", name).groups())
+    TM, TN = 32 * fi * wm, 32 * fj * wn
+    total, left = -(-M // TM) * -(-N // TN) * (2 if mlp else 1), 0
+    if len(ks) > 1:
+        (_, rblocks), = [k for k in ks if "reduce" in k[0]]
+        left = rblocks * 1024 * (2 if mlp else 1) // (TM * TN)
+        assert (blocks - (total - left)) % left == 0 and blocks > total
+    else:
+        assert blocks == total
+    return "%dx%d" % (TM, TN), "whole" if left == 0 else "split" if left == total else "both"
+
+
+def _quantized(gen, mode, N, K):
+    """A quantized weight, and it in float64."""
+    st = Q.Stream.torch_current()
+    wq, sc = Q.quantize(Q.Array.from_torch((torch.randn((N, K), generator=gen, device="cuda") * 0.02).to(torch.bfloat16)),
+                        mode, stream=st)
+    return (wq, sc), torch.from_numpy(Q.dequantize(wq, sc, mode, dtype=Q.FLOAT32, stream=st).numpy(st)).cuda().double()
+
+
+# Every tile of the MLP form with its tiles whole, all split along K and both, at ragged M, N and K
+# (the tile is what the plan takes on 256 CUs); at N just past whole tiles the second half of the
+# last pair is empty.  "three calls": gate alone splits tiles that have no MLP form (the other
+# tiles are slower), or mxfp8 K % 64 = 32.
+MLP_TILES = [
+    ("mxfp8", 212, 18471, 64, "256x256", "whole"), ("mxfp8", 465, 2787, 4864, "256x256", "split"),
+    ("mxfp8", 1165, 13189, 1536, "256x256", "both"), ("mxfp8", 188, 18422, 64, "192x256", "whole"),
+    ("mxfp8", 133, 2236, 1856, "192x256", "split"), ("mxfp8", 529, 22304, 2368, "192x256", "both"),
+    ("mxfp8", 70, 16610, 768, "128x256", "whole"), ("mxfp8", 83, 2717, 4288, "128x256", "split"),
+    ("mxfp8", 10, 83, 64, "128x128", "whole"), ("mxfp8", 66, 689, 1280, "128x128", "split"),
+    ("mxfp8", 845, 4707, 1152, "128x128", "both"), ("mxfp8", 12, 66, 128, "64x128", "whole"),
+    ("mxfp8", 9, 75, 832, "64x128", "split"), ("mxfp8", 233, 8329, 1024, "64x128", "both"),
+    ("nvfp4", 205, 16531, 128, "256x256", "whole"), ("nvfp4", 202, 10214, 4608, "256x256", "split"),
+    ("nvfp4", 1268, 13274, 1024, "256x256", "both"), ("nvfp4", 269, 15011, 64, "192x256", "whole"),
+    ("nvfp4", 132, 2332, 2336, "192x256", "split"), ("nvfp4", 530, 26557, 1728, "192x256", "both"),
+    ("nvfp4", 65, 17459, 1120, "128x256", "whole"), ("nvfp4", 130, 2807, 5120, "128x256", "split"),
+    ("nvfp4", 389, 16445, 5056, "128x256", "both"), ("nvfp4", 10, 102, 64, "128x128", "whole"),
+    ("nvfp4", 13, 69, 736, "128x128", "split"), ("nvfp4", 326, 11340, 1120, "128x128", "both"),
+    ("nvfp4", 11, 87, 352, "64x128", "whole"), ("nvfp4", 10, 91, 928, "64x128", "split"),
+    ("nvfp4", 304, 6576, 1280, "64x128", "both"), ("nvfp4", 76, 22309, 3232, "three calls", ""),
+    ("mxfp8", 200, 17408, 5120, "three calls", ""), ("nvfp4", 20, 17408, 5120, "three calls", ""),
+    ("mxfp8", 17, 33, 96, "three calls", ""), ("mxfp8", 64, 65, 224, "three calls", ""),
+    ("nvfp4", 17, 33, 96, "128x128", "whole"), ("nvfp4", 520, 5000, 288, "128x128", "whole"),
+]
+
+
+@pytest.mark.parametrize("mode,M,N,K,tile,split", MLP_TILES)
+def test_mlp_prefill_tiles(mode, M, N, K, tile, split):
+    """The one-launch prefill MLP equals quantized_matmul x 2 + silu_mul bit for bit: it splits each
+    column's sums along K as the projections alone do."""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + N + K)
+    (gate, _), (up, _) = _quantized(gen, mode, N, K), _quantized(gen, mode, N, K)
+    x = Q.Array.from_torch(torch.randn((M, K), generator=gen, device="cuda").to(torch.bfloat16))
+    h, g, u, h2 = (torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(4))
+    st = Q.Stream.torch_current()
+    for _ in range(2):
+        Q.mlp_gate_up_silu(x, *gate, *up, mode, out=Q.Array.from_torch(h), stream=st)
+        Q.quantized_matmul(x, *gate, mode, out=Q.Array.from_torch(g), stream=st)
+        Q.quantized_matmul(x, *up, mode, out=Q.Array.from_torch(u), stream=st)
+        Q.silu_mul(Q.Array.from_torch(g), Q.Array.from_torch(u), out=Q.Array.from_torch(h2), stream=st)
+        assert not h2.isnan().any()
+        assert torch.equal(h.view(torch.int16), h2.view(torch.int16))
+    call = lambda s: Q.mlp_gate_up_silu(x, *gate, *up, mode, out=Q.Array.from_torch(h), stream=s)  # noqa: E731
+    if tile == "three calls":
+        assert sum("silu_mul" in n for n, _ in kernels_of(call)) == 1
+    elif torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert tiles_of(call, M, N, mlp=True) == (tile, split)
 
 
 @pytest.mark.parametrize("mode,M,N", [("nvfp4", 1, 16400), ("nvfp4", 2, 4099), ("nvfp4", 3, 4099),
