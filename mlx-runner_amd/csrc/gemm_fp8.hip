@@ -150,7 +150,9 @@ struct MxGeom {
   static constexpr int NX = TM / 8 / NW;       // x DMAs per wave per step
   static constexpr int NWD = TN / 8 / NW + 1;  // W DMAs and one of the scales' per wave per stage
   static_assert(TM / 8 % NW == 0 && TN / 8 % NW == 0 && TN % 4 == 0 && NW % 2 == 0 && SD <= NW, "");
-  static_assert(SX >= 2 && SW >= 2 && SX <= 2 * SW - 1, "");
+  // (step 2 g + 1 of the kernel's MODE 3, g + SW the range's end, brings x of step 2 g + 1 + SX, which
+  // has to be one of the range's 2 (g + SW))
+  static_assert(SX >= 2 && SW >= 2 && SX <= 2 * SW - 2, "");
   static constexpr int REGION = 32 * (64 * FJ + 32);
   static_assert(NW * REGION <= LDS, "the epilogue regions fit the rings");
   // DMAs that may be in flight at the barrier of an even (odd) step s: x of step i + SX is
