@@ -142,7 +142,7 @@ static bool linear_gemv(int M) { return M <= QMV_MAX_M; }
 // ---------------------------------------------------------------- taller x
 
 namespace {
-constexpr int D_BK = 64;  // K elements of a step: 128 bytes of a row
+constexpr int D_BK = GP_STEP;  // K elements of a step: 128 bytes of a row
 // A block's tile: WM x WN waves of (32 FI) x (32 FJ); LDS rings of SX stages of x rows and
 // SW >= SX stages of W rows.
 template <int FI_, int FJ_, int WM_, int WN_, int SX_, int SW_>
@@ -323,19 +323,11 @@ using DnH = DnGeom<4, 2, 2, 2, 2, 4>;     // 256 x 128
 using Dn128 = DnGeom<2, 2, 2, 2, 2, 3>;   // 128 x 128, two blocks per CU
 using Dn64 = DnGeom<2, 1, 1, 4, 2, 4>;    // 64 x 128, two blocks per CU
 using DnS = DnGeom<1, 1, 2, 2, 2, 4>;     // 64 x 64, three blocks per CU
-// Measured on calls of whole rounds and of one block per CU, weights cold: on 39 shapes the plan's
-// choice takes 1.05 times the best configuration's time on average, at most 1.35 (1000 x 10240 x
-// 5120: 256 x 160 tiles fill one round of 256 CUs, 95 us; 256 x 256 ones, 160 of them, 99).
-constexpr GpCost DN_COST[] = {{256, 256, 1, 3.f, {1.24f}},         {256, 160, 1, 3.f, {1.10f}},
-                              {192, 256, 1, 3.f, {1.20f}},         {256, 128, 1, 3.f, {0.91f}},
-                              {128, 128, 2, 3.f, {0.64f, 0.90f}},  {64, 128, 2, 3.f, {0.56f, 0.74f}},
-                              {64, 64, 3, 3.f, {0.42f, 0.57f, 0.72f}}};
 }  // namespace
 
 // (split: with scratch for the partial sums of tiles split along K)
 static GpPlan dense_plan(int M, int N, int K, bool split) {
-  return gp_plan(DN_COST, sizeof(DN_COST) / sizeof(DN_COST[0]), M, N, (K + D_BK - 1) / D_BK, 1, device_cu_count(),
-                 split ? GP_MAX_SPLIT : 1);
+  return plan_dense(M, N, K, split, device_cu_count());
 }
 
 template <class G>

@@ -41,7 +41,7 @@ namespace qmm {
 
 // ---------------------------------------------------------------- x split pre-pass
 
-constexpr int X_BK = 64;  // K elements of a step: 64 bytes of hi and 64 of lo of an x row
+constexpr int X_BK = GP_STEP;  // K elements of a step: 64 bytes of hi and 64 of lo of an x row
 
 // The split of 16 consecutive elements (lane pair l, l ^ 1 shares a 32-block): E4M3
 // hi / lo words and the block's exponents th, tl.
@@ -423,21 +423,9 @@ using Mx128 = MxGeom<2, 2, 2, 2, 2, 2>;  // 128 x 128, two blocks per CU
 using Mx64 = MxGeom<1, 2, 2, 2, 3, 3>;   // 64 x 128, two blocks per CU
 using Mx160 = MxGeom<2, 5, 4, 1, 2, 2>;  // 256 x 160
 using Mx32 = MxGeom<1, 1, 1, 4, 3, 3>;   // 32 x 128, two blocks per CU
-// (fitted to 50 shapes of the declared range with every tile and split, rms error 8%; the
-// plan's choice is 1.01 of the best of them on average, at most 1.18.  The last two have no
-// MLP form: a wave's column blocks are not pairs.)
-constexpr GpCost MX_COST[] = {{256, 256, 1, 13.9f, {1.05f}},        {192, 256, 1, 13.4f, {0.83f}},
-                              {128, 256, 1, 13.6f, {0.61f}},        {128, 128, 2, 12.2f, {0.49f, 0.76f}},
-                              {64, 128, 2, 12.5f, {0.28f, 0.46f}},  {256, 160, 1, 13.7f, {0.72f}},
-                              {32, 128, 2, 11.8f, {0.24f, 0.40f}}};
-constexpr int MX_CONFIGS = sizeof(MX_COST) / sizeof(MX_COST[0]);
 }  // namespace
 
-static GpPlan mx_plan(const QmmArgs &a) {
-  const int steps = (a.K + X_BK - 1) / X_BK, cus = device_cu_count();
-  const GpPlan one = gp_plan(MX_COST, MX_CONFIGS, a.M, a.N, steps, 2, cus);
-  return a.w_up ? gp_plan_pair(MX_COST, MX_CONFIGS - 2, one, a.M, a.N, steps, 2, cus) : one;
-}
+static GpPlan mx_plan(const QmmArgs &a) { return plan_mxfp8(a.M, a.N, a.K, a.w_up != nullptr, device_cu_count()); }
 
 // The workspace: the split x, its scales, the repacked W scales that do not come tile-major,
 // and the split tiles' fp32 partial sums; each part a multiple of 256 bytes.

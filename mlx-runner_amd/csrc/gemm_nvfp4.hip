@@ -34,8 +34,8 @@
 namespace qmm {
 
 namespace {
-constexpr int V_BK = 64;   // K elements of a step: 128 bytes of an x row, 32 of a W row
-constexpr int V_SS = 4;    // steps of a W stage: 128 bytes of a W row, 16 of its scales
+constexpr int V_BK = GP_STEP;   // K elements of a step: 128 bytes of an x row, 32 of a W row
+constexpr int V_SS = NV_UNIT;    // steps of a W stage: 128 bytes of a W row, 16 of its scales
 // A block's tile: WM x WN waves of (32 FI) x (32 FJ); LDS rings of SX stages of x (a step
 // each) and two stages of W and its scales (V_SS steps each).
 template <int FI_, int FJ_, int WM_, int WN_, int SX_>
@@ -350,22 +350,13 @@ using NvW = NvGeom<4, 2, 1, 4, 2>;    // 128 x 256
 using Nv128 = NvGeom<4, 1, 1, 4, 2>;  // 128 x 128, two blocks per CU
 using Nv64 = NvGeom<2, 1, 1, 4, 4>;   // 64 x 128, two blocks per CU
 using Nv32 = NvGeom<1, 1, 1, 4, 4>;   // 32 x 128, three blocks per CU
-// (fitted to 45 shapes with every tile and split, rms error 7%; the
-// plan's choice is 1.01 of the best of them on average, at most 1.26)
-constexpr GpCost NV_COST[] = {{256, 256, 1, 9.7f, {1.10f}},         {192, 256, 1, 8.9f, {0.86f}},
-                              {128, 256, 1, 9.7f, {0.58f}},         {128, 128, 2, 7.8f, {0.42f, 0.69f}},
-                              {64, 128, 2, 8.6f, {0.26f, 0.43f}},   {32, 128, 3, 8.4f, {0.22f, 0.34f, 0.48f}}};
 }  // namespace
 
 // The MLP form needs a wave's column blocks in pairs: at 128 columns, 2 x 2 waves.
 using Nv128M = NvGeom<2, 2, 2, 2, 2>;  // 128 x 128, two blocks per CU
 using Nv64M = NvGeom<1, 2, 2, 2, 4>;   // 64 x 128, two blocks per CU
 
-static GpPlan nv_plan(const QmmArgs &a) {
-  const int n = sizeof(NV_COST) / sizeof(NV_COST[0]), steps = (a.K + V_BK - 1) / V_BK, cus = device_cu_count();
-  const GpPlan one = gp_plan(NV_COST, n, a.M, a.N, steps, V_SS, cus);
-  return a.w_up ? gp_plan_pair(NV_COST, n - 1, one, a.M, a.N, steps, V_SS, cus) : one;
-}
+static GpPlan nv_plan(const QmmArgs &a) { return plan_nvfp4(a.M, a.N, a.K, a.w_up != nullptr, device_cu_count()); }
 
 template <class G, bool MLP>
 static hipError_t launch_nv(const QmmArgs &a, const GpPlan &p, const uint8_t *sp, const uint8_t *sp_up, float *part,

@@ -1,54 +1,13 @@
 // Pieces shared by the pipelined GEMMs (mxfp8 on the scaled fp8 MFMA, nvfp4 and
 // dense bf16 on the bf16 MFMA): tile order, LDS DMA, barrier/wait helpers, the
-// epilogues, the split tiles' reduce, the weight-scale repack and the plan.
+// epilogues, the split tiles' reduce and the weight-scale repack.
 #pragma once
 
+#include "gemm_plan.h"
 #include "qmm_device.h"
 #include "qmm_launch.h"
 
 namespace qmm {
-
-// A call's blocks: [0, whole_tiles) run whole tiles, the others the S K-ranges of the tiles
-// that are left (whole_tiles on).  Tiles are numbered in groups of 4 x tiles walked down x
-// tiles first, and each XCD (the hardware hands it the blocks b with b % 8 = its number)
-// takes a contiguous run of them, so the ~32 blocks resident on one XCD cover a 4 x 8 patch of
-// (x rows, W rows) and share those operands in that XCD's L2.  Of a call that is all split, at few x tiles, the x tiles of
-// one W range of one K range run next to each other, so that they share its W.
-// PAIR (the MLP, whose tile holds half a tile's columns of gate and the same of up): tiles 2 t and
-// 2 t + 1 are the halves of tile t of one matrix alone.
-struct GpBlock {
-  int t, tm, tn, kr;
-  bool split;
-};
-template <bool PAIR>
-__device__ __forceinline__ void gp_tile_at(int t, int tiles_m, int tiles_n, int *tm, int *tn) {
-  constexpr int G = 4;
-  const int half = t & 1;
-  if (PAIR) t >>= 1;
-  const int first = t / (G * tiles_n) * G, gm = min(tiles_m - first, G), i = t - first * tiles_n;
-  *tm = first + i % gm;
-  *tn = PAIR ? 2 * (i / gm) + half : i / gm;
-}
-__device__ __forceinline__ int gp_xcd_run(int b, int n) {
-  const int base = n / 8, rem = n % 8, x = b % 8;
-  return x * base + min(x, rem) + b / 8;
-}
-template <bool PAIR = false>
-__device__ __forceinline__ GpBlock gp_block(int b, int tiles_m, int tiles_n, int whole_tiles, int S) {
-  GpBlock r;
-  r.split = b >= whole_tiles;
-  r.kr = 0;
-  if (!r.split) {
-    r.t = gp_xcd_run(b, whole_tiles);
-  } else {
-    const int left = tiles_m * tiles_n * (PAIR ? 2 : 1) - whole_tiles, u = gp_xcd_run(b - whole_tiles, left * S);
-    const int gm = whole_tiles == 0 && tiles_m <= 4 ? (PAIR ? 2 * tiles_m : tiles_m) : 1;
-    r.kr = u / gm % S;
-    r.t = whole_tiles + u / (gm * S) * gm + u % gm;
-  }
-  gp_tile_at<PAIR>(r.t, tiles_m, tiles_n, &r.tm, &r.tn);
-  return r;
-}
 
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
@@ -180,7 +139,6 @@ __device__ __forceinline__ void gp_store_partial(const f32x16_t (&acc)[FI][FJ], 
 // The split-tile reduce: the float4 at p is summed over the tile's S <= GP_MAX_SPLIT slots in
 // K order, the same order whichever block finished first, so the result is deterministic.
 // All S loads are issued before the first add, so a thread waits for one round trip, not S.
-constexpr int GP_MAX_SPLIT = 8;
 __device__ __forceinline__ float4 gp_sum_slots(const float4 *__restrict__ p, size_t slot, int S) {
   float4 f[GP_MAX_SPLIT];
 #pragma unroll
@@ -282,84 +240,6 @@ __global__ __launch_bounds__(256) void repack_scales_kernel(const uint8_t *__res
 #pragma unroll
     for (int k = 0; k < C; ++k) out[((tile * dpr + C * c + k) << 8) + rr] = d[k];
   }
-}
-
-// ---------------------------------------------------------------- host: the plan of a call
-
-// A tile size: TM x TN, per_cu blocks of it on a CU, and its measured cost: us per K step with
-// 1, 2, .. blocks on every CU, and us per round beside that.
-struct GpCost {
-  int TM, TN, per_cu;
-  float round, step[3];
-};
-struct GpPlan {
-  int cfg, whole, left, S;  // whole tiles, then `left` tiles split S ways along K
-  float us;                 // estimated
-};
-// The least estimated time over every tile size and every split of the tiles left after the
-// whole rounds (at most max_split ways, one round of blocks, at least 4 K steps each, in
-// units of `unit` steps).  Where several blocks share a CU, the last round may instead give
-// every CU `more` whole tiles and the split ones run beside them.  A split adds the reduce: its
-// launch and its partial sums' traffic.
-inline GpPlan gp_plan(const GpCost *costs, int n, int M, int64_t N, int steps, int unit, int cus,
-                      int max_split = GP_MAX_SPLIT) {
-  if (cus <= 0) cus = 256;  // (no device answers: the launch reports it)
-  GpPlan best{0, 0, 0, 1, 0.f};
-  float best_us = 1e30f;
-  const int units = (steps + unit - 1) / unit;
-  for (int c = 0; c < n; ++c) {
-    const GpCost &d = costs[c];
-    const int64_t T = (int64_t)((M + d.TM - 1) / d.TM) * ((N + d.TN - 1) / d.TN);
-    const int64_t slots = (int64_t)cus * d.per_cu, rounds = T / slots;
-    for (int more = 0; more < d.per_cu; ++more) {
-      const int64_t whole = rounds * slots + (int64_t)more * cus, left = T - whole;
-      if (left < 0) break;
-      for (int S = 1; S <= max_split; ++S) {
-        if (S > 1 && (left == 0 || left * S > slots - (int64_t)more * cus || units < S || steps < 4 * S)) break;
-        if (more && left && S == 1) continue;  // (the same blocks as more = 0)
-        const int mine = (units + S - 1) / S * unit, split_steps = mine < steps ? mine : steps;
-        int per = more + (int)((left * S + cus - 1) / cus);  // blocks on a CU in the last round
-        if (per > d.per_cu) per = d.per_cu;
-        float us = (float)rounds * ((float)steps * d.step[d.per_cu - 1] + d.round);
-        if (more) us += (float)(steps - split_steps) * d.step[more - 1];
-        if (per) us += (float)split_steps * d.step[per - 1] + d.round;
-        if (S > 1) us += 1.5f + (float)left * S * (M < d.TM ? M : d.TM) * d.TN * 8.f / 6.6e6f;
-        if (us < best_us) best_us = us, best = GpPlan{c, (int)whole, (int)left, S, us};
-      }
-    }
-  }
-  if (best.S == 1) best.whole += best.left, best.left = 0;
-  return best;
-}
-
-// The plan of an MLP's gate and up in one launch (tiles numbered in pairs, see gp_block) whose
-// sums run in the order of the two calls it replaces, so that its result is theirs bit for bit.
-// The order of a column's sums depends only on the split S of its tile along K: where `one`, a
-// call's own plan, splits no tile, or all, any of the n_pair tile sizes that have the form does,
-// with that split (the least estimated time); where it splits the last tiles, its own tile size
-// and twice its tiles.  cfg -1: that size has no MLP form, or the two calls and the activation (at
-// 2.7 TB/s) are estimated faster, as where their tile has no MLP form and twice the next one's
-// blocks need another round: nvfp4 20 x 17408 x 5120 50 us in one launch, 40 in three calls; mxfp8
-// 200 x 17408 x 5120 130 and 121 (64 rows: 63 and 75; 2048 rows: 572 and 614).
-inline GpPlan gp_plan_pair(const GpCost *costs, int n_pair, const GpPlan &one, int M, int64_t N, int steps, int unit,
-                           int cus) {
-  if (cus <= 0) cus = 256;
-  if (one.whole && one.left) return GpPlan{one.cfg < n_pair ? one.cfg : -1, 2 * one.whole, 2 * one.left, one.S, 0.f};
-  GpPlan best{-1, 0, 0, one.S, 0.f};
-  float best_us = 2.f * one.us + 3.f + (float)M * (float)N * 6.f / 2.7e6f;
-  const int units = (steps + unit - 1) / unit, mine = (units + one.S - 1) / one.S * unit;
-  for (int c = 0; c < n_pair; ++c) {
-    const GpCost &d = costs[c];
-    const int64_t T = (int64_t)((M + d.TM - 1) / d.TM) * ((N + d.TN - 1) / d.TN) * 2, blocks = T * one.S;
-    if (blocks > INT32_MAX) continue;
-    const int64_t slots = (int64_t)cus * d.per_cu, rounds = blocks / slots;
-    const int per = (int)((blocks - rounds * slots + cus - 1) / cus), n = mine < steps ? mine : steps;
-    float us = (float)rounds * ((float)n * d.step[d.per_cu - 1] + d.round);
-    if (per) us += (float)n * d.step[per - 1] + d.round;
-    if (one.S > 1) us += 1.5f + (float)blocks * (M < d.TM ? M : d.TM) * d.TN * 8.f / 6.6e6f;
-    if (us < best_us) best_us = us, best = GpPlan{c, one.S > 1 ? 0 : (int)T, one.S > 1 ? (int)T : 0, one.S, us};
-  }
-  return best;
 }
 
 }  // namespace qmm

@@ -7,12 +7,14 @@ double sum once to bf16); f32 outputs within the same bound.
 import ctypes
 import functools
 import re
+from math import ceil
 
 import numpy as np
 import pytest
 import torch
 
 import oracle as O
+import gemm_shapes as G
 import qmm as Q
 
 pytestmark = pytest.mark.gpu
@@ -369,15 +371,12 @@ def test_dense_linear_matches_fp32_reference(M):
 
 @pytest.mark.parametrize("M,N,K", [
     (1, 3, 16), (2, 2049, 1040), (5, 700, 4112), (8, 2047, 2064), (3, 4100, 2064), (4, 6146, 4096),  # the GEMV's forms
-    (6, 2048, 1040), (8, 5000, 528),                              # a few rows on the GEMM
-    (9, 1, 16), (10, 65, 48), (64, 63, 64), (65, 129, 1040),      # one partial tile, K ends inside a step
-    (33, 1000, 1040), (129, 273, 3328), (548, 256, 3584),         # tiles split along K
-    (1030, 492, 2848), (700, 2500, 1296),                         # 128-row tiles, whole and left over
-    (1000, 10240, 272), (1000, 10239, 288), (1300, 16400, 528),   # 256-row tiles: one round, and tiles left over
-])
+    (6, 2048, 1040), (8, 5000, 528),
+    (65, 129, 1040), (129, 273, 3328), (548, 256, 3584), (1030, 492, 2848), (700, 2500, 1296),
+    (1000, 10240, 272), (1000, 10239, 288), (1300, 16400, 528)] + [c[:3] for c in G.DENSE])
 def test_dense_linear_tiles(M, N, K):
-    """The dense GEMV and GEMM at the edges of their tiles, K steps and splits, against float64 on the
-    GPU: within the one bf16 rounding (2^-8 of the value) and the fp32 sums' error, which is
+    """The dense GEMV and GEMM at the edges of their tiles, K steps and splits (G.DENSE: every tile
+    whole, split and both), against float64 on the GPU: within the one bf16 rounding (2^-8 of the value) and the fp32 sums' error, which is
     below 2^-24 K of sum |x| |w|."""
     gen = torch.Generator(device="cuda")
     gen.manual_seed(M + N + K)
@@ -467,16 +466,13 @@ def test_dense_linear_takes_no_scratch_at_decode_or_in_a_graph(M):
     assert s.pool_used() == used
 
 
-@pytest.mark.parametrize("mode", ["nvfp4", "mxfp8"])
-@pytest.mark.parametrize("M,N,K", [
-    (17, 1, 32), (33, 129, 96), (64, 257, 224), (65, 300, 288),       # K ends inside a step or a stage of W
-    (33, 1000, 1056), (200, 320, 1024), (372, 328, 3456),             # tiles split along K
-    (68, 2700, 3392), (383, 2416, 992), (1030, 1000, 544),            # 64- and 128-row tiles
-    (520, 5000, 256), (1691, 10240, 288), (2049, 16480, 512),         # 256-wide tiles, rounds and tiles left over
-])
+@pytest.mark.parametrize("mode,M,N,K", [(m, *c) for m in ("nvfp4", "mxfp8") for c in [
+    (17, 1, 32), (33, 129, 96), (64, 257, 224), (65, 300, 288), (33, 1000, 1056), (200, 320, 1024), (372, 328, 3456),
+    (68, 2700, 3392), (383, 2416, 992), (1030, 1000, 544), (520, 5000, 256), (1691, 10240, 288), (2049, 16480, 512)]] +
+    [("nvfp4", *c[:3]) for c in G.NVFP4] + [("mxfp8", *c[:3]) for c in G.MXFP8])
 def test_prefill_tiles(mode, M, N, K):
-    """The prefill GEMMs at the edges of their tiles, K steps, W stages and splits, against
-    float64 on the GPU: within the bf16 rounding (2^-8 of the value) and the fp32 sums' (and
+    """The prefill GEMMs at the edges of their tiles, K steps, W stages and splits (G.NVFP4 and
+    G.MXFP8: every tile whole, split and both), against float64 on the GPU: within the bf16 rounding (2^-8 of the value) and the fp32 sums' (and
     the mxfp8 split of x, at most 2^-12 of a block's largest) error, below 2^-12 + K 2^-24 of
     sum |x| |w| taken with each 32-block's largest |x|."""
     gen = torch.Generator(device="cuda")
@@ -772,36 +768,69 @@ def _quantized(gen, mode, N, K):
     return (wq, sc), torch.from_numpy(Q.dequantize(wq, sc, mode, dtype=Q.FLOAT32, stream=st).numpy(st)).cuda().double()
 
 
-# Every tile of the MLP form with its tiles whole, all split along K and both, at ragged M, N and K
-# (the tile is what the plan takes on 256 CUs); at N just past whole tiles the second half of the
-# last pair is empty.  "three calls": gate alone splits tiles that have no MLP form (the other
-# tiles are slower), or mxfp8 K % 64 = 32.
-MLP_TILES = [
-    ("mxfp8", 212, 18471, 64, "256x256", "whole"), ("mxfp8", 465, 2787, 4864, "256x256", "split"),
-    ("mxfp8", 1165, 13189, 1536, "256x256", "both"), ("mxfp8", 188, 18422, 64, "192x256", "whole"),
-    ("mxfp8", 133, 2236, 1856, "192x256", "split"), ("mxfp8", 529, 22304, 2368, "192x256", "both"),
-    ("mxfp8", 70, 16610, 768, "128x256", "whole"), ("mxfp8", 83, 2717, 4288, "128x256", "split"),
-    ("mxfp8", 10, 83, 64, "128x128", "whole"), ("mxfp8", 66, 689, 1280, "128x128", "split"),
-    ("mxfp8", 845, 4707, 1152, "128x128", "both"), ("mxfp8", 12, 66, 128, "64x128", "whole"),
-    ("mxfp8", 9, 75, 832, "64x128", "split"), ("mxfp8", 233, 8329, 1024, "64x128", "both"),
-    ("nvfp4", 205, 16531, 128, "256x256", "whole"), ("nvfp4", 202, 10214, 4608, "256x256", "split"),
-    ("nvfp4", 1268, 13274, 1024, "256x256", "both"), ("nvfp4", 269, 15011, 64, "192x256", "whole"),
-    ("nvfp4", 132, 2332, 2336, "192x256", "split"), ("nvfp4", 530, 26557, 1728, "192x256", "both"),
-    ("nvfp4", 65, 17459, 1120, "128x256", "whole"), ("nvfp4", 130, 2807, 5120, "128x256", "split"),
-    ("nvfp4", 389, 16445, 5056, "128x256", "both"), ("nvfp4", 10, 102, 64, "128x128", "whole"),
-    ("nvfp4", 13, 69, 736, "128x128", "split"), ("nvfp4", 326, 11340, 1120, "128x128", "both"),
-    ("nvfp4", 11, 87, 352, "64x128", "whole"), ("nvfp4", 10, 91, 928, "64x128", "split"),
-    ("nvfp4", 304, 6576, 1280, "64x128", "both"), ("nvfp4", 76, 22309, 3232, "three calls", ""),
-    ("mxfp8", 200, 17408, 5120, "three calls", ""), ("nvfp4", 20, 17408, 5120, "three calls", ""),
-    ("mxfp8", 17, 33, 96, "three calls", ""), ("mxfp8", 64, 65, 224, "three calls", ""),
-    ("nvfp4", 17, 33, 96, "128x128", "whole"), ("nvfp4", 520, 5000, 288, "128x128", "whole"),
-]
+def _random_nvfp4(gen, N, K):
+    """Packed nvfp4 over every code, moderate scales, and the weight in float64."""
+    w = torch.randint(0, 256, (N, K // 2), generator=gen, device="cuda", dtype=torch.uint8)
+    s = torch.randint(0x20, 0x48, (N, K // 16), generator=gen, device="cuda", dtype=torch.uint8)
+    v = torch.tensor([0, .5, 1, 1.5, 2, 3, 4, 6, -0., -.5, -1, -1.5, -2, -3, -4, -6], dtype=torch.float64, device="cuda")
+    d = torch.stack((v[(w & 15).int()], v[(w >> 4).int()]), -1).view(N, K // 16, 16)
+    return w.view(torch.int32), s, (d * s.view(torch.float8_e4m3fn).double().unsqueeze(-1)).view(N, K)
+
+
+@pytest.mark.parametrize("M,N,K,flushes,mlp_flushes", [(6, 40001, 4096, 2, 3), (3, 70001, 2560, 2, 3), (4, 64500, 8192, 1, 0)])
+def test_qmv_any_many_row_blocks(M, N, K, flushes, mlp_flushes):
+    """Ranges of more row blocks per workgroup than the partial sums have slots for (8 in one pass):
+    several flushes, the last one short; and a two-pass MLP whose row blocks do not fit the LDS
+    (0 flushes: it runs as three calls).  Plain, grouped and as an MLP, every output against float64:
+    within the bf16 rounding (2^-8 of the value) and K 2^-24 of sum |x| |w|."""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(N + K)
+    x = torch.randn((M, K), generator=gen, device="cuda").to(torch.bfloat16)
+    st, A = Q.Stream.torch_current(), Q.Array.from_torch
+    xa, new = A(x), lambda n: torch.full((M, n), float("nan"), dtype=torch.bfloat16, device="cuda")  # noqa: E731
+    w, s, d = _random_nvfp4(gen, N, K)
+    ref = x.double() @ d.t()
+    bound = ref.abs() * 2.0 ** -8 + (x.double().abs() @ d.abs().t()) * (K * 2.0 ** -24) + 1e-30
+    del d
+    y, parts, h, g, u, h2 = new(N), [new(N - 12345), new(12345)], new(N), new(N), new(N), new(N)
+    Q.quantized_matmul(xa, A(w), A(s), "nvfp4", out=A(y), stream=st)
+    assert torch.all((y.double() - ref).abs() <= bound)
+    cut = N - 12345
+    Q.quantized_matmul_group(xa, [A(w[:cut]), A(w[cut:])], [A(s[:cut]), A(s[cut:])], "nvfp4",
+                             outs=[A(p) for p in parts], stream=st)
+    assert torch.equal(torch.cat(parts, 1), y)
+    wu, su, _ = _random_nvfp4(gen, N, K)
+    mlp = lambda st: Q.mlp_gate_up_silu(xa, A(w), A(s), A(wu), A(su), "nvfp4", out=A(h), stream=st)  # noqa: E731
+    mlp(st)
+    Q.quantized_matmul(xa, A(wu), A(su), "nvfp4", out=A(u), stream=st)
+    Q.silu_mul(A(y), A(u), out=A(h2), stream=st)
+    assert torch.equal(h, h2)
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        return
+
+    # the row blocks of a workgroup: those of its rows, in units of 16 (MLP: 8)
+    def check(call, rows, want):
+        (name, blocks), = [k for k in kernels_of(call) if "qmv_any" in k[0]]
+        row_blocks = ceil(ceil(N / blocks) / rows)
+        assert (ceil(row_blocks / 8) if K <= 4096 else 1) == want
+
+    check(lambda st: Q.quantized_matmul(xa, A(w), A(s), "nvfp4", out=A(y), stream=st), 16, flushes)
+    if mlp_flushes:
+        check(mlp, 8, mlp_flushes)
+    else:
+        names = [n for n, _ in kernels_of(mlp)]
+        assert sum("qmv_any" in n for n in names) == 2 and sum("silu_mul" in n for n in names) == 1
+
+
+MLP_TILES = [("nvfp4", *c) for c in G.NVFP4_MLP] + [("mxfp8", *c) for c in G.MXFP8_MLP] + [
+    ("mxfp8", 17, 33, 96, "none", ""), ("mxfp8", 64, 65, 224, "none", "")]  # K % 64 = 32
 
 
 @pytest.mark.parametrize("mode,M,N,K,tile,split", MLP_TILES)
 def test_mlp_prefill_tiles(mode, M, N, K, tile, split):
-    """The one-launch prefill MLP equals quantized_matmul x 2 + silu_mul bit for bit: it splits each
-    column's sums along K as the projections alone do."""
+    """The one-launch prefill MLP, every tile of it whole, split along K and both, equals
+    quantized_matmul x 2 + silu_mul bit for bit: it splits each column's sums as the projections
+    alone do."""
     gen = torch.Generator(device="cuda")
     gen.manual_seed(M + N + K)
     (gate, _), (up, _) = _quantized(gen, mode, N, K), _quantized(gen, mode, N, K)
@@ -816,7 +845,7 @@ def test_mlp_prefill_tiles(mode, M, N, K, tile, split):
         assert not h2.isnan().any()
         assert torch.equal(h.view(torch.int16), h2.view(torch.int16))
     call = lambda s: Q.mlp_gate_up_silu(x, *gate, *up, mode, out=Q.Array.from_torch(h), stream=s)  # noqa: E731
-    if tile == "three calls":
+    if tile == "none":
         assert sum("silu_mul" in n for n, _ in kernels_of(call)) == 1
     elif torch.cuda.get_device_properties(0).multi_processor_count == 256:
         assert tiles_of(call, M, N, mlp=True) == (tile, split)
