@@ -86,7 +86,8 @@ int qmm_synchronize(qmm_stream s);                /* mlx_synchronize */
  *  mode: "mxfp8" | "nvfp4".  y: [..., M, N] in x's dtype (fp32 accumulation, RNE).
  * If *res already holds an array of exactly the output shape and dtype its
  * buffer is written in place (no allocation); otherwise *res is replaced by a
- * new array.  Prefill calls (M > 8) read the scales in a tile-major copy that the
+ * new array.  Prefill calls (M > 8; and 5-8 rows of tall matrices that no decode kernel
+ * for so many rows takes) read the scales in a tile-major copy that the
  * library makes at the first such call with this scales handle (not while the
  * stream is being captured) and frees with the handle: as with mlx arrays, the
  * contents behind a handle must not change while it lives.  The copy holds
@@ -110,8 +111,9 @@ int qmm_quantized_matmul(qmm_array *res, qmm_array x, qmm_array w, qmm_array sca
  * (src/model.zig:1066-1074) and attention's q / k / v (:929-944).  When the
  * matrices lie back to back in memory, and so do their scales (in any order;
  * qmm_weights_load places each layer's groups so), with bfloat16 x, one kernel
- * runs over them as one matrix: the decode kernel at M <= 4, the prefill GEMM at
- * the sizes it takes (the stacked scales are then repacked per call); otherwise one
+ * runs over them as one matrix: a decode kernel at M <= 4, and nvfp4 at up to 8 rows
+ * where K is none of 5120, 6144, 10240, 17408 but a multiple of 128; the prefill GEMM
+ * at the sizes it takes (the stacked scales are then repacked per call); otherwise one
  * call per matrix.  Either way res[i] meets the bar of
  * qmm_quantized_matmul(x, w[i], scales[i]); the one launch picks its kernel and tiling
  * by the total row count, which can differ from the single call's choice, so the bf16
@@ -152,7 +154,8 @@ int qmm_quantize(qmm_vector_array *res, qmm_array w, qmm_optional_int group_size
  * (one per device and stream, kept until the process ends), or, while the stream
  * is being captured into a graph and that is too small, an allocation made on the
  * stream and released after the call's kernels.  The prefill GEMMs of
- * qmm_quantized_matmul (M > 8) take theirs the same way. */
+ * qmm_quantized_matmul take theirs the same way.  A call holds the workspace until its
+ * launches are enqueued, so host threads may share a stream. */
 int qmm_gdn_recurrence(qmm_array *y, qmm_array *state_out, qmm_array q, qmm_array k, qmm_array v, qmm_array g,
                        qmm_array beta, qmm_array state, qmm_dtype y_dtype, qmm_stream s);
 
@@ -179,8 +182,9 @@ int qmm_silu_mul(qmm_array *res, qmm_array g, qmm_array u, qmm_stream s);
 
 /* h = silu(x @ deq(Wg).T) * (x @ deq(Wu).T): the first three ops of mlpForwardQ
  * (src/model.zig:905-913) in one call, same arguments as qmm_quantized_matmul for
- * each projection.  Decode shapes (M <= 4) run one fused kernel (the gate and up
- * rows of an output in one wave, the activation in its epilogue); the result
+ * each projection.  Decode shapes (M <= 4; nvfp4 up to 8 rows as above) run one fused
+ * kernel (the gate and up rows of an output in one wave, the activation in its epilogue,
+ * or two calls and the activation where that is not there); the result
  * equals quantized_matmul x 2 + silu_mul.  Prefill shapes run one GEMM over both
  * matrices, rounded in the same places and summed in the same order: the result equals
  * quantized_matmul x 2 + silu_mul there too. */

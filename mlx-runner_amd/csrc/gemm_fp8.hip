@@ -30,7 +30,7 @@
 // 41 (199).
 // gate, up and silu(gate) * up of an MLP in one launch (MLP below), 2048 x (2 x 17408) x 5120 with
 // the split of x: 572 us, against 614 for the three calls, whose result it gives bit for bit
-// (gp_plan_pair; splitting the last tiles as suits one launch best took 550).
+// (gp_plan_pair; on another box 620, and 600 with the last tiles split as suits one launch best).
 #include <type_traits>
 
 #include "gemm_pipe.h"

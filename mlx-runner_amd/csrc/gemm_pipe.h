@@ -117,10 +117,10 @@ __device__ __forceinline__ void gp_store_tile_bf16(const f32x16_t (&acc)[FI][FJ]
 // Split tiles (a tile's K steps run by S blocks): each block stores its wave's FI x FJ
 // fp32 accumulators as they sit in the registers, the float4 of elements 4 v4 .. 4 v4 + 3
 // of accumulator (i, j) of lane l at ((wave * FI * FJ + i * FJ + j) * 4 + v4) * 64 + l of
-// the block's slot (8 waves: 8 * FI * FJ * 1 KiB per slot).  Accumulator rows i with
+// the block's slot (NW * FI * FJ * 1 KiB per slot).  Accumulator rows i with
 // 32 i >= live_rows (the wave's rows past the last x row: padding of a short x) are
 // neither stored nor summed.
-template <int FI, int FJ, int NW = 8>
+template <int FI, int FJ, int NW>
 __device__ __forceinline__ void gp_store_partial(const f32x16_t (&acc)[FI][FJ], float *__restrict__ slot, int wave,
                                                  int lane, int live_rows) {
   float4 *pw = (float4 *)slot + (size_t)wave * FI * FJ * 4 * 64 + lane;

@@ -18,8 +18,9 @@ constexpr int GP_MAX_SPLIT = 8;
 // that are left (whole_tiles on).  Tiles are numbered in groups of 4 x tiles walked down x
 // tiles first, and each XCD (the hardware hands it the blocks b with b % 8 = its number)
 // takes a contiguous run of them, so the ~32 blocks resident on one XCD cover a 4 x 8 patch of
-// (x rows, W rows) and share those operands in that XCD's L2.  Of a call that is all split, at few x tiles, the x tiles of
-// one W range of one K range run next to each other, so that they share its W.
+// (x rows, W rows) and share those operands in that XCD's L2.  Of a call that is all split, at
+// few x tiles, the x tiles of one W range of one K range run next to each other, so that they
+// share its W.
 // PAIR (the MLP, whose tile holds half a tile's columns of gate and the same of up): tiles 2 t and
 // 2 t + 1 are the halves of tile t of one matrix alone.
 struct GpBlock {
@@ -136,23 +137,28 @@ inline GpPlan gp_plan_pair(const GpCost *costs, int n_pair, const GpPlan &one, i
 
 // ---------------------------------------------------------------- the tile sizes and their costs
 
-// Dense bf16 (DnGeom).  Measured on calls of whole rounds and of one block per CU, weights cold: on 39 shapes the plan's
-// choice takes 1.05 times the best configuration's time on average, at most 1.35 (1000 x 10240 x
-// 5120: 256 x 160 tiles fill one round of 256 CUs, 95 us; 256 x 256 ones, 160 of them, 99).
+// Dense bf16 (DnGeom).  Measured on calls of whole rounds and of one block per CU, weights cold: on
+// 18 shapes of 300 to 2048 rows the plan's choice takes 1.02 times the best tile's time on average, at
+// most 1.07, on 39 of 9 rows up 1.05 and 1.35 (1000 x 10240 x 5120: 256 x 160 tiles fill one round of
+// 256 CUs, 95 us; 256 x 256 ones, 160 of them, 99).
 inline constexpr GpCost DN_COST[] = {{256, 256, 1, 3.f, {1.24f}},         {256, 160, 1, 3.f, {1.10f}},
                                      {192, 256, 1, 3.f, {1.20f}},         {256, 128, 1, 3.f, {0.91f}},
                                      {128, 128, 2, 3.f, {0.64f, 0.90f}},  {64, 128, 2, 3.f, {0.56f, 0.74f}},
                                      {64, 64, 3, 3.f, {0.42f, 0.57f, 0.72f}}};
 
-// nvfp4 (NvGeom).  (Fitted to 45 shapes with every tile and split, rms error 7%; the
-// plan's choice is 1.01 of the best of them on average, at most 1.26)
+// nvfp4 (NvGeom).  Fitted to 45 shapes of 5 to 1930 rows, two thirds under 400, with every tile and split:
+// rms error 7%, the plan's choice 1.01 of the best of them on average, at most 1.26.  On 19 others
+// of 300 to 2048 rows the choice is 1.01 of the best on average, at most 1.08; the estimate itself is
+// low there, as the clock is under full load: measured 0.94 to 1.27 times it, 1.11 on average.
 inline constexpr GpCost NV_COST[] = {{256, 256, 1, 9.7f, {1.10f}},         {192, 256, 1, 8.9f, {0.86f}},
                                      {128, 256, 1, 9.7f, {0.58f}},         {128, 128, 2, 7.8f, {0.42f, 0.69f}},
                                      {64, 128, 2, 8.6f, {0.26f, 0.43f}},   {32, 128, 3, 8.4f, {0.22f, 0.34f, 0.48f}}};
 
-// mxfp8 (MxGeom).  (Fitted to 50 shapes of the declared range with every tile and split, rms error 8%; the
-// plan's choice is 1.01 of the best of them on average, at most 1.18.  The last two have no
-// MLP form: a wave's column blocks are not pairs.)
+// mxfp8 (MxGeom).  Fitted to 50 shapes of 5 to 1930 rows likewise: rms error 8%, the choice 1.01 of the
+// best on average, at most 1.18.  On 22 others of 300 to 2048 rows 1.02, at most 1.19 (W of 20000 rows
+// and more at K of 1100: two blocks of 128 x 128 on a CU overlap their rounds, which the plan prices
+// one after the other); measured 0.73 to 1.34 times the estimate.  The last two have no MLP form: a
+// wave's column blocks are not pairs.
 inline constexpr GpCost MX_COST[] = {{256, 256, 1, 13.9f, {1.05f}},        {192, 256, 1, 13.4f, {0.83f}},
                                      {128, 256, 1, 13.6f, {0.61f}},        {128, 128, 2, 12.2f, {0.49f, 0.76f}},
                                      {64, 128, 2, 12.5f, {0.28f, 0.46f}},  {256, 160, 1, 13.7f, {0.72f}},

@@ -235,12 +235,10 @@ def test_decode_long_k_matches_oracle(mode, M, N, K):
 
 @pytest.mark.parametrize("K", [128, 256, 384, 512])
 def test_prefill_mxfp8_partial_last_round(K):
-    """x rows 300 (ragged against the 256-row tiles), W rows 33180: on a 256-CU
-    part the 256 x 256 tiles leave a last round of 4 tiles, which runs as 128 x 128
-    tiles over the last two tile-columns; every column from there on is checked
-    (plus a sample of the rest), all rows, at K = 128 to 512 (the tail kernel's
-    2-step, 4-step, 6-step and looped 8-step schedules), and a second call must
-    return the same bits."""
+    """x rows 300 (ragged against every tile), W rows 33180: several rounds of tiles, the last
+    one partial; the last columns are checked (plus a sample of the rest), all rows, at
+    K = 128 to 512 (1 to 4 stages of W, around the ring's depth of 2 or 3), and a second call
+    must return the same bits."""
     mode, M, N = "mxfp8", 300, 33180
     rng = np.random.default_rng(11)
     wq, s = rand_w(rng, mode, N, K)
@@ -306,8 +304,7 @@ def test_prefill_matches_oracle(mode, M, N, K):
 
 
 # K of one to three 64-element steps: the pipelined GEMMs' ring prologue issues fewer
-# steps than it has stages (nvfp4 at every K here, mxfp8 at K = 128), as whole tiles
-# (M = 300) and as the short-x tile heights (M = 40, 100).
+# steps than it has stages, in tiles of 32 to 128 rows.
 @pytest.mark.parametrize("mode", ["mxfp8", "nvfp4"])
 @pytest.mark.parametrize("M,N,K", [(300, 300, 64), (300, 300, 128), (300, 300, 192), (40, 600, 128), (100, 520, 192)])
 def test_prefill_short_k(mode, M, N, K):
@@ -541,11 +538,9 @@ def test_silu_mul_matches_oracle():
 @pytest.mark.parametrize("M,N,K", [(1, 200, 512), (2, 96, 5120), (3, 61, 1536), (4, 48, 5120), (20, 72, 512),
                                    (300, 130, 384), (40, 96, 192)])
 def test_mlp_gate_up_silu_matches_oracle(mode, M, N, K):
-    """silu(x Wg^T) * (x Wu^T) (src/model.zig:905-913): fused for M <= 4, projections
-    + activation for larger M (mxfp8: the up projection reuses the gate's x split, in
-    the pipelined layout at K = 384 and 512, the row-major one at K = 192); equal to
-    quantized_matmul x 2 + silu_mul bit for bit, and within tolerance of the oracle's
-    chain."""
+    """silu(x Wg^T) * (x Wu^T) (src/model.zig:905-913): fused decode kernels for M <= 4, one
+    prefill GEMM for larger M; equal to quantized_matmul x 2 + silu_mul bit for bit, and
+    within tolerance of the oracle's chain."""
     rng = np.random.default_rng(M * 100 + N + K)
     wg, sg = rand_w(rng, mode, N, K)
     wu, su = rand_w(rng, mode, N, K)
@@ -1135,14 +1130,9 @@ def test_random_shapes_match_oracle():
     torch.cuda.synchronize()
 
 
-# Prefill shapes whose 256 x 256 tiles leave a partial last round that whole W
-# tile-columns fill: those columns run as smaller tiles in the same launch (mxfp8:
-# 128 x 128, nvfp4: 128 x rows of x by 256 W rows).  M = 2000 (8 row tiles, the last one
-# ragged) with N = 8448 (33 tile-columns: 264 tiles, 8 left over = one column), N = 8348
-# (the same with a ragged last column) and N = 8704 (34 columns: 272 tiles, 16 left
-# over = two columns).  nvfp4 with one row tile: M = 100 and 200, N = 76800 (300 tiles,
-# 44 left over: one 128-row tail tile per column at M = 100, two at M = 200, the second
-# ragged).
+# Prefill shapes whose tiles fill rounds of the chip and part of another: M = 2000 (ragged
+# against the 192- and 256-row tiles) and 2048 with N = 8448, 8348 (ragged) and 8704; one
+# or two x tiles with very many of W (nvfp4 M = 100 and 200, N = 76800: 600 and 300 tiles).
 @pytest.mark.parametrize("mode,M,N", [("mxfp8", 2000, 8448), ("mxfp8", 2048, 8704), ("nvfp4", 2000, 8348),
                                       ("nvfp4", 2048, 8704), ("nvfp4", 100, 76800), ("nvfp4", 200, 76800)])
 def test_prefill_with_tail_tiles_in_one_launch(mode, M, N):
@@ -1151,8 +1141,7 @@ def test_prefill_with_tail_tiles_in_one_launch(mode, M, N):
     wq, s = rand_w(rng, mode, N, K)
     xb = make_x(rng, M, K, "edge")
     y = run_qmm(mode, xb, wq, s)
-    # every column of the last 640 (the tail tile-columns on a 256-CU part and their
-    # neighbours), plus a sample of the rest
+    # every column of the last 640 (those of the last tiles), plus a sample of the rest
     cols = np.unique(np.concatenate([np.arange(N - 640, N), np.arange(0, N - 640, 37)]))
     rows = np.unique(np.concatenate([np.arange(0, M, 61), [M - 1]]))
     ref = O.qmm(mode, xb[rows], wq, s, cols=cols)
