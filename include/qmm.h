@@ -290,7 +290,8 @@ int qmm_named_linear_q_group(qmm_array *res, size_t n, qmm_weight_map m, qmm_arr
 /* Dense y = x @ w.T for bf16 x [..., M, K] and bf16 w [N, K] (linear, src/model.zig:200-211).
  * Calls of up to 8 rows, and calls captured into a graph, need no scratch.  Eager calls of
  * more rows take partial sums from the stream's workspace (see qmm_gdn_recurrence) when it
- * can be had, and run without it otherwise; the order of the fp32 sums then differs. */
+ * can be had.  Without it (captured calls too) no tile is split along K: the fp32 sums run
+ * in another order, and some results round the other way in bf16. */
 int qmm_linear(qmm_array *res, qmm_array x, qmm_array w, qmm_stream s);
 /* mlpForwardQ (src/model.zig:905-915): down(silu(gate(x)) * up(x)) by checkpoint
  * names, in the reference's argument order (gate, down, up). */
